@@ -421,27 +421,6 @@ PXR_DEV void direct_deposit(const DirectIn<T> &in, const Acc &acc) {
 // ---------------------------------------------------------------------------
 // wavefront ballot ranking
 // ---------------------------------------------------------------------------
-// For every active lane: rank among the active lanes of its wave holding the
-// same key and a lower lane id, the number of such lanes (cnt) and the
-// lowest of them (leader).  One ballot per distinct key in the wave.
-PXR_DEV void wave_peers(bool active, int key, int &rank, int &cnt, int &leader) {
-  const int lane = __lane_id();
-  unsigned long long todo = __ballot(active);
-  unsigned long long mine = 0;
-  while (todo) {
-    const int l = __ffsll((unsigned long long)todo) - 1;
-    const int lk = __shfl(key, l);
-    const bool same = active && key == lk;
-    const unsigned long long m = __ballot(same);
-    if (same) mine = m;
-    todo &= ~m;
-  }
-  const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  rank = __popcll(mine & below);
-  cnt = __popcll(mine);
-  leader = mine ? __ffsll((unsigned long long)mine) - 1 : lane;
-}
-
 // Runs of equal keys on neighbouring active lanes (keys that are mostly
 // sorted along the lanes): head is the lowest lane of this lane's run, cnt
 // the run's length on its head lane and 0 elsewhere.  A run ends at a key

@@ -13,6 +13,7 @@
 #include "pxr_generic.h"
 #include "pxr_kernels.h"
 #include "pxr_leafbin.h"
+#include "pxr_radix.h"
 #include "pxr_runtime.h"
 
 using namespace pxr;
@@ -715,91 +716,65 @@ struct SortGeom {
   i64 nx3, ny3, nbins;
 };
 
-__global__ __launch_bounds__(256) void k_fill_i32(int *p, i64 n, int v) {
-  const i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = v;
-}
-
 __global__ __launch_bounds__(64) void k_fill_u64(unsigned long long *p, i64 n,
                                                  unsigned long long v) {
   const i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) p[t] = v;
 }
 
-// key (0-based bin = reference key - 1), histogram, range check
+// key (0-based bin = reference key - 1) and range check
 __global__ __launch_bounds__(256) void k_sort_keys(i64 np, const double *xp, const double *yp,
                                                    const double *zp, SortGeom s, int *key,
-                                                   int *hist, unsigned long long *bad) {
+                                                   unsigned long long *bad) {
   const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
   if (ip >= np) return;
   const i64 ix = (i64)floor((xp[ip] - s.xmin) * s.dxi);
   const i64 iy = (i64)floor((yp[ip] - s.ymin) * s.dyi);
   const i64 iz = (i64)floor((zp[ip] - s.zmin) * s.dzi);
-  const i64 k = iz * s.nx3 * s.ny3 + iy * s.nx3 + ix;  // reference key - 1 (sorting.F90:304)
+  i64 k = iz * s.nx3 * s.ny3 + iy * s.nx3 + ix;  // reference key - 1 (sorting.F90:304)
   if (k < 0 || k >= s.nbins) {
-    count_bad(bad);
-    key[ip] = -1;
-    return;
+    count_bad(bad);  // nothing will be moved
+    k = 0;
   }
   key[ip] = (int)k;
-  atomicAdd(hist + k, 1);
 }
 
-// exclusive scan of n ints, one workgroup of 1024 lanes (bins of one sort)
-__global__ __launch_bounds__(1024) void k_scan_1wg(int *v, i64 n) {
-  __shared__ int s[1024];
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (i64 base = 0; base < n; base += 1024) {
-    const i64 i = base + threadIdx.x;
-    int x = i < n ? v[i] : 0;
-    s[threadIdx.x] = x;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      int y = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0;
-      __syncthreads();
-      s[threadIdx.x] += y;
-      __syncthreads();
-    }
-    const int incl = s[threadIdx.x];
-    if (i < n) v[i] = carry + incl - x;
-    __syncthreads();
-    if (threadIdx.x == 1023) carry += incl;
-    __syncthreads();
+// The G arrays in sorted order into tmp, and back into the arrays.  Neither
+// moves anything when a key was out of range.
+template <int G> struct SortArrays {
+  double *a[G];
+};
+
+template <int G>
+__global__ __launch_bounds__(256) void k_sort_gather(i64 np, SortArrays<G> s, double *tmp,
+                                                     const int *perm,
+                                                     const unsigned long long *bad) {
+  const i64 j = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= np || *bad) return;
+  const i64 i = perm[j];
+#pragma unroll
+  for (int c = 0; c < G; c++) tmp[c * np + j] = s.a[c][i];
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void k_sort_store(i64 np, SortArrays<G> s, const double *tmp,
+                                                    const unsigned long long *bad) {
+  const i64 j = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= np || *bad) return;
+#pragma unroll
+  for (int c = 0; c < G; c++) s.a[c][j] = tmp[c * np + j];
+}
+
+template <int G>
+static void sort_move(i64 np, double *const *arr, double *tmp, const int *perm,
+                      const unsigned long long *bad, hipStream_t st) {
+  for (int c = 0; c < 8; c += G) {
+    SortArrays<G> s;
+    for (int k = 0; k < G; k++) s.a[k] = arr[c + k];
+    hipLaunchKernelGGL(k_sort_gather<G>, dim3(grid1d(np, 256)), dim3(256), 0, st, np, s, tmp, perm,
+                       bad);
+    hipLaunchKernelGGL(k_sort_store<G>, dim3(grid1d(np, 256)), dim3(256), 0, st, np, s, tmp, bad);
   }
-}
-
-// Stable scatter: destination of every particle, input order preserved
-// among equal keys.  One workgroup walks the particles in rounds of 1024;
-// inside a round each wave ranks its lanes among equal keys (ballot), and
-// the waves take turns, in order, to claim their slots from the bin
-// cursors, so the claim order is the input order.
-__global__ __launch_bounds__(1024) void k_sort_scatter_1wg(i64 np, const int *key, int *cursor,
-                                                          int *dest) {
-  __shared__ int s_slot[1024];
-  const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (i64 base = 0; base < np; base += blockDim.x) {
-    const i64 ip = base + threadIdx.x;
-    const bool act = ip < np;
-    const int k = act ? key[ip] : -1;
-    int rank, cnt, leader_lane;
-    wave_peers(act, k, rank, cnt, leader_lane);
-    for (int w = 0; w < nw; w++) {
-      // storing the returned value makes the wave wait for its atomic
-      // before the barrier, so the claims land in wave order
-      if (w == wave && act && rank == 0) s_slot[threadIdx.x] = atomicAdd(cursor + k, cnt);
-      __syncthreads();
-    }
-    if (act) dest[ip] = s_slot[(wave << 6) + leader_lane] + rank;
-    __syncthreads();
-  }
-}
-
-__global__ __launch_bounds__(256) void k_permute(i64 np, const double *src, double *dst,
-                                                 const int *dest) {
-  const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (ip < np) dst[dest[ip]] = src[ip];
 }
 
 }  // namespace pxr
@@ -1419,17 +1394,35 @@ static int bin_sort_geom(int64_t np2, double *const *arr, int64_t wpid, double x
   return PXRHIP_OK;
 }
 
-// The sort itself, on the library stream, with the caller's buffers: key
-// and dest hold np2 ints, tmp np2 doubles, hist s.nbins ints, bad one
-// counter that is zero on entry and left zero on return.  Keys are checked
-// before anything moves (the host reads the counter, so the call
-// synchronises the stream once).
-static int bin_sort_run(int64_t np2, double *const *arr, const SortGeom &s, int *key, int *hist,
-                        int *dest, double *tmp, unsigned long long *bad_ctr) {
+// Particles up to which the eight arrays are staged together (64 B each):
+// one gather and one store launch in place of eight of each.
+constexpr i64 SORT_GROUP_NP = 1 << 24;
+
+// The sort itself, on the library stream, with the caller's buffers: two
+// key and two index arrays of np2 ints (pairs whose place alternates), hist
+// of plan.hist_ints, tmp of np2 doubles per array staged at a time (eight of
+// them when `group`), bad one counter that is zero on entry and left zero on
+// return.  The sorted indices end in idx[0]; key[1], idx[1] are free by the
+// time tmp is used and may overlap it.  A key out of range leaves the arrays
+// as they are: the moving kernels see the counter, the host reads it at the
+// end (the call synchronises the stream once).
+//
+// One workgroup used to place all particles in order, whatever their number:
+// 8.5 ms of a 8.9 ms call for 1,000,003 particles in 48^3 cells.  The radix
+// sort spreads the ranking over the chip: 0.25 ms for the same call, of which
+// the sort is 0.08 ms, the gather of the eight arrays 0.042 and the store
+// 0.021 ms.
+static int bin_sort_run(int64_t np2, double *const *arr, const SortGeom &s, const RadixPlan &plan,
+                        int *const *key, int *const *idx, int *hist, double *tmp, bool group,
+                        unsigned long long *bad_ctr) {
   hipStream_t st = rt().stream;
-  hipLaunchKernelGGL(k_fill_i32, dim3(grid1d(s.nbins, 256)), dim3(256), 0, st, hist, s.nbins, 0);
+  const int f = plan.npass & 1;  // so that the last pass writes buffers 0
+  int *k2[2] = {key[f], key[f ^ 1]}, *i2[2] = {idx[f], idx[f ^ 1]};
   hipLaunchKernelGGL(k_sort_keys, dim3(grid1d(np2, 256)), dim3(256), 0, st, np2, arr[0], arr[1],
-                     arr[2], s, key, hist, bad_ctr);
+                     arr[2], s, k2[0], bad_ctr);
+  radix_sort(plan, k2, i2, hist, st);
+  if (group) sort_move<8>(np2, arr, tmp, idx[0], bad_ctr, st);
+  else sort_move<1>(np2, arr, tmp, idx[0], bad_ctr, st);
   PXR_LAUNCHED();
   unsigned long long bad = 0;
   PXR_HIP(hipMemcpyAsync(&bad, bad_ctr, sizeof(bad), hipMemcpyDeviceToHost, st));
@@ -1441,19 +1434,12 @@ static int bin_sort_run(int64_t np2, double *const *arr, const SortGeom &s, int 
                      "particle_bin_sorting: %llu particle(s) have a cell key outside [1,%lld]; "
                      "nothing was moved", bad, (long long)s.nbins);
   }
-  hipLaunchKernelGGL(k_scan_1wg, dim3(1), dim3(1024), 0, st, hist, s.nbins);
-  hipLaunchKernelGGL(k_sort_scatter_1wg, dim3(1), dim3(1024), 0, st, np2, key, hist, dest);
-  PXR_LAUNCHED();
-  for (int c = 0; c < 8; c++) {
-    hipLaunchKernelGGL(k_permute, dim3(grid1d(np2, 256)), dim3(256), 0, st, np2, arr[c], tmp, dest);
-    PXR_HIP(hipMemcpyAsync(arr[c], tmp, sizeof(double) * np2, hipMemcpyDeviceToDevice, st));
-  }
-  PXR_LAUNCHED();
   return PXRHIP_OK;
 }
 
-// Fixed device scratch of pxrhip_particle_bin_sorting_noalloc: key, dest,
-// tmp and hist of one sort of at most SORT_NA_NP particles over at most
+// Fixed device scratch of pxrhip_particle_bin_sorting_noalloc: the keys and
+// sorted indices, tmp (which first holds the second pair of them), the digit
+// counts of one sort of at most SORT_NA_NP particles over at most
 // SORT_NA_NBINS bins, and the bad-key counter.  Each GPU holds its own copy
 // until the process ends; calls on one GPU share it.
 constexpr i64 SORT_NA_NP = 1 << 20;
@@ -1501,12 +1487,20 @@ int pxrhip_particle_bin_sorting(int64_t np2, double *xp, double *yp, double *zp,
   int r = bin_sort_geom(np2, arr, wpid, xmin2, ymin2, zmin2, xmax2, ymax2, zmax2, dxf, dyf, dzf, s,
                         empty);
   if (r || empty) return r;
-  int *key = (int *)scratch(0, sizeof(int) * np2);
-  int *hist = (int *)scratch(1, sizeof(int) * s.nbins);
-  int *dest = (int *)scratch(2, sizeof(int) * np2);
-  double *tmp = (double *)scratch(3, sizeof(double) * np2);
-  if (!key || !hist || !dest || !tmp) return set_error(PXRHIP_ERR_HIP, "scratch allocation failed");
-  return bin_sort_run(np2, arr, s, key, hist, dest, tmp, rt().d_bad);
+  const RadixPlan plan = radix_plan(np2, s.nbins, 1 << 20);
+  bool group = np2 <= SORT_GROUP_NP;
+  int *key0 = (int *)scratch(0, sizeof(int) * np2);
+  int *hist = (int *)scratch(1, sizeof(int) * (size_t)plan.hist_ints);
+  int *idx0 = (int *)scratch(2, sizeof(int) * np2);
+  // the staging holds the second pair of keys and indices first
+  double *tmp = (double *)scratch(3, sizeof(double) * (size_t)np2 * (group ? 8 : 1));
+  if (!tmp && group) {
+    group = false;
+    tmp = (double *)scratch(3, sizeof(double) * (size_t)np2);
+  }
+  if (!key0 || !hist || !idx0 || !tmp) return set_error(PXRHIP_ERR_HIP, "scratch allocation failed");
+  int *key[2] = {key0, (int *)tmp}, *idx[2] = {idx0, (int *)tmp + np2};
+  return bin_sort_run(np2, arr, s, plan, key, idx, hist, tmp, group, rt().d_bad);
 }
 
 int pxrhip_particle_bin_sorting_noalloc(int64_t np2, double *xp, double *yp, double *zp,
@@ -1531,8 +1525,11 @@ int pxrhip_particle_bin_sorting_noalloc(int64_t np2, double *xp, double *yp, dou
                      "fixed sort scratch", (long long)s.nbins, (long long)SORT_NA_NBINS);
   unsigned char *base;
   if ((r = sort_scratch_ptr(&base))) return r;
-  return bin_sort_run(np2, arr, s, (int *)base, (int *)(base + SORT_NA_OFF_HIST),
-                      (int *)(base + SORT_NA_OFF_DEST), (double *)(base + SORT_NA_OFF_TMP),
+  const RadixPlan plan = radix_plan(np2, s.nbins, SORT_NA_NBINS);
+  double *tmp = (double *)(base + SORT_NA_OFF_TMP);
+  int *key[2] = {(int *)base, (int *)tmp};
+  int *idx[2] = {(int *)(base + SORT_NA_OFF_DEST), (int *)tmp + SORT_NA_NP};
+  return bin_sort_run(np2, arr, s, plan, key, idx, (int *)(base + SORT_NA_OFF_HIST), tmp, false,
                       (unsigned long long *)(base + SORT_NA_OFF_BAD));
 }
 
