@@ -1057,8 +1057,8 @@ int pxrhip_depose_jxjyjz(double *jx, double *jy, double *jz, int64_t np, const d
   dim3 grd(grid1d(np, 256 * DEP_S)), blk(256);
   hipStream_t st = rt().stream;
   const bool direct = current_depo_algo >= 2;  // depose_jxjyjz_generic CASE(2), CASE(3)
-  if (!direct && leaf_binned_esirkepov_pays(np, a.g)) {
-    r = leaf_binned_esirkepov(a, (int)nox, st);
+  if (leaf_binned_current_pays(np, a.g)) {
+    r = direct ? leaf_binned_direct(a, (int)nox, st) : leaf_binned_esirkepov(a, (int)nox, st);
     if (r) return r;
   } else if (direct) {
     if (nox == 1) hipLaunchKernelGGL(k_direct<1>, grd, blk, 0, st, a);

@@ -42,16 +42,17 @@ struct GlobalAcc {
   PXR_DEV void add_row(double *r, int o, double v) const { unsafeAtomicAdd(r + o, v); }
 };
 
-// Binned forms: the particles are counted into cubic blocks of nodes,
-// ordered by block, and each block's current (or charge) is summed in LDS
+// Binned forms: the particles are ordered by cubic blocks of nodes
+// and each block's current (or charge) is summed in LDS
 // before one global add per node.  Return PXRHIP_OK, or an error code
 // (scratch memory could not be allocated) before anything is launched.
 int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st);
+int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st);
 int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st);
 // whether a call of np particles on grid g takes the binned form: at least
 // the runtime's leaf_bin_min particles and one per block, and no graph
 // capture open (the scratch may have to grow)
-bool leaf_binned_esirkepov_pays(i64 np, const GridGeom &g);
+bool leaf_binned_current_pays(i64 np, const GridGeom &g);
 bool leaf_binned_rho_pays(i64 np, const GridGeom &g);
 
 }  // namespace pxr

@@ -1,26 +1,27 @@
-// pxr_leafbin.hip -- the leaf current and charge deposition (depose_jxjyjz
-// with the Esirkepov current, pxr_depose_rho_n) for large particle sets,
-// summed block by block in LDS.
+// pxr_leafbin.hip -- the leaf current and charge deposition (depose_jxjyjz,
+// pxr_depose_rho_n) for large particle sets, summed block by block in LDS.
 //
 // A caller of the leaf routines hands over particles in any order, anywhere
 // in the grid arrays.  Adding every contribution to global memory costs one
 // FP64 L2 atomic per node and particle (144 for an order-3 Esirkepov
 // particle that keeps its nodes), and those atomics bound the kernel.  Here
-// the particles are first counted into cubic blocks of B^3 nodes (by the
-// node floor(x) of their new position), ordered by block with a counting
-// sort of their indices, and cut into work items of at most `chunk`
-// particles of one block.  A workgroup sums its work item's contributions
-// into an LDS copy of the block with its halo (the nodes that the shapes
-// and one cell of motion reach) and adds the block to the grid array once
-// per non-zero node.
+// the particles are first keyed by cubic blocks of B^3 nodes (by the node
+// floor(x) of their new position, or of the mid position for the direct
+// current), ordered by block with a radix sort of their indices, and cut
+// into work items of at most `chunk` particles of one block.  A workgroup
+// sums its work item's contributions into an LDS copy of the block with its
+// halo (the nodes that the shapes and one cell of motion reach) and adds the
+// block to the grid array once per non-zero node.
 //
 // The contributions are the same arithmetic as the global-atomic kernels
-// (esirkepov_deposit, the nodal shapes of pxr_depose_rho_n); only the order
-// of the FP64 sums differs.  Nothing synchronises with the host, so the
-// sequence can be captured in a HIP graph once its scratch is allocated.
+// (esirkepov_deposit, direct_deposit, the nodal shapes of pxr_depose_rho_n);
+// only the order of the FP64 sums differs.  Nothing synchronises with the
+// host, so the sequence can be captured in a HIP graph once its scratch is
+// allocated.
 #include <algorithm>
 
 #include "pxr_leafbin.h"
+#include "pxr_radix.h"
 #include "pxr_runtime.h"
 
 namespace pxr {
@@ -53,129 +54,72 @@ template <int B> PXR_DEV int block_axis(double x, int g, int na) {
   return ((int)f + g) / B;
 }
 
-__global__ __launch_bounds__(256) void k_lb_fill(int *p, i64 n) {
-  const i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
+// positions (and, for the mid positions, velocities and h = dt / (2 dx)) of
+// one call
+struct LbPos {
+  i64 np;
+  const double *x, *y, *z, *ux, *uy, *uz, *gi;
+  double xmin, ymin, zmin, dxi, dyi, dzi, h[3];
+  int l4symtry;
+};
 
-// Runs of equal keys among a workgroup's particles (keys in skey[0..n),
-// every lane of the workgroup calls): the first lane of lane t's run.  A
-// wave finds the nearest run start at or before each lane from the ballot
-// of run starts; lanes with none in their wave take the last one of the
-// waves before.
-PXR_DEV int lb_run_start(const int *skey, int *wlast, int t, int n) {
-  const int lane = t & 63, w = t >> 6;
-  const bool head = t < n && (t == 0 || skey[t - 1] != skey[t]);
-  const unsigned long long H = __ballot(head);
-  if (lane == 0) wlast[w] = H ? (w << 6) + 63 - __clzll((long long)H) : -1;
-  __syncthreads();
-  const unsigned long long le = lane == 63 ? ~0ull : ((1ull << (lane + 1)) - 1ull);
-  const unsigned long long hb = H & le;
-  if (hb) return (w << 6) + 63 - __clzll((long long)hb);
-  int st = -1;
-  for (int v = 0; v < w; v++) st = max(st, wlast[v]);
-  return st;
-}
-
-// the last lane of a run of equal keys
-PXR_DEV bool lb_run_end(const int *skey, int t, int n) {
-  return t < n && (t == n - 1 || skey[t + 1] != skey[t]);
-}
-
-// Per particle its block, and counts per block.  The counts are kept in
-// `copies` counters per block, workgroup w adding to copy w % copies, and
-// each run of equal keys in a workgroup adds its length with one atomic:
-// cell-ordered input, where consecutive workgroups meet the same blocks,
-// then spreads its few atomics over many addresses.
-template <int B>
-__global__ __launch_bounds__(1024) void k_lb_count(i64 np, const double *xp, const double *yp,
-                                                   const double *zp, double xmin, double ymin,
-                                                   double zmin, double dxi, double dyi,
-                                                   double dzi, int l4symtry, BinGeom bg,
-                                                   int copies, int *key, int *cnt) {
-  __shared__ int skey[1024], wlast[16];
-  const int t = threadIdx.x;
-  const i64 base = (i64)blockIdx.x * 1024, ip = base + t;
-  const int n = (int)min((i64)1024, np - base);
-  int b = -1;
-  if (ip < np) {
-    double x = (xp[ip] - xmin) * dxi, y = (yp[ip] - ymin) * dyi;
-    const double z = (zp[ip] - zmin) * dzi;
-    if (l4symtry) {
-      x = fabs(x);
-      y = fabs(y);
-    }
-    b = block_axis<B>(x, bg.gd[0], bg.na[0]) +
-        bg.nb[0] * (block_axis<B>(y, bg.gd[1], bg.na[1]) +
-                    bg.nb[1] * block_axis<B>(z, bg.gd[2], bg.na[2]));
-    key[ip] = b;
+// Block of every particle, by the node of its position (MID: of its
+// position half a step back, where the direct current is deposited).
+template <int B, bool MID>
+__global__ __launch_bounds__(256) void k_lb_keys(LbPos a, BinGeom bg, int *key) {
+  const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (ip >= a.np) return;
+  double x = (a.x[ip] - a.xmin) * a.dxi, y = (a.y[ip] - a.ymin) * a.dyi;
+  double z = (a.z[ip] - a.zmin) * a.dzi;
+  if (MID) {
+    const double gi = a.gi[ip];
+    x -= a.h[0] * (a.ux[ip] * gi);
+    y -= a.h[1] * (a.uy[ip] * gi);
+    z -= a.h[2] * (a.uz[ip] * gi);
+  } else if (a.l4symtry) {
+    x = fabs(x);
+    y = fabs(y);
   }
-  skey[t] = b;
-  __syncthreads();
-  const int st = lb_run_start(skey, wlast, t, n);
-  if (lb_run_end(skey, t, n)) atomicAdd(cnt + (i64)b * copies + blockIdx.x % copies, t - st + 1);
+  key[ip] = block_axis<B>(x, bg.gd[0], bg.na[0]) +
+            bg.nb[0] * (block_axis<B>(y, bg.gd[1], bg.na[1]) +
+                        bg.nb[1] * block_axis<B>(z, bg.gd[2], bg.na[2]));
 }
 
-// One workgroup: exclusive scan of the counts, block by block and copy by
-// copy, into the copies' first slots (cursor), and the work items (block,
-// first slot, count) of at most `chunk` particles of one block.  Each
-// thread owns a contiguous range of blocks.
-__global__ __launch_bounds__(1024) void k_lb_plan(const int *cnt, i64 nblocks, int copies,
-                                                  int chunk, int *cursor, int4 *items,
-                                                  int *nitems) {
-  __shared__ long long sp[1024], si[1024];
-  const int t = threadIdx.x;
+// first[b]: the first sorted particle of block b (first[nblocks] = np)
+__global__ __launch_bounds__(256) void k_lb_first(i64 np, const int *key, i64 nblocks,
+                                                  int *first) {
+  const i64 j = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j > np) return;
+  const i64 prev = j ? key[j - 1] : -1, here = j < np ? key[j] : nblocks;
+  for (i64 b = prev + 1; b <= here; b++) first[b] = (int)j;
+}
+
+// One workgroup: the work items (block, first slot, count) of at most
+// `chunk` particles of one block.  Each thread owns a contiguous range of
+// blocks.
+__global__ __launch_bounds__(1024) void k_lb_plan(const int *first, i64 nblocks, int chunk,
+                                                  int4 *items, int *nitems) {
+  __shared__ int s[16];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const i64 per = (nblocks + 1023) / 1024;
   const i64 b0 = min(nblocks, (i64)t * per), b1 = min(nblocks, b0 + per);
-  long long np = 0, ni = 0;
+  int ni = 0;
+  for (i64 b = b0; b < b1; b++) ni += (first[b + 1] - first[b] + chunk - 1) / chunk;
+  int inc = ni;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(inc, off);
+    if (lane >= off) inc += y;
+  }
+  if (lane == 63) s[w] = inc;
+  __syncthreads();
+  int it = inc - ni;
+  for (int k = 0; k < w; k++) it += s[k];
   for (i64 b = b0; b < b1; b++) {
-    int c = 0;
-    for (int q = 0; q < copies; q++) c += cnt[b * copies + q];
-    np += c;
-    ni += (c + chunk - 1) / chunk;
+    const int f = first[b], c = first[b + 1] - f;
+    for (int k = 0; k < c; k += chunk) items[it++] = make_int4((int)b, f + k, min(chunk, c - k), 0);
   }
-  sp[t] = np;
-  si[t] = ni;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const long long a = t >= off ? sp[t - off] : 0, c = t >= off ? si[t - off] : 0;
-    __syncthreads();
-    sp[t] += a;
-    si[t] += c;
-    __syncthreads();
-  }
-  long long pos = sp[t] - np, it = si[t] - ni;
-  for (i64 b = b0; b < b1; b++) {
-    const long long first = pos;
-    for (int q = 0; q < copies; q++) {
-      cursor[b * copies + q] = (int)pos;
-      pos += cnt[b * copies + q];
-    }
-    const int c = (int)(pos - first);
-    for (int k = 0; k < c; k += chunk)
-      items[it++] = make_int4((int)b, (int)(first + k), min(chunk, c - k), 0);
-  }
-  if (t == 1023) *nitems = (int)si[1023];
-}
-
-// Particle indices in block order: each run of equal keys in a workgroup
-// claims its slots with one atomic on its copy's cursor (the workgroups
-// and copies of k_lb_count), so a block's slots keep the input order
-// within each run.
-__global__ __launch_bounds__(1024) void k_lb_scatter(i64 np, const int *key, int copies,
-                                                     int *cursor, int *perm) {
-  __shared__ int skey[1024], sbase[1024], wlast[16];
-  const int t = threadIdx.x;
-  const i64 base = (i64)blockIdx.x * 1024, ip = base + t;
-  const int n = (int)min((i64)1024, np - base);
-  const int b = ip < np ? key[ip] : -1;
-  skey[t] = b;
-  __syncthreads();
-  const int st = lb_run_start(skey, wlast, t, n);
-  if (lb_run_end(skey, t, n))
-    sbase[st] = atomicAdd(cursor + (i64)b * copies + blockIdx.x % copies, t - st + 1);
-  __syncthreads();
-  if (ip < np) perm[sbase[st] + (t - st)] = (int)ip;
+  if (t == 1023) *nitems = it;
 }
 
 // LDS block of one work item: nodes [o0, o0 + L) per axis (grid indices)
@@ -271,6 +215,50 @@ __global__ __launch_bounds__(256) void k_lb_esirkepov(DepoArgs a, BinGeom bg, co
   }
 }
 
+// Direct current: the nodes of an order-N particle lie within
+// [floor(m) - 2, floor(m) + 3] of its mid position m (order 1: [-1, +2]) on
+// each axis.
+//
+// Global FP64 atomics bound the unbinned form (k_direct: 24, 81 or 192 adds
+// per particle into L2; 2.75 ms for a million order-2 particles on 64^3
+// cells); here they go to LDS and one add per node and block remains
+// (0.12 ms, and 0.06 ms to key and order the particles).
+template <int N, int B>
+__global__ __launch_bounds__(256) void k_lb_direct(DepoArgs a, BinGeom bg, const int *perm,
+                                                   const int4 *items, const int *nitems) {
+  constexpr int HLO = (N == 1) ? -1 : -2, HHI = (N == 1) ? 2 : 3;
+  extern __shared__ double lds[];
+  const i64 o = a.g.idx(0, 0, 0);
+  const GlobalAcc gacc{{a.jx + o, a.jy + o, a.jz + o}, a.g.NX, a.g.NX * a.g.NY};
+  double *dst[3] = {a.jx, a.jy, a.jz};
+  const int nit = *nitems;
+  for (int w = blockIdx.x; w < nit; w += gridDim.x) {
+    const int4 it = items[w];
+    LdsBlock blk;
+    lb_block<B, HLO, HHI>(bg, it.x, blk, lds, 3);
+    const LdsAccB acc{lds, blk.o[0], blk.o[1], blk.o[2], blk.L, blk.L * blk.L, blk.nodes};
+    const int n = it.z, S = lb_stride(n);
+    for (int k = 0; k < S; k++) {
+      const int p = (int)threadIdx.x * S + k;
+      if (p >= n) break;
+      const i64 ip = perm[it.y + p];
+      DirectIn<double> in;
+      direct_prepare<N, double>(in, a.xp[ip], a.yp[ip], a.zp[ip], a.ux[ip], a.uy[ip], a.uz[ip],
+                                a.gi[ip], a.w[ip], a.q, a.xmin, a.ymin, a.zmin, a.dt, a.dx, a.dy,
+                                a.dz, a.s);
+      int lo[3], hi[3];
+      direct_box<N>(in, lo, hi);
+      if (!a.g.inside(lo[0], lo[1], lo[2]) || !a.g.inside(hi[0], hi[1], hi[2])) {
+        count_bad(a.bad);
+        continue;
+      }
+      if (blk.holds(lo, hi)) direct_deposit<N, double>(in, acc);
+      else direct_deposit<N, double>(in, gacc);  // not reached: the halo holds every box
+    }
+    lb_flush(blk, a.g, dst, 3);
+  }
+}
+
 // charge density: nodes [floor(x) - 1, floor(x) + 2] (order 1: [0, 1])
 template <int N, int B>
 __global__ __launch_bounds__(256) void k_lb_rho(RhoArgs a, BinGeom bg, const int *perm,
@@ -325,34 +313,35 @@ __global__ __launch_bounds__(256) void k_lb_rho(RhoArgs a, BinGeom bg, const int
   }
 }
 
-// counting sort of the particle indices by block; work items into *items
-template <int B>
-static int lb_sort(i64 np, const double *xp, const double *yp, const double *zp, double xmin,
-                   double ymin, double zmin, double dxi, double dyi, double dzi, int l4symtry,
-                   const GridGeom &g, int chunk, hipStream_t st, BinGeom &bg, int *&perm,
-                   int4 *&items, int *&nitems, i64 &maxitems) {
+// Particle indices in block order (radix sort: the input order is kept
+// inside a block) and the work items.  Counting and placing the particles
+// with global atomics on the blocks' counters took 0.32 ms for two million
+// in random order (every particle its own atomic), this 0.09 ms.
+template <int B, bool MID>
+static int lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st, BinGeom &bg,
+                   int *&perm, int4 *&items, int *&nitems, i64 &maxitems) {
   bg = make_bin_geom(g, B);
+  const i64 np = a.np;
   maxitems = bg.nblocks + np / chunk + 1;
   if (np >= (i64)1 << 31 || bg.nblocks >= (i64)1 << 31 || maxitems >= (i64)1 << 31)
     return set_error(PXRHIP_ERR_ARG, "binned deposition: more than 2^31 particles or blocks");
-  // counters per block: up to 16 copies while they stay below 2^18
-  const int copies = (int)std::max<i64>(1, std::min<i64>(16, ((i64)1 << 18) / bg.nblocks));
-  const i64 ncnt = bg.nblocks * copies;
-  int *key = (int *)scratch(24, sizeof(int) * (size_t)np);
-  perm = (int *)scratch(25, sizeof(int) * (size_t)np);
-  int *cnt = (int *)scratch(26, sizeof(int) * (size_t)ncnt);
-  int *cursor = (int *)scratch(27, sizeof(int) * (size_t)ncnt);
+  const RadixPlan plan = radix_plan(np, bg.nblocks, (i64)1 << 21);
+  int *keys = (int *)scratch(24, 2 * sizeof(int) * (size_t)np);
+  int *idxs = (int *)scratch(25, 2 * sizeof(int) * (size_t)np);
+  int *hist = (int *)scratch(26, sizeof(int) * (size_t)plan.hist_ints);
+  int *first = (int *)scratch(27, sizeof(int) * (size_t)(bg.nblocks + 1));
   items = (int4 *)scratch(28, sizeof(int4) * (size_t)maxitems);
   nitems = (int *)scratch(29, sizeof(int));
-  if (!key || !perm || !cnt || !cursor || !items || !nitems)
+  if (!keys || !idxs || !hist || !first || !items || !nitems)
     return set_error(PXRHIP_ERR_HIP, "binned deposition: out of device memory");
-  hipLaunchKernelGGL(k_lb_fill, dim3(grid1d(ncnt, 256)), dim3(256), 0, st, cnt, ncnt);
-  hipLaunchKernelGGL(k_lb_count<B>, dim3(grid1d(np, 1024)), dim3(1024), 0, st, np, xp, yp, zp,
-                     xmin, ymin, zmin, dxi, dyi, dzi, l4symtry, bg, copies, key, cnt);
-  hipLaunchKernelGGL(k_lb_plan, dim3(1), dim3(1024), 0, st, cnt, bg.nblocks, copies, chunk,
-                     cursor, items, nitems);
-  hipLaunchKernelGGL(k_lb_scatter, dim3(grid1d(np, 1024)), dim3(1024), 0, st, np, key, copies,
-                     cursor, perm);
+  int *key[2] = {keys, keys + np}, *idx[2] = {idxs, idxs + np};
+  hipLaunchKernelGGL((k_lb_keys<B, MID>), dim3(grid1d(np, 256)), dim3(256), 0, st, a, bg, keys);
+  const int at = radix_sort(plan, key, idx, hist, st);
+  perm = idx[at];
+  hipLaunchKernelGGL(k_lb_first, dim3(grid1d(np + 1, 256)), dim3(256), 0, st, np, key[at],
+                     bg.nblocks, first);
+  hipLaunchKernelGGL(k_lb_plan, dim3(1), dim3(1024), 0, st, first, bg.nblocks, chunk, items,
+                     nitems);
   PXR_LAUNCHED();
   return PXRHIP_OK;
 }
@@ -380,8 +369,29 @@ static bool pays(i64 np, const GridGeom &g, int edge) {
          np >= make_bin_geom(g, edge).nblocks;
 }
 
-bool leaf_binned_esirkepov_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
+bool leaf_binned_current_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
 bool leaf_binned_rho_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
+
+int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st) {
+  BinGeom bg;
+  int *perm, *nitems;
+  int4 *items;
+  i64 maxitems;
+  const EsirkConst<double> &c = a.ec;
+  const LbPos pos{a.np, a.xp, a.yp, a.zp, a.ux, a.uy, a.uz, a.gi, c.xmin, c.ymin, c.zmin, c.dxi,
+                  c.dyi, c.dzi, {0.5 * c.dtsdx0, 0.5 * c.dtsdy0, 0.5 * c.dtsdz0}, 0};
+  int r = lb_sort<LB_EDGE, true>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems,
+                                 maxitems);
+  if (r) return r;
+  const int L = LB_EDGE + (order == 1 ? 3 : 5);
+  const size_t lds = sizeof(double) * 3 * (size_t)(L * L * L);
+  const dim3 grd(lb_grid(maxitems, lds)), blk(256);
+  if (order == 1) LB_LAUNCH((k_lb_direct<1, LB_EDGE>), a);
+  else if (order == 2) LB_LAUNCH((k_lb_direct<2, LB_EDGE>), a);
+  else LB_LAUNCH((k_lb_direct<3, LB_EDGE>), a);
+  PXR_LAUNCHED();
+  return PXRHIP_OK;
+}
 
 int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st) {
   BinGeom bg;
@@ -389,8 +399,10 @@ int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st) {
   int4 *items;
   i64 maxitems;
   const EsirkConst<double> &c = a.ec;
-  int r = lb_sort<LB_EDGE>(a.np, a.xp, a.yp, a.zp, c.xmin, c.ymin, c.zmin, c.dxi, c.dyi, c.dzi, 0,
-                           a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems, maxitems);
+  const LbPos pos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, c.xmin, c.ymin,
+                  c.zmin, c.dxi, c.dyi, c.dzi, {0.0, 0.0, 0.0}, 0};
+  int r = lb_sort<LB_EDGE, false>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems,
+                                  maxitems);
   if (r) return r;
   const int L = LB_EDGE + (order == 1 ? 3 : 5);
   const size_t lds = sizeof(double) * 3 * (size_t)(L * L * L);
@@ -408,8 +420,9 @@ int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st) {
   int *perm, *nitems;
   int4 *items;
   i64 maxitems;
-  int r = lb_sort<E>(a.np, a.xp, a.yp, a.zp, a.xmin, a.ymin, a.zmin, a.dxi, a.dyi, a.dzi,
-                     a.l4symtry, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems, maxitems);
+  const LbPos pos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, a.xmin, a.ymin,
+                  a.zmin, a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, a.l4symtry};
+  int r = lb_sort<E, false>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems, maxitems);
   if (r) return r;
   const int L = E + (order == 1 ? 1 : 3);
   const size_t lds = sizeof(double) * (size_t)(L * L * L);
