@@ -16,6 +16,7 @@
 #include <limits.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "pxr_device.h"
@@ -466,13 +467,23 @@ __global__ __launch_bounds__(1024) void k_scan_i64_1wg(i64 *v, i64 nb, i64 *tota
 // a single pair of banks).
 __device__ __forceinline__ int scan_slot(int e) { return e + (e >> 4); }
 
+// SELF: boff holds the blocks' own sums, and each block adds up those before
+// it (see scan_counts).
+template <bool SELF>
 __global__ __launch_bounds__(256) void k_scan_apply(const int *in, i64 n, const i64 *boff,
                                                     i64 *out, i64 *cursor) {
   constexpr int PER = SCAN_B / 256;
   __shared__ i64 sv[SCAN_B + SCAN_B / 16];
-  __shared__ i64 s[4];
+  __shared__ i64 s[4], sb[4];
   const i64 b0 = (i64)blockIdx.x * SCAN_B;
   const int t = (int)threadIdx.x;
+  if (SELF) {
+    i64 acc = 0;
+    for (int k = t; k < (int)blockIdx.x; k += 256) acc += boff[k];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
+    if ((t & 63) == 0) sb[t >> 6] = acc;
+  }
 #pragma unroll
   for (int k = 0; k < PER; k++) {
     const i64 i = b0 + k * 256 + t;
@@ -495,7 +506,7 @@ __global__ __launch_bounds__(256) void k_scan_apply(const int *in, i64 n, const 
   __syncthreads();
   i64 wbase = 0;
   for (int w = 0; w < wv; w++) wbase += s[w];
-  i64 run = boff[blockIdx.x] + wbase + inc - acc;
+  i64 run = (SELF ? sb[0] + sb[1] + sb[2] + sb[3] : boff[blockIdx.x]) + wbase + inc - acc;
 #pragma unroll
   for (int k = 0; k < PER; k++) {
     const int e = scan_slot(t * PER + k);
@@ -513,6 +524,24 @@ __global__ __launch_bounds__(256) void k_scan_apply(const int *in, i64 n, const 
       out[i] = v;
       if (cursor) cursor[i] = v;
     }
+  }
+}
+
+// out[0..n] = exclusive scan of n counts (and cursor[0..n) = out); bsum: one
+// value per SCAN_B counts.  Up to SCAN_SELF blocks each sums the blocks before
+// it itself; beyond that the sums are scanned by a launch of their own (4.5 us,
+// as much as the others at small sizes).
+constexpr i64 SCAN_SELF = 2048;
+
+static void scan_counts(const int *in, i64 n, i64 *bsum, i64 *out, i64 *cursor, hipStream_t st) {
+  const i64 nblk = (n + SCAN_B - 1) / SCAN_B;
+  const dim3 grd((unsigned)nblk), blk(256);
+  hipLaunchKernelGGL(k_scan_blocks, grd, blk, 0, st, in, n, bsum);
+  if (nblk <= SCAN_SELF) {
+    hipLaunchKernelGGL(k_scan_apply<true>, grd, blk, 0, st, in, n, bsum, out, cursor);
+  } else {
+    hipLaunchKernelGGL(k_scan_i64_1wg, dim3(1), dim3(1024), 0, st, bsum, nblk, (i64 *)nullptr);
+    hipLaunchKernelGGL(k_scan_apply<false>, grd, blk, 0, st, in, n, bsum, out, cursor);
   }
 }
 
@@ -1170,13 +1199,14 @@ static int build_chunks(const TileTable *tt, const pxrhip_species *sp, const Box
   ca.bad = rt().d_bad;
   ca.jroom = jroom;
   ca.sk4 = sk4;
-  hipLaunchKernelGGL(k_chunk_groups, dim3(grid1d(tt->ntiles, 64)), dim3(64), 0, st, ca);
-  hipLaunchKernelGGL(k_chunk_count, dim3(grid1d(nunits, 256)), dim3(256), 0, st, ca);
-  hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nblk), dim3(256), 0, st, cnt, nunits, bsum);
-  hipLaunchKernelGGL(k_scan_i64_1wg, dim3(1), dim3(1024), 0, st, bsum, nblk, (i64 *)nullptr);
-  hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nblk), dim3(256), 0, st, cnt, nunits, bsum,
-                     cstart, (i64 *)nullptr);
-  hipLaunchKernelGGL(k_chunk_write, dim3(grid1d(nunits, 256)), dim3(256), 0, st, ca);
+  hipLaunchKernelGGL(k_chunk_groups, dim3(grid1d((i64)tt->ntiles * CG, 256)), dim3(256), 0, st, ca);
+  hipLaunchKernelGGL(k_chunk_count, dim3(grid1d(nunits * CG, 256)), dim3(256), 0, st, ca);
+  if (nunits <= CHUNK_SELF_SCAN) {
+    ca.start = nullptr;
+  } else {
+    scan_counts(cnt, nunits, bsum, cstart, nullptr, st);
+  }
+  hipLaunchKernelGGL(k_chunk_write, dim3(grid1d(nunits * CG, 256)), dim3(256), 0, st, ca);
   PXR_LAUNCHED();
   *chunks_out = chunks;
   *ctl_out = ctl;
@@ -1436,7 +1466,10 @@ int pxrhip_tiles_rebin_sort(const pxrhip_grid *grid, pxrhip_species *src, pxrhip
   const i64 nbins = tt->nbins;
   hipStream_t st = rt().stream;
   int *key = (int *)scratch(4, sizeof(int) * (size_t)(cap > 1 ? cap : 1));
-  int *hist = (int *)scratch(5, sizeof(int) * (size_t)nbins);
+  // counts of the bins, flags of the bins to order, and the number of those
+  // listed for k_rb_order_big: cleared in one launch
+  int *hist = (int *)scratch(5, sizeof(int) * (size_t)(2 * nbins + 1));
+  int *flag = hist + nbins;
   const i64 nblk = (nbins + SCAN_B - 1) / SCAN_B;
   i64 *bsum = (i64 *)scratch(6, sizeof(i64) * (size_t)(nblk + 1));
   unsigned long long *cursor = (unsigned long long *)scratch(7, sizeof(i64) * (size_t)nbins);
@@ -1456,13 +1489,11 @@ int pxrhip_tiles_rebin_sort(const pxrhip_grid *grid, pxrhip_species *src, pxrhip
   a.key = key;
   a.hist = hist;
   a.bad = rt().d_bad;
-  hipLaunchKernelGGL(k_fill_i32_t, dim3(grid1d(nbins, 256)), dim3(256), 0, st, hist, nbins);
+  hipLaunchKernelGGL(k_fill_i32_t, dim3(grid1d(2 * nbins + 1, 256)), dim3(256), 0, st, hist,
+                     2 * nbins + 1);
   hipLaunchKernelGGL(k_rb_keys, dim3(grid1d((cap + RB_ILP - 1) / RB_ILP, 256)), dim3(256), 0, st, a,
                      cap);
-  hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nblk), dim3(256), 0, st, hist, nbins, bsum);
-  hipLaunchKernelGGL(k_scan_i64_1wg, dim3(1), dim3(1024), 0, st, bsum, nblk, (i64 *)nullptr);
-  hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nblk), dim3(256), 0, st, hist, nbins, bsum,
-                     (i64 *)dst->bin_start, (i64 *)cursor);
+  scan_counts(hist, nbins, bsum, (i64 *)dst->bin_start, (i64 *)cursor, st);
   ScatterArgs sa;
   double *S[3] = {src->x, src->y, src->z}, *D[3] = {dst->x, dst->y, dst->z};
   void *SQ[5] = {src->ux, src->uy, src->uz, src->gaminv, src->w};
@@ -1487,16 +1518,29 @@ int pxrhip_tiles_rebin_sort(const pxrhip_grid *grid, pxrhip_species *src, pxrhip
   sa.cursor = cursor;
   if (g_tune.stable_rebin) {
     int *perm = (int *)scratch(16, sizeof(int) * (size_t)(cap > 1 ? cap : 1));
-    int *flag = (int *)scratch(18, sizeof(int) * (size_t)nbins);  // bins to order
-    if (!perm || !flag) return set_error(PXRHIP_ERR_HIP, "scratch allocation failed");
-    hipLaunchKernelGGL(k_fill_i32_t, dim3(grid1d(nbins, 256)), dim3(256), 0, st, flag, nbins);
+    const i64 maxbig = std::min<i64>(nbins, cap / RB_SMALL + 1);
+    int *big = (int *)scratch(17, sizeof(int) * (size_t)maxbig);
+    if (!perm || !big) return set_error(PXRHIP_ERR_HIP, "scratch allocation failed");
     hipLaunchKernelGGL(k_rb_slots, dim3(grid1d((cap + RB_ILP_SLOTS - 1) / RB_ILP_SLOTS, 256)),
                        dim3(256), 0, st,
                        (const int *)key,
                        (const int64_t *)src->tile_off, tt->ntiles, cursor,
                        (const i64 *)dst->bin_start, flag, perm, cap);
-    hipLaunchKernelGGL(k_rb_order, dim3(grid1d(nbins, 256)), dim3(256), 0, st,
-                       (const i64 *)dst->bin_start, nbins, flag, perm);
+    OrderArgs oa;
+    oa.bin_start = (const i64 *)dst->bin_start;
+    oa.nbins = nbins;
+    oa.flag = flag;
+    oa.perm = perm;
+    oa.big = big;
+    oa.nbig = flag + nbins;
+    oa.ntiles = tt->ntiles;
+    oa.bin_base = tt->bin_base;
+    oa.off = dst->tile_off;
+    oa.np = dst->tile_np;
+    hipLaunchKernelGGL(k_rb_order, dim3(grid1d(nbins > tt->ntiles ? nbins : tt->ntiles + 1, 256)),
+                       dim3(256), 0, st, oa);
+    hipLaunchKernelGGL(k_rb_order_big, dim3((unsigned)std::min<i64>(maxbig, 4 * rt().num_cus)),
+                       dim3(256), 0, st, (const i64 *)dst->bin_start, big, oa.nbig, perm);
     GatherArgs ga;
     for (int k = 0; k < 3; k++) {
       ga.src[k] = S[k];
