@@ -409,6 +409,7 @@ struct NorderArgs {
   double mudt;
   Coefs co;
   int nxs, nys, nzs, ist;
+  int zchunk;  // planes per thread of k_norder_z
 };
 
 PXR_DEV int imin3(int a, int b, int c) { return min(min(a, b), c); }
@@ -505,16 +506,14 @@ __global__ __launch_bounds__(256) void k_norder(NorderArgs a) {
 
 // Register-blocked form for a full stencil of NH terms on every axis and a
 // staggering shift IST known at compile time.  A thread owns one (x, y)
-// column of the loop box and marches up ZCHUNK planes of it.  The two fields
+// column of the loop box and marches up a.zchunk planes of it.  The two fields
 // differenced along z (B_y and B_x for E; E_y and E_x for B) are kept as a
 // window of 2 NH + 1 planes in registers, so each plane of them is loaded
 // once; the x and y differences read the plane from memory (neighbouring
 // lanes and the block's rows share those lines in L1/L2).  Nodes whose
 // stencil is cut at the guards take the per-node form.  The terms are
 // summed in the reference's order, so the results equal k_norder's.
-#ifndef ZCHUNK
-#define ZCHUNK 64  // planes per thread
-#endif
+constexpr int ZCHUNK = 64;  // most planes per thread
 #ifndef ZBX
 #define ZBX 64     // columns of a block along x (256 / ZBX along y)
 #endif
@@ -526,8 +525,8 @@ __global__ __launch_bounds__(256) void k_norder_z(NorderArgs a) {
   const int ku = (int)blockIdx.y * (256 / ZBX) + (int)(threadIdx.x / ZBX);
   if (ju >= nxu || ku >= nyu) return;
   const int j = -a.nxs + ju, k = -a.nys + ku;
-  const int l0 = -a.nzs + (int)blockIdx.z * ZCHUNK;
-  const int l1 = min(l0 + ZCHUNK, -a.nzs + nzu);  // exclusive
+  const int l0 = -a.nzs + (int)blockIdx.z * a.zchunk;
+  const int l1 = min(l0 + a.zchunk, -a.nzs + nzu);  // exclusive
   const int nxh = imin3(a.co.nh[0], (g.nx - j) + g.gx, j + g.gx);
   const int nyh = imin3(a.co.nh[1], (g.ny - k) + g.gy, k + g.gy);
   // planes whose z stencil is whole: -gz + NH .. nz + gz - NH
