@@ -80,6 +80,8 @@ int pxrhip_memcpy_htod(void *dst, const void *src, int64_t bytes);
 int pxrhip_memcpy_dtoh(void *dst, const void *src, int64_t bytes);
 int pxrhip_memcpy_dtod(void *dst, const void *src, int64_t bytes);
 int pxrhip_fill_f64(double *p, int64_t n, double value);
+/* three arrays of n values, in one launch */
+int pxrhip_fill_f64_vec(double *p0, double *p1, double *p2, int64_t n, double value);
 int pxrhip_fill_i64(int64_t *p, int64_t n, int64_t value);
 /* dst[i] = (double)src[i]: the weights of a mixed-precision species for
  * routines that take FP64 arrays (the charge density) */
@@ -254,10 +256,20 @@ int pxrhip_push_em3d_bvec_norder(
  * (field_boundaries.F90:81-260) when every neighbour is the rank itself. */
 int pxrhip_field_bc_periodic(double *field, int64_t nx, int64_t ny, int64_t nz,
                              int64_t nxg, int64_t nyg, int64_t nzg);
+/* the same for the three components of a field (efield_bcs, bfield_bcs,
+ * field_boundaries.F90:1757, 1808) */
+int pxrhip_field_bc_periodic_vec(double *fx, double *fy, double *fz, int64_t nx,
+                                 int64_t ny, int64_t nz, int64_t nxg,
+                                 int64_t nyg, int64_t nzg);
 /* summation_bcs (field_boundaries.F90:403-500) on one periodic rank. */
 int pxrhip_current_bc_periodic(double *array, int64_t nx, int64_t ny,
                                int64_t nz, int64_t nxg, int64_t nyg,
                                int64_t nzg);
+/* the same for the three components of the current (current_bcs,
+ * field_boundaries.F90:1861) */
+int pxrhip_current_bc_periodic_vec(double *jx, double *jy, double *jz,
+                                   int64_t nx, int64_t ny, int64_t nz,
+                                   int64_t nxg, int64_t nyg, int64_t nzg);
 
 /* ---- sorting ------------------------------------------------------------- */
 /* pxr_particle_bin_sorting, sorting.F90:247-361: stable counting sort of

@@ -39,6 +39,7 @@ SIGNATURES = {
     "pxrhip_memcpy_dtoh": [_P, _P, _I],
     "pxrhip_memcpy_dtod": [_P, _P, _I],
     "pxrhip_fill_f64": [_P, _I, _F],
+    "pxrhip_fill_f64_vec": [_P] * 3 + [_I, _F],
     "pxrhip_fill_i64": [_P, _I, _I],
     "pxrhip_convert_f32_f64": [_P, _P, _I],
     "pxrhip_timer_record": [_i32],
@@ -66,7 +67,9 @@ SIGNATURES = {
     "pxrhip_push_em3d_evec_norder": [_P] * 9 + [_F] + [_P] * 3 + [_I] * 13,
     "pxrhip_push_em3d_bvec_norder": [_P] * 6 + [_P] * 3 + [_I] * 13,
     "pxrhip_field_bc_periodic": [_P] + [_I] * 6,
+    "pxrhip_field_bc_periodic_vec": [_P] * 3 + [_I] * 6,
     "pxrhip_current_bc_periodic": [_P] + [_I] * 6,
+    "pxrhip_current_bc_periodic_vec": [_P] * 3 + [_I] * 6,
     "pxrhip_particle_bin_sorting": [_I] + [_P] * 8 + [_I] + [_F] * 9,
     "pxrhip_particle_bin_sorting_noalloc": [_I] + [_P] * 8 + [_I] + [_F] * 9,
     "pxrhip_laserp_pusher_gaussian": [_I, _I] + [_P] * 8 + [_F, _I] + [_F] * 3 + [_P, _P, _F, _P]

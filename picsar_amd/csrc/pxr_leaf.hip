@@ -600,12 +600,21 @@ __global__ __launch_bounds__(256) void k_norder_z(NorderArgs a) {
   for (int l = max(m1, l0); l < l1; l++) node(l);
 }
 
+// Planes per thread: 64 where that leaves at least four blocks per CU, else
+// halved until it does (a column then primes its window of 2 NH planes more
+// often, but a grid of 96 x 96 x 192 would run 200 blocks on 256 CUs).
+// Measured at order 4 on 96 x 96 x 192: B half step 152, now 42 us, E step 144,
+// now 53 us (8 planes per thread); 512 x 512 x 1024 keeps 64, where 32 was 1-7%
+// slower.
 template <int NH, bool E>
-static void launch_norder_z(const NorderArgs &a, hipStream_t st) {
+static void launch_norder_z(NorderArgs a, hipStream_t st) {
   const int nxu = a.g.nx + 2 * a.nxs + 1, nyu = a.g.ny + 2 * a.nys + 1;
   const int nzu = a.g.nz + 2 * a.nzs + 1;
-  const dim3 gr((nxu + ZBX - 1) / ZBX, (nyu + 256 / ZBX - 1) / (256 / ZBX),
-               (nzu + ZCHUNK - 1) / ZCHUNK), bl(256);
+  const i64 bx = (nxu + ZBX - 1) / ZBX, by = (nyu + 256 / ZBX - 1) / (256 / ZBX);
+  a.zchunk = ZCHUNK;
+  while (a.zchunk > 4 && bx * by * ((nzu + a.zchunk - 1) / a.zchunk) < 4 * (i64)rt().num_cus)
+    a.zchunk /= 2;
+  const dim3 gr((unsigned)bx, (unsigned)by, (unsigned)((nzu + a.zchunk - 1) / a.zchunk)), bl(256);
   if (a.ist) hipLaunchKernelGGL((k_norder_z<NH, E, 1>), gr, bl, 0, st, a);
   else hipLaunchKernelGGL((k_norder_z<NH, E, 0>), gr, bl, 0, st, a);
 }
@@ -636,40 +645,51 @@ static void launch_norder(const NorderArgs &a, bool e, i64 tot) {
 // ---------------------------------------------------------------------------
 // periodic guards on one rank
 // ---------------------------------------------------------------------------
-// One axis of field_bc: nodes n..n+g take nodes 0..g, nodes -g..-1 take
-// n-g..n-1 (node 0 is unchanged: it receives node n, itself a copy of 0).
-__global__ __launch_bounds__(256) void k_field_bc_axis(double *f, GridGeom g, int axis) {
-  int n = axis == 0 ? g.nx : axis == 1 ? g.ny : g.nz;
-  int gg = axis == 0 ? g.gx : axis == 1 ? g.gy : g.gz;
-  const int e0 = g.nx + 1 + 2 * g.gx, e1 = g.ny + 1 + 2 * g.gy, e2 = g.nz + 1 + 2 * g.gz;
-  int ext[3] = {e0, e1, e2};
-  ext[axis] = 2 * gg + 1;  // gg nodes below, gg+1 nodes from n up
-  const i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (i64)ext[0] * ext[1] * ext[2]) return;
+// the arrays of one guard call: one, or the three components of a field
+struct GuardArrays {
+  double *p[3];
+};
+
+// field_bc on all axes: nodes n..n+g take nodes 0..g and nodes -g..-1 take
+// n-g..n-1 on x, then y, then z, which leaves every node outside 0..n-1 with
+// the value of the node 0..n-1 that it is a periodic image of.  The shell is
+// walked as three slabs (z planes whole, then y rows of the inner planes,
+// then x ends of the inner rows); no node it reads is written.  Bound by its
+// launch: one launch for a field in place of nine of 4-5 us each (three
+// axes, three components).
+__global__ __launch_bounds__(256) void k_field_bc(GuardArrays a, GridGeom g) {
+  const i64 e0 = g.NX, e1 = g.NY;
+  const i64 nzs = e0 * e1 * (2 * g.gz + 1), nys = e0 * (2 * g.gy + 1) * g.nz;
+  const i64 nxs = (i64)(2 * g.gx + 1) * g.ny * g.nz;
+  i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nzs + nys + nxs) return;
+  // r-th node outside 0..n-1: -w..-1, then n..n+w
+  auto outer = [](int r, int w, int n) { return r < w ? r - w : n + r - w; };
   int c[3];
-  c[0] = (int)(t % ext[0]);
-  c[1] = (int)((t / ext[0]) % ext[1]);
-  c[2] = (int)(t / ((i64)ext[0] * ext[1]));
-  int lo[3] = {-g.gx, -g.gy, -g.gz};
-  for (int d = 0; d < 3; d++) c[d] += lo[d];
-  // along the axis: r in [-gg, gg]; r < 0 -> node r (lower guard) gets r+n;
-  // r >= 0 -> node n+r gets r
-  int r = c[axis];
-  int dst[3] = {c[0], c[1], c[2]}, src[3] = {c[0], c[1], c[2]};
-  if (r < 0) {
-    dst[axis] = r;
-    src[axis] = r + n;
+  if (t < nzs) {
+    c[0] = (int)(t % e0) - g.gx;
+    c[1] = (int)(t / e0 % e1) - g.gy;
+    c[2] = outer((int)(t / (e0 * e1)), g.gz, g.nz);
+  } else if ((t -= nzs) < nys) {
+    c[0] = (int)(t % e0) - g.gx;
+    c[1] = outer((int)(t / e0 % (2 * g.gy + 1)), g.gy, g.ny);
+    c[2] = (int)(t / (e0 * (2 * g.gy + 1)));
   } else {
-    dst[axis] = n + r;
-    src[axis] = r;
+    t -= nys;
+    c[0] = outer((int)(t % (2 * g.gx + 1)), g.gx, g.nx);
+    c[1] = (int)(t / (2 * g.gx + 1) % g.ny);
+    c[2] = (int)(t / ((i64)(2 * g.gx + 1) * g.ny));
   }
-  f[g.idx(dst[0], dst[1], dst[2])] = f[g.idx(src[0], src[1], src[2])];
+  auto image = [](int i, int n) { return i < 0 ? i + n : i >= n ? i - n : i; };
+  double *f = a.p[blockIdx.y];
+  f[g.idx(c[0], c[1], c[2])] = f[g.idx(image(c[0], g.nx), image(c[1], g.ny), image(c[2], g.nz))];
 }
 
 // One axis of summation_bcs: a(0:g) += a(n:n+g); then a(n-g:n) += a(-g:0)
 // with a(0) already updated.  Written per node in closed form; node 0 and
 // node n are handled by one lane since each reads the other.
-__global__ __launch_bounds__(256) void k_current_bc_axis(double *a, GridGeom g, int axis) {
+__global__ __launch_bounds__(256) void k_current_bc_axis(GuardArrays arr, GridGeom g, int axis) {
+  double *a = arr.p[blockIdx.y];
   int n = axis == 0 ? g.nx : axis == 1 ? g.ny : g.nz;
   int gg = axis == 0 ? g.gx : axis == 1 ? g.gy : g.gz;
   int ext[3] = {g.nx + 1 + 2 * g.gx, g.ny + 1 + 2 * g.gy, g.nz + 1 + 2 * g.gz};
@@ -1325,44 +1345,72 @@ int pxrhip_push_em3d_bvec_norder(const double *ex, const double *ey, const doubl
   return PXRHIP_OK;
 }
 
-int pxrhip_field_bc_periodic(double *f, int64_t nx, int64_t ny, int64_t nz, int64_t nxg,
-                             int64_t nyg, int64_t nzg) {
-  PXR_INIT();
+static int guard_args(double *const *p, int ncomp, int64_t nx, int64_t ny, int64_t nz,
+                      int64_t nxg, int64_t nyg, int64_t nzg, GuardArrays &a, GridGeom &g) {
   int r = check_grid(nx, ny, nz, nxg, nyg, nzg);
   if (r) return r;
-  if (!f) return set_error(PXRHIP_ERR_ARG, "null array");
+  for (int c = 0; c < 3; c++) {
+    a.p[c] = p[c < ncomp ? c : 0];
+    if (!a.p[c]) return set_error(PXRHIP_ERR_ARG, "null array");
+  }
   if (nx <= 2 * nxg || ny <= 2 * nyg || nz <= 2 * nzg)
     return set_error(PXRHIP_ERR_UNSUPPORTED, "periodic guards need n > 2*guards on every axis");
-  GridGeom g = mkgeom(nx, ny, nz, nxg, nyg, nzg);
+  g = mkgeom(nx, ny, nz, nxg, nyg, nzg);
+  return PXRHIP_OK;
+}
+
+static int field_bc(double *const *p, int ncomp, int64_t nx, int64_t ny, int64_t nz, int64_t nxg,
+                    int64_t nyg, int64_t nzg) {
+  PXR_INIT();
+  GuardArrays a;
+  GridGeom g;
+  int r = guard_args(p, ncomp, nx, ny, nz, nxg, nyg, nzg, a, g);
+  if (r) return r;
+  const i64 tot = g.NX * g.NY * (2 * nzg + 1) + g.NX * (2 * nyg + 1) * nz + (2 * nxg + 1) * ny * nz;
+  hipLaunchKernelGGL(k_field_bc, dim3(grid1d(tot, 256), ncomp), dim3(256), 0, rt().stream, a, g);
+  PXR_LAUNCHED();
+  return PXRHIP_OK;
+}
+
+static int current_bc(double *const *p, int ncomp, int64_t nx, int64_t ny, int64_t nz,
+                      int64_t nxg, int64_t nyg, int64_t nzg) {
+  PXR_INIT();
+  GuardArrays a;
+  GridGeom g;
+  int r = guard_args(p, ncomp, nx, ny, nz, nxg, nyg, nzg, a, g);
+  if (r) return r;
   const int64_t ext[3] = {nx + 1 + 2 * nxg, ny + 1 + 2 * nyg, nz + 1 + 2 * nzg};
   const int64_t gg[3] = {nxg, nyg, nzg};
   for (int ax = 0; ax < 3; ax++) {
     int64_t tot = 1;
     for (int d = 0; d < 3; d++) tot *= (d == ax) ? 2 * gg[d] + 1 : ext[d];
-    hipLaunchKernelGGL(k_field_bc_axis, dim3(grid1d(tot, 256)), dim3(256), 0, rt().stream, f, g, ax);
+    hipLaunchKernelGGL(k_current_bc_axis, dim3(grid1d(tot, 256), ncomp), dim3(256), 0, rt().stream,
+                       a, g, ax);
     PXR_LAUNCHED();
   }
   return PXRHIP_OK;
 }
 
+int pxrhip_field_bc_periodic(double *f, int64_t nx, int64_t ny, int64_t nz, int64_t nxg,
+                             int64_t nyg, int64_t nzg) {
+  return field_bc(&f, 1, nx, ny, nz, nxg, nyg, nzg);
+}
+
+int pxrhip_field_bc_periodic_vec(double *fx, double *fy, double *fz, int64_t nx, int64_t ny,
+                                 int64_t nz, int64_t nxg, int64_t nyg, int64_t nzg) {
+  double *p[3] = {fx, fy, fz};
+  return field_bc(p, 3, nx, ny, nz, nxg, nyg, nzg);
+}
+
 int pxrhip_current_bc_periodic(double *a, int64_t nx, int64_t ny, int64_t nz, int64_t nxg,
                                int64_t nyg, int64_t nzg) {
-  PXR_INIT();
-  int r = check_grid(nx, ny, nz, nxg, nyg, nzg);
-  if (r) return r;
-  if (!a) return set_error(PXRHIP_ERR_ARG, "null array");
-  if (nx <= 2 * nxg || ny <= 2 * nyg || nz <= 2 * nzg)
-    return set_error(PXRHIP_ERR_UNSUPPORTED, "periodic guards need n > 2*guards on every axis");
-  GridGeom g = mkgeom(nx, ny, nz, nxg, nyg, nzg);
-  const int64_t ext[3] = {nx + 1 + 2 * nxg, ny + 1 + 2 * nyg, nz + 1 + 2 * nzg};
-  const int64_t gg[3] = {nxg, nyg, nzg};
-  for (int ax = 0; ax < 3; ax++) {
-    int64_t tot = 1;
-    for (int d = 0; d < 3; d++) tot *= (d == ax) ? 2 * gg[d] + 1 : ext[d];
-    hipLaunchKernelGGL(k_current_bc_axis, dim3(grid1d(tot, 256)), dim3(256), 0, rt().stream, a, g, ax);
-    PXR_LAUNCHED();
-  }
-  return PXRHIP_OK;
+  return current_bc(&a, 1, nx, ny, nz, nxg, nyg, nzg);
+}
+
+int pxrhip_current_bc_periodic_vec(double *jx, double *jy, double *jz, int64_t nx, int64_t ny,
+                                   int64_t nz, int64_t nxg, int64_t nyg, int64_t nzg) {
+  double *p[3] = {jx, jy, jz};
+  return current_bc(p, 3, nx, ny, nz, nxg, nyg, nzg);
 }
 
 }  // extern "C"

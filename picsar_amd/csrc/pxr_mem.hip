@@ -18,6 +18,19 @@ __global__ __launch_bounds__(256) void k_fill_f64(double *p, i64 n, double v) {
   if (i < n) p[i] = v;
 }
 
+// two values per lane in one 16 B store where the array starts on 16 B
+__global__ __launch_bounds__(256) void k_fill3_f64(double *p0, double *p1, double *p2, i64 n,
+                                                   double v) {
+  double *p = blockIdx.y == 0 ? p0 : blockIdx.y == 1 ? p1 : p2;
+  const i64 i = 2 * ((i64)blockIdx.x * blockDim.x + threadIdx.x);
+  if (i + 1 < n && !((uintptr_t)p & 15)) {
+    *(double2 *)(p + i) = make_double2(v, v);
+  } else {
+    if (i < n) p[i] = v;
+    if (i + 1 < n) p[i + 1] = v;
+  }
+}
+
 __global__ __launch_bounds__(256) void k_fill_i64(int64_t *p, i64 n, int64_t v) {
   const i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -227,6 +240,16 @@ int pxrhip_fill_f64(double *p, int64_t n, double value) {
   if (n < 0 || (n && !p)) return set_error(PXRHIP_ERR_ARG, "bad fill");
   if (!n) return PXRHIP_OK;
   hipLaunchKernelGGL(k_fill_f64, dim3(grid1d(n, 256)), dim3(256), 0, rt().stream, p, n, value);
+  PXR_LAUNCHED();
+  return PXRHIP_OK;
+}
+
+int pxrhip_fill_f64_vec(double *p0, double *p1, double *p2, int64_t n, double value) {
+  PXR_INIT();
+  if (n < 0 || (n && (!p0 || !p1 || !p2))) return set_error(PXRHIP_ERR_ARG, "bad fill");
+  if (!n) return PXRHIP_OK;
+  hipLaunchKernelGGL(k_fill3_f64, dim3(grid1d((n + 1) / 2, 256), 3), dim3(256), 0, rt().stream, p0,
+                     p1, p2, n, value);
   PXR_LAUNCHED();
   return PXRHIP_OK;
 }

@@ -354,8 +354,7 @@ class Simulation:
         """field_gathering_plus_particle_pusher + pxrdepose_currents_on_grid_jxjyjz
         for every species (J is zeroed first, current_deposition_manager_3d.F90:247)
         in one kernel per species, then the antennas."""
-        for k in ("jx", "jy", "jz"):
-            self.fields[k].fill(0.0)
+        self._zero_current()
         for sp in self.species:
             self.gather_push_deposit_species(sp)
         self.laser_push_deposit()
@@ -408,8 +407,7 @@ class Simulation:
         """pxrdepose_currents_on_grid_jxjyjz (current_deposition_manager_3d.F90:
         224-505): J = 0, then the current of every species that deposits and
         of the antennas."""
-        for k in ("jx", "jy", "jz"):
-            self.fields[k].fill(0.0)
+        self._zero_current()
         for sp in self.species:
             if sp.ldodepos and sp.npart:
                 self.depose_currents_species(sp)
@@ -423,20 +421,33 @@ class Simulation:
             if sp.npart and not sp.lfreeze:
                 self._rebin(sp)
 
+    def _grids(self, *names):
+        """Device pointers of grid arrays, each checked to have this grid's shape."""
+        shp = (self.nx + 1 + 2 * self.ng, self.ny + 1 + 2 * self.ng, self.nz + 1 + 2 * self.ng)
+        out = []
+        for k in names:
+            f = self.fields[k]
+            if tuple(f.shape) != shp:
+                raise ValueError(f"{k}: grid shape {f.shape} != {shp}")
+            out.append(f.ptr)
+        return out
+
+    def _zero_current(self):
+        n = (self.nx + 1 + 2 * self.ng) * (self.ny + 1 + 2 * self.ng) * (self.nz + 1 + 2 * self.ng)
+        _lib.call("pxrhip_fill_f64_vec", *self._grids("jx", "jy", "jz"), n, 0.0)
+
+    def _guards(self, entry, *names):
+        g = self.ng
+        _lib.call(entry, *self._grids(*names), self.nx, self.ny, self.nz, g, g, g)
+
     def current_bcs(self):
-        n, g = (self.nx, self.ny, self.nz), self.ng
-        for k in ("jx", "jy", "jz"):
-            _pxr.summation_bcs(self.fields[k], g, g, g, *n)
+        self._guards("pxrhip_current_bc_periodic_vec", "jx", "jy", "jz")
 
     def efield_bcs(self):
-        n, g = (self.nx, self.ny, self.nz), self.ng
-        for k in ("ex", "ey", "ez"):
-            _pxr.field_bc(self.fields[k], g, g, g, *n)
+        self._guards("pxrhip_field_bc_periodic_vec", "ex", "ey", "ez")
 
     def bfield_bcs(self):
-        n, g = (self.nx, self.ny, self.nz), self.ng
-        for k in ("bx", "by", "bz"):
-            _pxr.field_bc(self.fields[k], g, g, g, *n)
+        self._guards("pxrhip_field_bc_periodic_vec", "bx", "by", "bz")
 
     def push_bfield(self):
         """push_bfield (maxwell_solver_manager.F90:44): half step, 0.5*dt/dx."""
