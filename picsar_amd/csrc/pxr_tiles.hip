@@ -635,59 +635,121 @@ __global__ __launch_bounds__(256) void k_rb_slots(const int *key, const int64_t 
   }
 }
 
-// Source indices in bin b's slots put in increasing order.  Up to 16 are
-// loaded at once and sorted in registers by a fixed exchange network (no
-// chain of dependent loads); longer bins take an insertion sort in memory.
-PXR_DEV void order_bin(const i64 *bin_start, int b, int *perm) {
-  const i64 s = bin_start[b], e = bin_start[b + 1];
-  const i64 n = e - s;
-  if (n < 2) return;
-  if (n <= 16) {
-    int v[16];
+// v[0..M) in increasing order: Batcher's odd-even merge network (63
+// exchanges for 16, 191 for 32), fully unrolled
+template <int M> PXR_DEV void sort_network(int *v) {
 #pragma unroll
-    for (int j = 0; j < 16; j++) v[j] = j < n ? perm[s + j] : INT_MAX;
+  for (int p = 1; p < M; p *= 2)
 #pragma unroll
-    for (int i = 1; i < 16; i++)
+    for (int k = p; k >= 1; k /= 2)
 #pragma unroll
-      for (int j = i; j > 0; j--) {
-        const int lo = min(v[j - 1], v[j]), hi = max(v[j - 1], v[j]);
-        v[j - 1] = lo;
-        v[j] = hi;
-      }
+      for (int j = k % p; j + k < M; j += 2 * k)
 #pragma unroll
-    for (int j = 0; j < 16; j++)
-      if (j < n) perm[s + j] = v[j];
-    return;
-  }
-  int prev = perm[s];
-  for (i64 j = s + 1; j < e; j++) {
-    const int v = perm[j];
-    if (v >= prev) {
-      prev = v;
-      continue;
-    }
-    i64 k = j - 1;
-    while (k >= s && perm[k] > v) {
-      perm[k + 1] = perm[k];
-      k--;
-    }
-    perm[k + 1] = v;
-  }
+        for (int i = 0; i < k; i++)
+          if (i + j + k < M && (i + j) / (2 * p) == (i + j + k) / (2 * p)) {
+            const int lo = min(v[i + j], v[i + j + k]), hi = max(v[i + j], v[i + j + k]);
+            v[i + j] = lo;
+            v[i + j + k] = hi;
+          }
 }
 
-// 2. k_rb_order: one thread per flagged bin sorts the source indices of its
-//    slots (insertion sort: the slots hold a few increasing runs), so that
-//    a bin lists its particles in source order, as the reference's stable
-//    counting sort does (sorting.F90:333-343), whatever order the runs
-//    arrived in.  Bins filled by one run are in order already.  (Listing a
-//    wave's flagged bins among 512 and sorting them one per lane took the
-//    256^3 plasma's pass from 0.36 to 0.32 ms, but the bunch's from 0.7 to
-//    3.2 ms: its dense flagged bins then fell to a few waves.)
-__global__ __launch_bounds__(256) void k_rb_order(const i64 *bin_start, i64 nbins,
-                                                  const int *flag, int *perm) {
+template <int M> PXR_DEV void order_slots(int *perm, int n) {
+  int v[M];
+#pragma unroll
+  for (int j = 0; j < M; j++) v[j] = j < n ? perm[j] : INT_MAX;
+  sort_network<M>(v);
+#pragma unroll
+  for (int j = 0; j < M; j++)
+    if (j < n) perm[j] = v[j];
+}
+
+// 2. k_rb_order: the source indices of every flagged bin's slots in
+//    increasing order, so that a bin lists its particles in source order, as
+//    the reference's stable counting sort does (sorting.F90:333-343),
+//    whatever order its runs arrived in.  Bins filled by one run are in
+//    order already.  A thread sorts a bin of up to 32 in registers; larger
+//    ones are listed for k_rb_order_big, one wave each, since a dense region
+//    (the bunch) would otherwise fall to a few waves.  The first threads also
+//    write the tile offsets.
+//    A chain of dependent loads bounded the former insertion sort of bins
+//    over 16: 0.286 ms per species at 128^3, 16 ppc, 0.214 ms for the bunch
+//    of 64 ppc in 128^3; now 0.085 + 0.002 and 0.014 + 0.006 ms.
+constexpr int RB_SMALL = 32;
+
+struct OrderArgs {
+  const i64 *bin_start;
+  i64 nbins;
+  const int *flag;
+  int *perm;
+  int *big, *nbig;  // bins of more than RB_SMALL
+  int ntiles;
+  const int64_t *bin_base;
+  int64_t *off, *np;
+};
+
+__global__ __launch_bounds__(256) void k_rb_order(OrderArgs a) {
   const i64 b = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nbins || !flag[b]) return;
-  order_bin(bin_start, (int)b, perm);
+  if (b <= a.ntiles) {
+    const int64_t o = a.bin_start[a.bin_base[b]];
+    a.off[b] = o;
+    if (b < a.ntiles) a.np[b] = a.bin_start[a.bin_base[b + 1]] - o;
+  }
+  if (b >= a.nbins || !a.flag[b]) return;
+  const i64 s = a.bin_start[b], n = a.bin_start[b + 1] - s;
+  if (n > RB_SMALL) a.big[atomicAdd(a.nbig, 1)] = (int)b;
+  else if (n > 16) order_slots<32>(a.perm + s, (int)n);
+  else order_slots<16>(a.perm + s, (int)n);
+}
+
+// The listed bins, a wave each.  Up to RB_RANK indices sit in LDS and every
+// lane counts the smaller ones of its own; beyond that one lane inserts them
+// in memory.
+constexpr int RB_RANK = 1024;
+
+__global__ __launch_bounds__(256) void k_rb_order_big(const i64 *bin_start, const int *big,
+                                                      const int *nbig, int *perm) {
+  __shared__ int4 sv[4][RB_RANK / 4];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int nb = *nbig;
+  for (int q = blockIdx.x * 4 + w; q < nb; q += gridDim.x * 4) {
+    const i64 s = bin_start[big[q]];
+    const int n = (int)(bin_start[big[q] + 1] - s);
+    int *p = perm + s;
+    if (n > RB_RANK) {
+      if (lane == 0) {
+        int prev = p[0];
+        for (int j = 1; j < n; j++) {
+          const int v = p[j];
+          if (v >= prev) {
+            prev = v;
+            continue;
+          }
+          int k = j - 1;
+          while (k >= 0 && p[k] > v) {
+            p[k + 1] = p[k];
+            k--;
+          }
+          p[k + 1] = v;
+        }
+      }
+      continue;
+    }
+    int *v = (int *)sv[w];
+    const int n4 = (n + 3) >> 2;
+    for (int j = lane; j < 4 * n4; j += 64) v[j] = j < n ? p[j] : INT_MAX;
+    // only this wave uses its part of sv: its own LDS order suffices
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int j = lane; j < n; j += 64) {
+      const int mine = v[j];
+      int r = 0;
+      for (int k = 0; k < n4; k++) {
+        const int4 o = sv[w][k];
+        r += (o.x < mine) + (o.y < mine) + (o.z < mine) + (o.w < mine);
+      }
+      p[r] = mine;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
 }
 
 struct GatherArgs {
@@ -787,43 +849,74 @@ PXR_DEV bool blocks_fit(const ChunkArgs &a, int t, int z0, int z1, int y0, int y
          a.jnode_bytes * jpz * j2 <= a.j_bytes;
 }
 
+// The chunker gives CG lanes to a tile (grouping its planes) or a plane
+// (cutting its rows): the lanes load the counts of CG planes or rows and test
+// CG candidate ends against the LDS budgets at once, and the first that fails
+// closes the group or chunk.  One thread walking them one by one waited for
+// two dependent loads and a block geometry per row: 57 + 59 us for the 34
+// planes of one 33^3-node tile, now 23 + 27 us (37 + 35, now 12 + 14, for
+// 61 x 45 x 70 cells in 60 tiles; grouping the planes of the 4096 tiles of a
+// 128^3 bunch 40, now 21 us).
+constexpr int CG = 16;
+
+// the bits of this lane's group in a ballot
+PXR_DEV unsigned cg_ballot(bool p) {
+  return (unsigned)(__ballot(p) >> (__lane_id() & ~(CG - 1))) & ((1u << CG) - 1u);
+}
+
+PXR_DEV i64 cg_scan(i64 v, int lane) {  // inclusive sum over the group's lanes
+#pragma unroll
+  for (int off = 1; off < CG; off <<= 1) {
+    const i64 y = __shfl_up(v, off, CG);
+    if (lane >= off) v += y;
+  }
+  return v;
+}
+
 // Groups of consecutive whole planes of tile t that together hold at most
 // `ch` particles and whose blocks fit: sparse planes then share one work
 // item instead of paying a work item's fixed cost each.  A plane too large
 // to be taken whole is cut into runs of rows by walk_unit.
 __global__ __launch_bounds__(256) void k_chunk_groups(ChunkArgs a) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = (blockIdx.x * blockDim.x + threadIdx.x) / CG, lane = threadIdx.x % CG;
   if (t >= a.ntiles) return;
   int *grp = a.group + (i64)t * a.nzmax;
   const int nx3 = a.n3[3 * t], ny3 = a.n3[3 * t + 1], nz3 = a.n3[3 * t + 2];
   if (!a.bin_start) {
-    for (int z = 0; z < a.nzmax; z++) grp[z] = GROUP_ROWS;
+    for (int z = lane; z < a.nzmax; z += CG) grp[z] = GROUP_ROWS;
     return;
   }
-  for (int z = nz3; z < a.nzmax; z++) grp[z] = GROUP_EMPTY;
+  for (int z = nz3 + lane; z < a.nzmax; z += CG) grp[z] = GROUP_EMPTY;
   const i64 plane = (i64)ny3 * nx3, base = a.bin_base[t];
-  auto count = [&](int z) { return a.bin_start[base + (z + 1) * plane] - a.bin_start[base + z * plane]; };
+  auto count = [&](int z) {
+    return z < nz3 ? a.bin_start[base + (z + 1) * plane] - a.bin_start[base + z * plane] : 0;
+  };
   int z = 0;
   while (z < nz3) {
-    const i64 n = count(z);
-    if (n <= 0) {
-      grp[z++] = GROUP_EMPTY;
-      continue;
+    // planes z .. z + CG - 1: empty ones, ones to be cut, ones that may group
+    const i64 n = count(z + lane);
+    const bool in = z + lane < nz3, empty = n <= 0;
+    const bool cut = !empty && (n > a.ch || !blocks_fit(a, t, z + lane, z + lane, 0, ny3 - 1));
+    const unsigned whole = cg_ballot(in && !empty && !cut);
+    const int skip = whole ? __ffs(whole) - 1 : CG;  // planes before the first groupable one
+    if (in && lane < skip) grp[z + lane] = empty ? GROUP_EMPTY : GROUP_ROWS;
+    z += skip;
+    if (!whole) continue;
+    i64 sum = 0;
+    int z1 = z;  // last plane of the group headed by z
+    for (int w = z;; w += CG) {
+      const i64 m = count(w + lane);
+      const i64 tot = sum + cg_scan(m, lane);
+      const bool ok = m > 0 && tot <= a.ch && blocks_fit(a, t, z, w + lane, 0, ny3 - 1);
+      const unsigned bad = cg_ballot(!ok);
+      if (bad) {
+        z1 = w + __ffs(bad) - 2;
+        break;
+      }
+      sum = __shfl(tot, CG - 1, CG);
     }
-    if (n > a.ch || !blocks_fit(a, t, z, z, 0, ny3 - 1)) {
-      grp[z++] = GROUP_ROWS;
-      continue;
-    }
-    int z1 = z;
-    i64 cnt = n;
-    while (z1 + 1 < nz3) {
-      const i64 m = count(z1 + 1);
-      if (m <= 0 || cnt + m > a.ch || !blocks_fit(a, t, z, z1 + 1, 0, ny3 - 1)) break;
-      cnt += m;
-      z1++;
-    }
-    grp[z] = z1;
-    for (int zz = z + 1; zz <= z1; zz++) grp[zz] = GROUP_MEMBER;
+    if (lane == 0) grp[z] = z1;
+    for (int zz = z + 1 + lane; zz <= z1; zz += CG) grp[zz] = GROUP_MEMBER;
     z = z1 + 1;
   }
 }
@@ -834,33 +927,37 @@ __global__ __launch_bounds__(256) void k_chunk_groups(ChunkArgs a) {
 // field and current blocks fit the LDS budget; rows denser than that are
 // cut.  Such a chunk spans a compact block of cells: the tile's width in x,
 // a few rows in y, one plane in z.  Without sorting information the tile is
-// one unit cut into runs of ch particles.
+// one unit cut into runs of ch particles.  Called by the CG lanes of the
+// unit; returns its number of chunks.
 template <bool WRITE>
-PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, i64 pos) {
+PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, i64 pos, int lane) {
   int nch = 0;
   auto emit = [&](int64_t b, int64_t n, int zz, int zz1, int y0, int y1) {
-    if (WRITE && pos + nch >= a.maxchunks) count_bad(a.bad);  // cannot happen: see the bound
-    if (WRITE && pos + nch < a.maxchunks) {
-      Chunk c;
-      c.begin = b;
-      c.n = (int)n;
-      c.tile = t;
-      c.z = zz;
-      c.z1 = zz1;
-      c.y0 = y0;
-      c.y1 = y1;
-      c.s = 0;
-      c.pad = 0;
-      if (a.sk4 > 0 && zz >= 0) {
-        // lanes a few sorting cells apart: sk4 / 4 times the particles per
-        // cell, to the nearest power of two (on a log scale)
-        const i64 cells = (i64)a.n3[3 * t] * (y1 - y0 + 1) * (zz1 - zz + 1);
-        const double want = (double)a.sk4 * (double)n / (4.0 * (double)cells);
-        int p2 = 1;
-        while (p2 < (1 << 20) && want > 1.4142135623730951 * p2) p2 <<= 1;
-        c.s = p2;
+    if (WRITE && lane == 0) {
+      if (pos + nch >= a.maxchunks) {
+        count_bad(a.bad);  // cannot happen: see the bound
+      } else {
+        Chunk c;
+        c.begin = b;
+        c.n = (int)n;
+        c.tile = t;
+        c.z = zz;
+        c.z1 = zz1;
+        c.y0 = y0;
+        c.y1 = y1;
+        c.s = 0;
+        c.pad = 0;
+        if (a.sk4 > 0 && zz >= 0) {
+          // lanes a few sorting cells apart: sk4 / 4 times the particles per
+          // cell, to the nearest power of two (on a log scale)
+          const i64 cells = (i64)a.n3[3 * t] * (y1 - y0 + 1) * (zz1 - zz + 1);
+          const double want = (double)a.sk4 * (double)n / (4.0 * (double)cells);
+          int p2 = 1;
+          while (p2 < (1 << 20) && want > 1.4142135623730951 * p2) p2 <<= 1;
+          c.s = p2;
+        }
+        a.out[pos + nch] = c;
       }
-      a.out[pos + nch] = c;
     }
     nch++;
   };
@@ -881,28 +978,45 @@ PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, i64 pos) {
     return nch;
   }
   if (g != GROUP_ROWS) return 0;
+  auto rows = [&](int y) {  // particles of row y
+    const int64_t r = base + (int64_t)y * nx3;
+    return y < ny3 ? a.bin_start[r + nx3] - a.bin_start[r] : 0;
+  };
+  int y = 0;  // next row to look at
   int64_t cb = 0, cnt = 0;
   int y0 = 0, ylast = 0;  // first and last row of the open chunk
-  for (int y = 0; y < ny3; y++) {
-    const int64_t row = base + (int64_t)y * nx3;
-    const int64_t rb = a.bin_start[row], rn = a.bin_start[row + nx3] - rb;
-    if (rn <= 0) continue;
-    const bool fits = cnt == 0 || blocks_fit(a, t, z, z, y0, y);
-    if (cnt > 0 && (cnt + rn > a.ch || !fits)) {
+  while (y < ny3) {
+    const int64_t rn = rows(y + lane);
+    if (cnt == 0) {  // open a chunk at the first row with particles
+      const unsigned some = cg_ballot(rn > 0);
+      if (!some) {
+        y += CG;
+        continue;
+      }
+      const int f = __ffs(some) - 1;
+      y0 = ylast = y + f;
+      cnt = __shfl(rn, f, CG);
+      cb = a.bin_start[base + (int64_t)y0 * nx3];
+      while (cnt > a.ch) {  // a row denser than a chunk: cut it
+        emit(cb, a.ch, z, z, y0, y0);
+        cb += a.ch;
+        cnt -= a.ch;
+      }
+      y = y0 + 1;
+      continue;
+    }
+    // the rows from y on that still belong to the open chunk
+    const int64_t sum = cnt + cg_scan(rn, lane);
+    const bool end = rn > 0 && (sum > a.ch || !blocks_fit(a, t, z, z, y0, y + lane));
+    const unsigned ends = cg_ballot(end);
+    const int take = ends ? __ffs(ends) - 1 : CG;
+    const unsigned used = cg_ballot(rn > 0) & ((1u << take) - 1u);
+    if (used) ylast = y + 31 - __clz(used);
+    if (take) cnt = __shfl(sum, take - 1, CG);
+    y += take;
+    if (ends) {
       emit(cb, cnt, z, z, y0, ylast);
       cnt = 0;
-    }
-    if (cnt == 0) {
-      cb = rb;
-      y0 = y;
-    }
-    cnt += rn;
-    ylast = y;
-    while (cnt > a.ch) {  // a row denser than a chunk: cut it
-      emit(cb, a.ch, z, z, y0, y);
-      cb += a.ch;
-      cnt -= a.ch;
-      y0 = y;
     }
   }
   if (cnt > 0) emit(cb, cnt, z, z, y0, ylast);
@@ -910,8 +1024,11 @@ PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, i64 pos) {
 }
 
 __global__ __launch_bounds__(256) void k_chunk_count(ChunkArgs a) {
-  const i64 u = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u < (i64)a.ntiles * a.nzmax) a.count[u] = walk_unit<false>(a, (int)(u / a.nzmax), (int)(u % a.nzmax), 0);
+  const i64 u = ((i64)blockIdx.x * blockDim.x + threadIdx.x) / CG;
+  const int lane = threadIdx.x % CG;
+  if (u >= (i64)a.ntiles * a.nzmax) return;
+  const int n = walk_unit<false>(a, (int)(u / a.nzmax), (int)(u % a.nzmax), 0, lane);
+  if (lane == 0) a.count[u] = n;
 }
 
 // Largest-first queue order of the work items: a counting sort of the
@@ -945,12 +1062,34 @@ __global__ __launch_bounds__(256) void k_order_scatter(const Chunk *chunks, cons
   order[atomicAdd(bucket + (n > 0 ? 31 - __clz(n) : 0), 1)] = c;
 }
 
+// The chunks of every unit.  a.start null: few units, and each block sums
+// the counts before its own itself, which saves the three launches of the
+// scan.
+constexpr i64 CHUNK_SELF_SCAN = 16384;
+
 __global__ __launch_bounds__(256) void k_chunk_write(ChunkArgs a) {
+  constexpr int PER = 256 / CG;  // units per block
+  __shared__ int before[4];
   const i64 nu = (i64)a.ntiles * a.nzmax;
-  const i64 u = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u < nu) walk_unit<true>(a, (int)(u / a.nzmax), (int)(u % a.nzmax), a.start[u]);
-  if (u == 0) {
-    const i64 tot = a.start[nu];
+  const int lane = threadIdx.x % CG, k = threadIdx.x / CG;
+  const i64 u0 = (i64)blockIdx.x * PER, u = u0 + k;
+  i64 pos = 0, tot = 0;
+  if (a.start) {
+    if (u < nu) pos = a.start[u];
+    tot = a.start[nu];
+  } else {
+    int acc = 0;
+    for (i64 i = threadIdx.x; i < u0; i += 256) acc += a.count[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
+    if ((threadIdx.x & 63) == 0) before[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    pos = before[0] + before[1] + before[2] + before[3];
+    for (i64 i = u0; i < min(u, nu); i++) pos += a.count[i];
+    tot = pos + (u < nu ? a.count[u] : 0);
+  }
+  if (u < nu) walk_unit<true>(a, (int)(u / a.nzmax), (int)(u % a.nzmax), pos, lane);
+  if (u == nu - 1 && lane == 0) {
     *a.nchunks = (int)min(tot, a.maxchunks);
     *a.queue = 0;
     a.queue[1] = 0;  // overflow count (ctl[2])
@@ -1561,9 +1700,9 @@ int pxrhip_tiles_rebin_sort(const pxrhip_grid *grid, pxrhip_species *src, pxrhip
     hipLaunchKernelGGL(k_rb_gather, dim3(grid1d(cap, 256)), dim3(256), 0, st, ga, cap);
   } else {
     hipLaunchKernelGGL(k_rb_scatter, dim3(grid1d(cap, 256)), dim3(256), 0, st, sa, cap);
+    hipLaunchKernelGGL(k_rb_tiles, dim3(grid1d(tt->ntiles + 1, 256)), dim3(256), 0, st,
+                       tt->ntiles, tt->bin_base, dst->bin_start, dst->tile_off, dst->tile_np);
   }
-  hipLaunchKernelGGL(k_rb_tiles, dim3(grid1d(tt->ntiles + 1, 256)), dim3(256), 0, st, tt->ntiles,
-                     tt->bin_base, dst->bin_start, dst->tile_off, dst->tile_np);
   PXR_LAUNCHED();
   return PXRHIP_OK;
 }
