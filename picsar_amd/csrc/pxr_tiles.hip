@@ -1841,6 +1841,14 @@ static int tiles_fused(const pxrhip_grid *grid, const pxrhip_species *sp, const 
   a.ovf_count = ctl + 2;
   a.ovf = ovf;
   a.ovf_cap = maxchunks < INT_MAX ? (int)maxchunks : INT_MAX;
+  a.nodekey = a.slots = nullptr;
+  a.slot_stride = 0;
+  if (use_banks((int)order, depo_algo ? 3 : 0, jacc) && (phase & PHASE_DEPOSIT)) {
+    a.slot_stride = (ch + 63) & ~63;
+    a.nodekey = (unsigned short *)scratch(19, sizeof(short) * (size_t)(sp->capacity > 1 ? sp->capacity : 1));
+    a.slots = (unsigned short *)scratch(22, sizeof(short) * (size_t)a.slot_stride * rt().num_cus * wg_per_cu);
+    if (!a.nodekey || !a.slots) return set_error(PXRHIP_ERR_HIP, "scratch allocation failed");
+  }
   a.order = nullptr;
   if (g_tune.order) {
     int *bucket = (int *)scratch(20, sizeof(int) * 32);
