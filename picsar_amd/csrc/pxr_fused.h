@@ -238,11 +238,14 @@ PXR_DEV double fx_weight(const FusedArgs &a, double qw, double vx, double vy, do
 // Launch times at 96^3, 8 particles per cell (ms per species, before and with
 // it): FP64 1.07 -> 0.98, mixed precision 0.85 -> 0.81 (0.80 -> 0.75 for the
 // colder ions), the gamma = 10 bunch 0.37 -> 0.34; at 16 particles per cell
-// 1.88 -> 1.68, at 64 (mixed) 0.92 -> 0.82.  At order 2 it lost 2%, at order 1
-// 15%, and the order-3 direct current was unchanged.
+// 1.88 -> 1.68, at 64 (mixed) 0.92 -> 0.82, at 1 0.315 -> 0.325 (FP64) and
+// 0.209 -> 0.207 (mixed).  At order 2 it lost 2%, at order 1 15%, and the
+// order-3 direct current was unchanged.
 constexpr bool use_banks(int order, int depo, int jacc) {
   return order == 3 && depo == 0 && jacc == 3;
 }
+
+constexpr int BANK_CHUNK = 16384;  // most particles of a work item dealt so
 
 PXR_DEV unsigned short node_key(const int *b0) {  // the first node modulo 16 on each axis
   return (unsigned short)((b0[0] & 15) | (b0[1] & 15) << 4 | (b0[2] & 15) << 8);

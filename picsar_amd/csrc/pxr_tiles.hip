@@ -1728,7 +1728,7 @@ static int tiles_fused(const pxrhip_grid *grid, const pxrhip_species *sp, const 
     return set_error(PXRHIP_ERR_ARG, "null field array");
   if ((phase & PHASE_DEPOSIT) && (!jx || !jy || !jz)) return set_error(PXRHIP_ERR_ARG, "null current array");
   if (!(dt > 0)) return set_error(PXRHIP_ERR_ARG, "dt must be > 0");
-  const int ch = chunk > 0 ? (int)(chunk < (1 << 20) ? chunk : (1 << 20)) : g_tune.chunk;
+  int ch = chunk > 0 ? (int)(chunk < (1 << 20) ? chunk : (1 << 20)) : g_tune.chunk;
   hipStream_t st = rt().stream;
   // block geometry of the work items
   BoxGeom bg;
@@ -1756,6 +1756,11 @@ static int tiles_fused(const pxrhip_grid *grid, const pxrhip_species *sp, const 
     bg.n3 = tt->n3;
   }
   const bool mx = sp->precision == 1;
+  // lanes dealt by bank: the slots hold 16-bit places in a work item, and a
+  // row of them is kept for every workgroup
+  const bool banks = use_banks((int)order, depo_algo ? 3 : 0,
+                               mx ? g_tune.jacc : g_tune.fp64_jacc) && (phase & PHASE_DEPOSIT);
+  if (banks && ch > BANK_CHUNK) ch = BANK_CHUNK;
   const int esize = mx ? 4 : 8;
   // LDS current: mixed.jacc (0 FP32, 1 compensated FP32, 2 FP64, 3 fixed
   // point) for a mixed-precision species, fused.jacc (0 FP64, 3 fixed point)
@@ -1843,7 +1848,7 @@ static int tiles_fused(const pxrhip_grid *grid, const pxrhip_species *sp, const 
   a.ovf_cap = maxchunks < INT_MAX ? (int)maxchunks : INT_MAX;
   a.nodekey = a.slots = nullptr;
   a.slot_stride = 0;
-  if (use_banks((int)order, depo_algo ? 3 : 0, jacc) && (phase & PHASE_DEPOSIT)) {
+  if (banks) {
     a.slot_stride = (ch + 63) & ~63;
     a.nodekey = (unsigned short *)scratch(19, sizeof(short) * (size_t)(sp->capacity > 1 ? sp->capacity : 1));
     a.slots = (unsigned short *)scratch(22, sizeof(short) * (size_t)a.slot_stride * rt().num_cus * wg_per_cu);

@@ -58,3 +58,13 @@ def test_uneven_classes(torch, orc, n, box):
     ref.step()
     for k in ("ex", "ey", "ez", "jx", "jy", "jz"):
         assert rel(tng(sim.fields[k]), ref.f[k]) <= 1e-12, k
+
+
+def test_large_chunk(torch, orc):
+    """A work-item size beyond the 16-bit slots is taken as a smaller one."""
+    sim, ref, tng = build(torch, orc, 3, True, "vay", "esirkepov", chunk=1 << 20, ntiles=(1, 1, 1))
+    add_both(sim, ref, np.random.default_rng(8), 70000, (4.0, 4.0, 4.0), (4.4, 4.4, 4.4))
+    sim.step(1)
+    ref.step()
+    for k in ("ex", "ey", "ez", "jx", "jy", "jz"):
+        assert rel(tng(sim.fields[k]), ref.f[k]) <= 1e-12, k
