@@ -23,20 +23,10 @@ namespace pxr {
 // ---------------------------------------------------------------------------
 // field gathering
 // ---------------------------------------------------------------------------
-struct GatherArgs {
-  i64 np;
-  const double *xp, *yp, *zp;
-  double *ex, *ey, *ez, *bx, *by, *bz;
-  double xmin, ymin, zmin, dxi, dyi, dzi, s;
-  GridGeom g;
-  const double *exg, *eyg, *ezg, *bxg, *byg, *bzg;
-  unsigned long long *bad;
-};
-
 template <int N, int M>
-__global__ __launch_bounds__(256) void k_gather(GatherArgs a) {
+__global__ __launch_bounds__(256) void k_gather(LeafGatherArgs a) {
   const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (ip >= a.np) return;
+  if (ip >= a.np || (a.skip && *a.skip)) return;
   const double x = (a.xp[ip] - a.xmin) * a.dxi;
   const double y = (a.yp[ip] - a.ymin) * a.dyi;
   const double z = (a.zp[ip] - a.zmin) * a.dzi;
@@ -54,6 +44,18 @@ __global__ __launch_bounds__(256) void k_gather(GatherArgs a) {
   a.bx[ip] += out[3];
   a.by[ip] += out[4];
   a.bz[ip] += out[5];
+}
+
+static void launch_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st) {
+  const dim3 grd(grid1d(a.np, 256)), blk(256);
+  switch (order * 2 + (lower ? 1 : 0)) {
+    case 2: hipLaunchKernelGGL((k_gather<1, 1>), grd, blk, 0, st, a); break;
+    case 3: hipLaunchKernelGGL((k_gather<1, 0>), grd, blk, 0, st, a); break;
+    case 4: hipLaunchKernelGGL((k_gather<2, 2>), grd, blk, 0, st, a); break;
+    case 5: hipLaunchKernelGGL((k_gather<2, 1>), grd, blk, 0, st, a); break;
+    case 6: hipLaunchKernelGGL((k_gather<3, 3>), grd, blk, 0, st, a); break;
+    default: hipLaunchKernelGGL((k_gather<3, 2>), grd, blk, 0, st, a); break;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -878,7 +880,7 @@ int pxrhip_geteb3d_energy_conserving(
     PXR_LAUNCHED();
     return finish_checked("geteb3d_energy_conserving");
   }
-  GatherArgs a;
+  LeafGatherArgs a;
   a.np = np;
   a.xp = xp; a.yp = yp; a.zp = zp;
   a.ex = ex; a.ey = ey; a.ez = ez; a.bx = bx; a.by = by; a.bz = bz;
@@ -887,17 +889,20 @@ int pxrhip_geteb3d_energy_conserving(
   a.s = l_nodal ? 0.0 : 0.5;
   a.g = mkgeom(nx, ny, nz, nxguard, nyguard, nzguard);
   a.exg = exg; a.eyg = eyg; a.ezg = ezg; a.bxg = bxg; a.byg = byg; a.bzg = bzg;
+  a.skip = nullptr;
   a.bad = rt().d_bad;
   const bool lo = l_lower_order_in_v != 0;
-  dim3 grd(grid1d(np, 256)), blk(256);
   hipStream_t st = rt().stream;
-  switch (nox * 2 + (lo ? 1 : 0)) {
-    case 2: hipLaunchKernelGGL((k_gather<1, 1>), grd, blk, 0, st, a); break;
-    case 3: hipLaunchKernelGGL((k_gather<1, 0>), grd, blk, 0, st, a); break;
-    case 4: hipLaunchKernelGGL((k_gather<2, 2>), grd, blk, 0, st, a); break;
-    case 5: hipLaunchKernelGGL((k_gather<2, 1>), grd, blk, 0, st, a); break;
-    case 6: hipLaunchKernelGGL((k_gather<3, 3>), grd, blk, 0, st, a); break;
-    default: hipLaunchKernelGGL((k_gather<3, 2>), grd, blk, 0, st, a); break;
+  const bool probe = leaf_binned_gather_may_pay(a, (int)nox);
+  if (probe && (r = leaf_probe_start(a, st))) return r;
+  launch_gather(a, (int)nox, lo, st);
+  if (probe) {
+    bool scattered;
+    if ((r = leaf_probe_read(scattered))) return r;
+    a.skip = nullptr;
+    i64 done = np;
+    if (scattered && (r = leaf_binned_gather(a, (int)nox, lo, st, done))) return r;
+    if (done < np) launch_gather(a.part(done, np - done), (int)nox, lo, st);
   }
   PXR_LAUNCHED();
   return finish_checked("geteb3d_energy_conserving");
@@ -1076,9 +1081,13 @@ int pxrhip_depose_jxjyjz(double *jx, double *jy, double *jz, int64_t np, const d
   dim3 grd(grid1d(np, 256 * DEP_S)), blk(256);
   hipStream_t st = rt().stream;
   const bool direct = current_depo_algo >= 2;  // depose_jxjyjz_generic CASE(2), CASE(3)
+  bool done = false;
   if (leaf_binned_current_pays(np, a.g)) {
-    r = direct ? leaf_binned_direct(a, (int)nox, st) : leaf_binned_esirkepov(a, (int)nox, st);
+    r = direct ? leaf_binned_direct(a, (int)nox, st, done)
+               : leaf_binned_esirkepov(a, (int)nox, st, done);
     if (r) return r;
+  }
+  if (done) {
   } else if (direct) {
     if (nox == 1) hipLaunchKernelGGL(k_direct<1>, grd, blk, 0, st, a);
     else if (nox == 2) hipLaunchKernelGGL(k_direct<2>, grd, blk, 0, st, a);
@@ -1137,9 +1146,12 @@ int pxrhip_depose_rho_n(double *rho, int64_t np, const double *xp, const double 
   a.bad = rt().d_bad;
   dim3 grd(grid1d(np, 256 * DEP_S)), blk(256);
   hipStream_t st = rt().stream;
+  bool done = false;
   if (leaf_binned_rho_pays(np, a.g)) {
-    r = leaf_binned_rho(a, (int)nox, st);
+    r = leaf_binned_rho(a, (int)nox, st, done);
     if (r) return r;
+  }
+  if (done) {
   } else if (nox == 1) hipLaunchKernelGGL(k_rho<1>, grd, blk, 0, st, a);
   else if (nox == 2) hipLaunchKernelGGL(k_rho<2>, grd, blk, 0, st, a);
   else hipLaunchKernelGGL(k_rho<3>, grd, blk, 0, st, a);

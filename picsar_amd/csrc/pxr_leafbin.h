@@ -19,6 +19,19 @@ struct DepoArgs {
   unsigned long long *bad;
 };
 
+// one call of geteb3d_energy_conserving with one order on all axes
+struct LeafGatherArgs {
+  i64 np;
+  const double *xp, *yp, *zp;
+  double *ex, *ey, *ez, *bx, *by, *bz;
+  double xmin, ymin, zmin, dxi, dyi, dzi, s;
+  GridGeom g;
+  const double *exg, *eyg, *ezg, *bxg, *byg, *bzg;
+  unsigned long long *bad;
+  const int *skip;  // not null: k_gather leaves the set alone if *skip is set
+  LeafGatherArgs part(i64 first, i64 n) const;  // the same call for n particles from `first`
+};
+
 // charge density of one call of pxr_depose_rho_n
 struct RhoArgs {
   i64 np;
@@ -46,13 +59,25 @@ struct GlobalAcc {
 // and each block's current (or charge) is summed in LDS
 // before one global add per node.  Return PXRHIP_OK, or an error code
 // (scratch memory could not be allocated) before anything is launched.
-int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st);
-int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st);
-int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st);
+int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, bool &done);
+int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, bool &done);
+int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done);
 // whether a call of np particles on grid g takes the binned form: at least
 // the runtime's leaf_bin_min particles and one per block, and no graph
 // capture open (the scratch may have to grow)
 bool leaf_binned_current_pays(i64 np, const GridGeom &g);
 bool leaf_binned_rho_pays(i64 np, const GridGeom &g);
+
+// The gather of a set in no order: particles ordered by blocks, the block's
+// fields staged in LDS.  A set in cell order reads the grid arrays through the
+// caches faster without, so for a call that may gain a probe looks at the
+// order first.  leaf_probe_start sets a.skip, so that the plain kernel can be
+// launched behind it at once and steps aside for a set in no order;
+// leaf_probe_read waits for the answer.  leaf_binned_gather returns how many
+// particles are done: all of them, or fewer where it ran out of memory.
+bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order);
+int leaf_probe_start(LeafGatherArgs &a, hipStream_t st);
+int leaf_probe_read(bool &scattered);
+int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st, i64 &done);
 
 }  // namespace pxr

@@ -1,5 +1,6 @@
-// pxr_leafbin.hip -- the leaf current and charge deposition (depose_jxjyjz,
-// pxr_depose_rho_n) for large particle sets, summed block by block in LDS.
+// pxr_leafbin.hip -- the leaf routines on large particle sets, block by block in
+// LDS: the current and charge deposition (depose_jxjyjz, pxr_depose_rho_n) and
+// the field gather.
 //
 // A caller of the leaf routines hands over particles in any order, anywhere
 // in the grid arrays.  Adding every contribution to global memory costs one
@@ -15,9 +16,11 @@
 //
 // The contributions are the same arithmetic as the global-atomic kernels
 // (esirkepov_deposit, direct_deposit, the nodal shapes of pxr_depose_rho_n);
-// only the order of the FP64 sums differs.  Nothing synchronises with the
-// host, so the sequence can be captured in a HIP graph once its scratch is
-// allocated.
+// only the order of the FP64 sums differs.  A call that has no memory for the
+// ordering, or that is captured in a HIP graph, takes the unbinned kernel.
+//
+// The gather of the fields (geteb3d_energy_conserving) uses the same order
+// for a large set whose particles are in none.
 #include <algorithm>
 
 #include "pxr_leafbin.h"
@@ -61,6 +64,13 @@ struct LbPos {
   const double *x, *y, *z, *ux, *uy, *uz, *gi;
   double xmin, ymin, zmin, dxi, dyi, dzi, h[3];
   int l4symtry;
+  double *rec;  // not null: the normalised positions go to 6-double records too
+};
+
+// arguments of the binned gather: the call's, and the particles' records
+struct LbGather {
+  LeafGatherArgs c;
+  double *rec;
 };
 
 // Block of every particle, by the node of its position (MID: of its
@@ -79,6 +89,11 @@ __global__ __launch_bounds__(256) void k_lb_keys(LbPos a, BinGeom bg, int *key) 
   } else if (a.l4symtry) {
     x = fabs(x);
     y = fabs(y);
+  }
+  if (a.rec) {
+    a.rec[6 * ip] = x;
+    a.rec[6 * ip + 1] = y;
+    a.rec[6 * ip + 2] = z;
   }
   key[ip] = block_axis<B>(x, bg.gd[0], bg.na[0]) +
             bg.nb[0] * (block_axis<B>(y, bg.gd[1], bg.na[1]) +
@@ -313,18 +328,122 @@ __global__ __launch_bounds__(256) void k_lb_rho(RhoArgs a, BinGeom bg, const int
   }
 }
 
+// Gather: the stencils of a particle at x lie within [floor(x) - 1,
+// floor(x) + 2], and with a staggered shape of order 3 from floor(x) - 2 on.
+// One workgroup per work item stages the six blocks, as the tiled kernel
+// does, and its particles read them there.
+//
+// In random order k_gather is bound by its cache lines: 96 rows of three or
+// four nodes per order-3 particle, each in lines that no other lane of the
+// wave wants.  Staged, a line is read once per work item.  What is left are
+// the particles' own scattered accesses, so those go through one record of
+// 48 bytes per particle (its position, then its six field values) instead of
+// three reads and six read-modify-writes in nine arrays.  Two million order-3
+// particles on 64^3 cells: 1.35 ms plain, 0.67 ms staged, 0.46 ms with the
+// records (ordering 0.09 ms); 16 million on 128^3: 22.9 -> 3.6 ms.
+template <int N, int M, int B>
+__global__ __launch_bounds__(512) void k_lb_gather(LbGather a, BinGeom bg, const int *perm,
+                                                   const int4 *items, const int *nitems) {
+  constexpr int HLO = M == 3 ? -2 : -1, HHI = 2, L = B + HHI - HLO, LN = L * L * L;
+  extern __shared__ double lds[];
+  const int nit = *nitems;
+  const i64 org = a.c.g.idx(0, 0, 0);
+  FieldView<double> fg[6];
+  const double *F[6] = {a.c.exg, a.c.eyg, a.c.ezg, a.c.bxg, a.c.byg, a.c.bzg};
+  for (int f = 0; f < 6; f++) fg[f] = FieldView<double>{F[f] + org, a.c.g.NX, a.c.g.NX * a.c.g.NY};
+  for (int w = blockIdx.x; w < nit; w += gridDim.x) {
+    const int4 it = items[w];
+    const int b = it.x;
+    const int o[3] = {b % bg.nb[0] * B - bg.gd[0] + HLO, b / bg.nb[0] % bg.nb[1] * B - bg.gd[1] + HLO,
+                      b / (bg.nb[0] * bg.nb[1]) * B - bg.gd[2] + HLO};
+    __syncthreads();  // the previous item's block is no longer read
+    for (int t = threadIdx.x; t < LN; t += 512) {
+      const int i = o[0] + t % L, j = o[1] + t / L % L, k = o[2] + t / (L * L);
+      const bool in = a.c.g.inside(i, j, k);
+      const i64 ix = in ? a.c.g.idx(i, j, k) : 0;
+      double v[6];
+#pragma unroll
+      for (int f = 0; f < 6; f++) v[f] = in ? F[f][ix] : 0.0;
+#pragma unroll
+      for (int f = 0; f < 6; f++) lds[f * LN + t] = v[f];
+    }
+    __syncthreads();
+    LdsView<double> fl[6];
+    for (int f = 0; f < 6; f++) fl[f] = LdsView<double>{lds + f * LN, o[0], o[1], o[2], L, L * L};
+    for (int p = threadIdx.x; p < it.z; p += 512) {
+      double *rec = a.rec + 6 * (i64)perm[it.y + p];
+      const double x = rec[0], y = rec[1], z = rec[2];
+      GatherStencil<N, M, double> st;
+      gather_stencil<N, M, double>(st, x, y, z, a.c.s);
+      int lo[3], hi[3];
+      gather_bounds<N, M, double>(st, lo, hi);
+      bool held = a.c.g.inside(lo[0], lo[1], lo[2]) && a.c.g.inside(hi[0], hi[1], hi[2]);
+      for (int d = 0; d < 3; d++) held = held && lo[d] >= o[d] && hi[d] < o[d] + L;
+      double e[6];
+      if (held) {
+        gather_apply<N, M, double>(st, fl, e);
+      } else if (!gather_eb<N, M, double>(x, y, z, a.c.s, a.c.g, fg, e)) {
+        count_bad(a.c.bad);  // outside the arrays
+        for (int f = 0; f < 6; f++) e[f] = -0.0;  // the outputs stay as they are
+      }
+#pragma unroll
+      for (int f = 0; f < 6; f++) rec[f] = e[f];
+    }
+  }
+}
+
+// the records' field values added to the caller's arrays
+__global__ __launch_bounds__(256) void k_lb_gather_add(LeafGatherArgs a, const double *rec) {
+  const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (ip >= a.np) return;
+  const double2 *r = (const double2 *)(rec + 6 * ip);
+  const double2 r0 = r[0], r1 = r[1], r2 = r[2];
+  a.ex[ip] += r0.x;
+  a.ey[ip] += r0.y;
+  a.ez[ip] += r1.x;
+  a.bx[ip] += r1.y;
+  a.by[ip] += r2.x;
+  a.bz[ip] += r2.y;
+}
+
+// One workgroup looks at 64 runs of 64 consecutive particles spread over the
+// set: it is in no order if most particles have another block than their
+// predecessor (a set in cell order crosses blocks a few times a run).
+template <int B>
+__global__ __launch_bounds__(1024) void k_lb_probe(LbPos a, BinGeom bg, int *out, int *host_out) {
+  __shared__ int s[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int b[4], n = 0;
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const i64 ip = (a.np - 64) * (4 * wave + r) / 63 + lane;
+    b[r] = block_axis<B>((a.x[ip] - a.xmin) * a.dxi, bg.gd[0], bg.na[0]) +
+           bg.nb[0] * (block_axis<B>((a.y[ip] - a.ymin) * a.dyi, bg.gd[1], bg.na[1]) +
+                       bg.nb[1] * block_axis<B>((a.z[ip] - a.zmin) * a.dzi, bg.gd[2], bg.na[2]));
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) n += __popcll(__ballot(lane > 0 && b[r] != __shfl_up(b[r], 1)));
+  if (lane == 0) s[wave] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; w++) n += s[w];
+    *out = *host_out = n > 64 * 24;
+  }
+}
+
 // Particle indices in block order (radix sort: the input order is kept
 // inside a block) and the work items.  Counting and placing the particles
 // with global atomics on the blocks' counters took 0.32 ms for two million
-// in random order (every particle its own atomic), this 0.09 ms.
+// in random order (every particle its own atomic), this 0.09 ms.  Returns false,
+// with nothing launched, for a set it has no memory or index range for.
 template <int B, bool MID>
-static int lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st, BinGeom &bg,
-                   int *&perm, int4 *&items, int *&nitems, i64 &maxitems) {
+static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st, BinGeom &bg,
+                    int *&perm, int4 *&items, int *&nitems, i64 &maxitems) {
   bg = make_bin_geom(g, B);
   const i64 np = a.np;
   maxitems = bg.nblocks + np / chunk + 1;
   if (np >= (i64)1 << 31 || bg.nblocks >= (i64)1 << 31 || maxitems >= (i64)1 << 31)
-    return set_error(PXRHIP_ERR_ARG, "binned deposition: more than 2^31 particles or blocks");
+    return false;
   const RadixPlan plan = radix_plan(np, bg.nblocks, (i64)1 << 21);
   int *keys = (int *)scratch(24, 2 * sizeof(int) * (size_t)np);
   int *idxs = (int *)scratch(25, 2 * sizeof(int) * (size_t)np);
@@ -332,8 +451,7 @@ static int lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st,
   int *first = (int *)scratch(27, sizeof(int) * (size_t)(bg.nblocks + 1));
   items = (int4 *)scratch(28, sizeof(int4) * (size_t)maxitems);
   nitems = (int *)scratch(29, sizeof(int));
-  if (!keys || !idxs || !hist || !first || !items || !nitems)
-    return set_error(PXRHIP_ERR_HIP, "binned deposition: out of device memory");
+  if (!keys || !idxs || !hist || !first || !items || !nitems) return false;
   int *key[2] = {keys, keys + np}, *idx[2] = {idxs, idxs + np};
   hipLaunchKernelGGL((k_lb_keys<B, MID>), dim3(grid1d(np, 256)), dim3(256), 0, st, a, bg, keys);
   const int at = radix_sort(plan, key, idx, hist, st);
@@ -342,11 +460,19 @@ static int lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st,
                      bg.nblocks, first);
   hipLaunchKernelGGL(k_lb_plan, dim3(1), dim3(1024), 0, st, first, bg.nblocks, chunk, items,
                      nitems);
-  PXR_LAUNCHED();
-  return PXRHIP_OK;
+  return true;
 }
 
 constexpr int LB_EDGE = 8;  // nodes per block edge
+// Particles from which a gather asks for their order, at order 2 and 3.  The
+// question costs a call in cell order 4 to 8 us, so it has to be a small part
+// of the call: order 3, a million on 64^3 cells, 152 -> 156 us in cell order
+// and 615 -> 293 in random order; order 2, two million, 154 -> 160 and
+// 900 -> 371 (a million: 101 us in cell order).  At order 1 a particle's
+// eight-node reads cost no more than ordering it (a million 201 us plain, 395
+// binned).
+constexpr i64 GATHER_BIN_MIN2 = 3 << 19, GATHER_BIN_MIN3 = 3 << 18;
+constexpr int GATHER_CHUNK = 1024;  // particles of a gather's work item
 
 // persistent workgroups: as many as the CUs hold at this LDS size, or one
 // per work item if there are fewer
@@ -369,20 +495,90 @@ static bool pays(i64 np, const GridGeom &g, int edge) {
          np >= make_bin_geom(g, edge).nblocks;
 }
 
+static LbPos gather_pos(const LeafGatherArgs &a, double *rec) {
+  return LbPos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, a.xmin, a.ymin, a.zmin,
+               a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, 0, rec};
+}
+
+LeafGatherArgs LeafGatherArgs::part(i64 first, i64 n) const {
+  LeafGatherArgs p = *this;
+  p.np = n;
+  for (const double **q : {&p.xp, &p.yp, &p.zp}) *q += first;
+  for (double **q : {&p.ex, &p.ey, &p.ez, &p.bx, &p.by, &p.bz}) *q += first;
+  return p;
+}
+
+bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order) {
+  return order >= 2 && rt().checks && pays(a.np, a.g, LB_EDGE) &&
+         a.np >= (order == 3 ? GATHER_BIN_MIN3 : GATHER_BIN_MIN2);
+}
+
+int leaf_probe_start(LeafGatherArgs &a, hipStream_t st) {
+  int *out = (int *)(rt().d_bad + 2);
+  hipLaunchKernelGGL(k_lb_probe<LB_EDGE>, dim3(1), dim3(1024), 0, st, gather_pos(a, nullptr),
+                     make_bin_geom(a.g, LB_EDGE), out, rt().h_probe);
+  PXR_LAUNCHED();
+  PXR_HIP(hipEventRecord(rt().probe_done, st));
+  a.skip = out;
+  return PXRHIP_OK;
+}
+
+int leaf_probe_read(bool &scattered) {
+  PXR_HIP(hipEventSynchronize(rt().probe_done));
+  scattered = *(volatile int *)rt().h_probe != 0;
+  return PXRHIP_OK;
+}
+
+int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st,
+                       i64 &done) {
+  const i64 nblocks = make_bin_geom(a.g, LB_EDGE).nblocks;
+  const i64 most = std::max<i64>((i64)1 << 22, 512 * nblocks);
+  const i64 nparts = (a.np + most - 1) / most, size = (a.np + nparts - 1) / nparts;
+  const int L = LB_EDGE + (order == 3 && !lower ? 4 : 3);
+  const size_t lds = sizeof(double) * 6 * (size_t)(L * L * L);
+  done = 0;
+  LbGather ga;
+  if (!(ga.rec = (double *)scratch(30, 6 * sizeof(double) * (size_t)size))) return PXRHIP_OK;
+  while (done < a.np) {
+    ga.c = a.part(done, std::min(size, a.np - done));
+    BinGeom bg;
+    int *perm, *nitems;
+    int4 *items;
+    i64 maxitems;
+    if (!lb_sort<LB_EDGE, false>(gather_pos(ga.c, ga.rec), a.g,
+                                 std::min(rt().leaf_bin_chunk, GATHER_CHUNK), st, bg, perm, items,
+                                 nitems, maxitems))
+      return PXRHIP_OK;
+    const dim3 grd(lb_grid(maxitems, lds)), blk(512);
+    switch (order * 2 + (lower ? 1 : 0)) {
+      case 4: LB_LAUNCH((k_lb_gather<2, 2, LB_EDGE>), ga); break;
+      case 5: LB_LAUNCH((k_lb_gather<2, 1, LB_EDGE>), ga); break;
+      case 6: LB_LAUNCH((k_lb_gather<3, 3, LB_EDGE>), ga); break;
+      default: LB_LAUNCH((k_lb_gather<3, 2, LB_EDGE>), ga); break;
+    }
+    hipLaunchKernelGGL(k_lb_gather_add, dim3(grid1d(ga.c.np, 256)), dim3(256), 0, st, ga.c,
+                       ga.rec);
+    PXR_LAUNCHED();
+    done += ga.c.np;
+  }
+  return PXRHIP_OK;
+}
+
 bool leaf_binned_current_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
 bool leaf_binned_rho_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
 
-int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st) {
+int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, bool &done) {
+  done = false;
   BinGeom bg;
   int *perm, *nitems;
   int4 *items;
   i64 maxitems;
   const EsirkConst<double> &c = a.ec;
   const LbPos pos{a.np, a.xp, a.yp, a.zp, a.ux, a.uy, a.uz, a.gi, c.xmin, c.ymin, c.zmin, c.dxi,
-                  c.dyi, c.dzi, {0.5 * c.dtsdx0, 0.5 * c.dtsdy0, 0.5 * c.dtsdz0}, 0};
-  int r = lb_sort<LB_EDGE, true>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems,
-                                 maxitems);
-  if (r) return r;
+                  c.dyi, c.dzi, {0.5 * c.dtsdx0, 0.5 * c.dtsdy0, 0.5 * c.dtsdz0}, 0, nullptr};
+  if (!lb_sort<LB_EDGE, true>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems,
+                                 maxitems))
+    return PXRHIP_OK;
   const int L = LB_EDGE + (order == 1 ? 3 : 5);
   const size_t lds = sizeof(double) * 3 * (size_t)(L * L * L);
   const dim3 grd(lb_grid(maxitems, lds)), blk(256);
@@ -390,20 +586,22 @@ int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st) {
   else if (order == 2) LB_LAUNCH((k_lb_direct<2, LB_EDGE>), a);
   else LB_LAUNCH((k_lb_direct<3, LB_EDGE>), a);
   PXR_LAUNCHED();
+  done = true;
   return PXRHIP_OK;
 }
 
-int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st) {
+int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, bool &done) {
+  done = false;
   BinGeom bg;
   int *perm, *nitems;
   int4 *items;
   i64 maxitems;
   const EsirkConst<double> &c = a.ec;
   const LbPos pos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, c.xmin, c.ymin,
-                  c.zmin, c.dxi, c.dyi, c.dzi, {0.0, 0.0, 0.0}, 0};
-  int r = lb_sort<LB_EDGE, false>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems,
-                                  maxitems);
-  if (r) return r;
+                  c.zmin, c.dxi, c.dyi, c.dzi, {0.0, 0.0, 0.0}, 0, nullptr};
+  if (!lb_sort<LB_EDGE, false>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems,
+                                  maxitems))
+    return PXRHIP_OK;
   const int L = LB_EDGE + (order == 1 ? 3 : 5);
   const size_t lds = sizeof(double) * 3 * (size_t)(L * L * L);
   const dim3 grd(lb_grid(maxitems, lds)), blk(256);
@@ -411,19 +609,21 @@ int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st) {
   else if (order == 2) LB_LAUNCH((k_lb_esirkepov<2, LB_EDGE>), a);
   else LB_LAUNCH((k_lb_esirkepov<3, LB_EDGE>), a);
   PXR_LAUNCHED();
+  done = true;
   return PXRHIP_OK;
 }
 
-int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st) {
+int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done) {
+  done = false;
   constexpr int E = LB_EDGE;
   BinGeom bg;
   int *perm, *nitems;
   int4 *items;
   i64 maxitems;
   const LbPos pos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, a.xmin, a.ymin,
-                  a.zmin, a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, a.l4symtry};
-  int r = lb_sort<E, false>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems, maxitems);
-  if (r) return r;
+                  a.zmin, a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, a.l4symtry, nullptr};
+  if (!lb_sort<E, false>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems, maxitems))
+    return PXRHIP_OK;
   const int L = E + (order == 1 ? 1 : 3);
   const size_t lds = sizeof(double) * (size_t)(L * L * L);
   const dim3 grd(lb_grid(maxitems, lds)), blk(256);
@@ -431,6 +631,7 @@ int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st) {
   else if (order == 2) LB_LAUNCH((k_lb_rho<2, E>), a);
   else LB_LAUNCH((k_lb_rho<3, E>), a);
   PXR_LAUNCHED();
+  done = true;
   return PXRHIP_OK;
 }
 

@@ -15,7 +15,10 @@ struct Runtime {
   bool own_stream = false;  // created by pxrhip_init
   bool capturing = false;   // a graph capture of the stream is open
   bool checks = true;
-  unsigned long long *d_bad = nullptr;  // device counter of skipped particles
+  // device counter of skipped particles; [2] holds the answer of k_lb_probe
+  unsigned long long *d_bad = nullptr;
+  int *h_probe = nullptr;               // pinned host int that a kernel reports through
+  hipEvent_t probe_done = nullptr;
   int num_cus = 256;
   // leaf deposition summed in LDS blocks (pxr_leafbin.hip) from this many
   // particles on (0: never), work items of at most leaf_bin_chunk particles
@@ -30,7 +33,9 @@ struct Runtime {
 Runtime &rt();
 int set_error(int code, const char *fmt, ...);
 int ensure_init();
-// library-owned scratch buffer number `slot`, grown to at least `bytes`
+// library-owned scratch buffer number `slot`, grown to at least `bytes`; null
+// if there is no memory for it (with the runtime's error state cleared, so
+// that a caller that has a form without scratch can launch that)
 void *scratch(int slot, size_t bytes);
 // read the bad-particle counter (synchronises the stream), reset it to 0
 int take_bad(unsigned long long *n);

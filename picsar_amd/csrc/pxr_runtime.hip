@@ -15,6 +15,7 @@ static thread_local char g_err[1024] = "";
 struct Scratch {
   void *p = nullptr;
   size_t bytes = 0;
+  bool in_graph = false;  // handed out while a graph was recorded
 };
 static std::vector<Scratch> g_scratch(32);
 
@@ -36,17 +37,20 @@ int ensure_init() {
 void *scratch(int slot, size_t bytes) {
   if (slot < 0 || slot >= (int)g_scratch.size()) return nullptr;
   Scratch &s = g_scratch[slot];
+  if (g_rt.capturing) s.in_graph = true;
   if (s.bytes >= bytes && s.p) return s.p;
   if (s.p) {
     hipStreamSynchronize(g_rt.stream);
     hipFree(s.p);
     s.p = nullptr;
     s.bytes = 0;
-    g_rt.mem_gen++;
+    if (s.in_graph) g_rt.mem_gen++;
+    s.in_graph = g_rt.capturing;
   }
   size_t want = bytes < 4096 ? 4096 : bytes;
   if (hipMalloc(&s.p, want) != hipSuccess) {
     s.p = nullptr;
+    (void)hipGetLastError();
     return nullptr;
   }
   s.bytes = want;
@@ -86,9 +90,11 @@ int pxrhip_init(int device) {
     g_rt.own_stream = true;
   }
   if (!g_rt.d_bad) {
-    PXR_HIP(hipMalloc(&g_rt.d_bad, 2 * sizeof(unsigned long long)));
-    PXR_HIP(hipMemset(g_rt.d_bad, 0, 2 * sizeof(unsigned long long)));
+    PXR_HIP(hipMalloc(&g_rt.d_bad, 3 * sizeof(unsigned long long)));
+    PXR_HIP(hipMemset(g_rt.d_bad, 0, 3 * sizeof(unsigned long long)));
   }
+  if (!g_rt.h_probe) PXR_HIP(hipHostMalloc(&g_rt.h_probe, sizeof(int), 0));
+  if (!g_rt.probe_done) PXR_HIP(hipEventCreateWithFlags(&g_rt.probe_done, hipEventDisableTiming));
   g_rt.device = dev;
   return PXRHIP_OK;
 }
@@ -103,6 +109,10 @@ int pxrhip_finalize(void) {
   }
   if (g_rt.d_bad) hipFree(g_rt.d_bad);
   g_rt.d_bad = nullptr;
+  if (g_rt.h_probe) hipHostFree(g_rt.h_probe);
+  g_rt.h_probe = nullptr;
+  if (g_rt.probe_done) hipEventDestroy(g_rt.probe_done);
+  g_rt.probe_done = nullptr;
   if (g_rt.own_stream && g_rt.stream) hipStreamDestroy(g_rt.stream);
   g_rt.stream = nullptr;
   g_rt.own_stream = false;
