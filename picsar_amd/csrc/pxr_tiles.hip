@@ -1256,8 +1256,22 @@ struct RhoTileArgs {
   unsigned long long *bad;
 };
 
+struct Pair {  // aligned to a double only
+  double v[2];
+};
+
+// A thread takes up to G consecutive particles of the work item: binned
+// particles lie in cell order, and lanes that all add to the nodes of one
+// cell wait for each other.  The more adds a particle makes, the more the
+// spread pays against the lines of particle data that it keeps in flight;
+// loads of two particles at a time keep those few.  Both species of 8
+// particles per cell on 96^3 cells (consecutive lanes -> G = 4, 8, 16):
+// order 1 289 -> 258 us, order 2 1296 -> 440, order 3 1385 -> 880; 64 per
+// cell on 48^3: 397 -> 376, 2069 -> 1290, 2146 -> 1241.  The LDS adds bound
+// order 3 (1.1 T adds/s).
 template <int N>
 __global__ __launch_bounds__(256) void k_rho_tiles(RhoTileArgs a) {
+  constexpr int G = N == 1 ? 4 : N == 2 ? 8 : 16;
   extern __shared__ double srho[];
   __shared__ int s_chunk;
   const GridGeom &g = a.g;
@@ -1288,35 +1302,53 @@ __global__ __launch_bounds__(256) void k_rho_tiles(RhoTileArgs a) {
     const int nb = blk ? e[0] * e[1] * e[2] : 0;
     for (int i = threadIdx.x; i < nb; i += 256) srho[i] = 0.0;
     __syncthreads();
-    for (int k = threadIdx.x; k < ch.n; k += 256) {
-      const i64 p = ch.begin + k;
-      double sx[N + 1], sy[N + 1], sz[N + 1];
-      const int j0 = shape_nodal<N, double>((a.x[p] - a.xmin) * a.dxi, sx);
-      const int k0 = shape_nodal<N, double>((a.y[p] - a.ymin) * a.dyi, sy);
-      const int l0 = shape_nodal<N, double>((a.z[p] - a.zmin) * a.dzi, sz);
-      const double w = a.mixed ? (double)((const float *)a.w)[p] : ((const double *)a.w)[p];
-      const double wq = a.q * w * a.invvol;
-      if (blk && j0 >= R0[0] && j0 + N < R0[0] + e[0] && k0 >= R0[1] && k0 + N < R0[1] + e[1] &&
-          l0 >= R0[2] && l0 + N < R0[2] + e[2]) {
-        double *r = srho + (j0 - R0[0]) + e[0] * ((k0 - R0[1]) + e[1] * (l0 - R0[2]));
+    for (int kb = 0; kb < ch.n; kb += 256 * G) {
+      const int S = min(G, (ch.n - kb + 255) / 256);
+      const int first = kb + (int)threadIdx.x * S, last = min(first + S, ch.n);
+      for (int k = first; k < last; k += 2) {
+        const i64 p = ch.begin + k;
+        const int two = k + 1 < last;
+        Pair px, py, pz;
+        double w[2];
+        if (two) {
+          px = *(const Pair *)(a.x + p);
+          py = *(const Pair *)(a.y + p);
+          pz = *(const Pair *)(a.z + p);
+        } else {
+          px.v[0] = a.x[p]; py.v[0] = a.y[p]; pz.v[0] = a.z[p];
+        }
+        w[0] = a.mixed ? (double)((const float *)a.w)[p] : ((const double *)a.w)[p];
+        if (two) w[1] = a.mixed ? (double)((const float *)a.w)[p + 1] : ((const double *)a.w)[p + 1];
+        for (int h = 0; h <= two; h++) {
+          double sx[N + 1], sy[N + 1], sz[N + 1];
+          const int j0 = shape_nodal<N, double>(((h ? px.v[1] : px.v[0]) - a.xmin) * a.dxi, sx);
+          const int k0 = shape_nodal<N, double>(((h ? py.v[1] : py.v[0]) - a.ymin) * a.dyi, sy);
+          const int l0 = shape_nodal<N, double>(((h ? pz.v[1] : pz.v[0]) - a.zmin) * a.dzi, sz);
+          const double wq = a.q * (h ? w[1] : w[0]) * a.invvol;
+          if (blk && j0 >= R0[0] && j0 + N < R0[0] + e[0] && k0 >= R0[1] &&
+              k0 + N < R0[1] + e[1] && l0 >= R0[2] && l0 + N < R0[2] + e[2]) {
+            double *r = srho + (j0 - R0[0]) + e[0] * ((k0 - R0[1]) + e[1] * (l0 - R0[2]));
 #pragma unroll
-        for (int cc = 0; cc <= N; cc++)
+            for (int cc = 0; cc <= N; cc++)
 #pragma unroll
-          for (int bb = 0; bb <= N; bb++)
+              for (int bb = 0; bb <= N; bb++)
 #pragma unroll
-            for (int aa = 0; aa <= N; aa++)
-              atomicAdd(r + aa + e[0] * (bb + e[1] * cc), sx[aa] * sy[bb] * sz[cc] * wq);
-      } else if (g.inside(j0, k0, l0) && g.inside(j0 + N, k0 + N, l0 + N)) {
-        double *r = a.rho + g.idx(j0, k0, l0);
+                for (int aa = 0; aa <= N; aa++)
+                  atomicAdd(r + aa + e[0] * (bb + e[1] * cc), sx[aa] * sy[bb] * sz[cc] * wq);
+          } else if (g.inside(j0, k0, l0) && g.inside(j0 + N, k0 + N, l0 + N)) {
+            double *r = a.rho + g.idx(j0, k0, l0);
 #pragma unroll
-        for (int cc = 0; cc <= N; cc++)
+            for (int cc = 0; cc <= N; cc++)
 #pragma unroll
-          for (int bb = 0; bb <= N; bb++)
+              for (int bb = 0; bb <= N; bb++)
 #pragma unroll
-            for (int aa = 0; aa <= N; aa++)
-              unsafeAtomicAdd(r + aa + g.NX * (bb + g.NY * (i64)cc), sx[aa] * sy[bb] * sz[cc] * wq);
-      } else {
-        count_bad(a.bad);
+                for (int aa = 0; aa <= N; aa++)
+                  unsafeAtomicAdd(r + aa + g.NX * (bb + g.NY * (i64)cc),
+                                  sx[aa] * sy[bb] * sz[cc] * wq);
+          } else {
+            count_bad(a.bad);
+          }
+        }
       }
     }
     __syncthreads();
