@@ -859,6 +859,7 @@ struct ChunkArgs {
   const int64_t *bin_base;
   int *count;       // chunks per unit (tile, plane)
   int *group;       // per unit: last plane of the plane group it heads, or GROUP_*
+  Chunk *stage;     // the first STAGE chunks of every unit, or null
   i64 *start;       // exclusive scan of count, nunits+1 entries
   Chunk *out;
   int *nchunks, *queue;
@@ -874,13 +875,27 @@ constexpr int GROUP_ROWS = -1;    // cut into runs of rows by walk_unit
 constexpr int GROUP_MEMBER = -2;  // inside a group headed by an earlier plane
 constexpr int GROUP_EMPTY = -3;   // no particles
 
-// whether the field and current blocks of the particles of tile t in rows
-// y0..y1 of planes z0..z1 fit the LDS budgets
-PXR_DEV bool blocks_fit(const ChunkArgs &a, int t, int z0, int z1, int y0, int y1) {
-  double ulo[3], uhi[3];
-  int FR0[3], fe[3], JR0[3], je[3];
-  rows_range(a.bg, t, z0, z1, y0, y1, ulo, uhi);
-  blocks_for(a.bg, ulo, uhi, FR0, fe, JR0, je);
+// The test whether the field and current blocks of the particles of a tile
+// in rows y0..y1 of planes z0..z1 fit the LDS budgets, axis by axis (as
+// rows_range and blocks_for do for all three): a walk along one axis computes
+// the others once.
+struct AxisFit {
+  double so, lo, hi;  // origin of the sorting grid, membership of the tile
+  PXR_DEV AxisFit(const ChunkArgs &a, int t, int d)
+      : so(a.bg.sorg[3 * t + d]), lo(a.bg.tbox[6 * t + d]), hi(a.bg.tbox[6 * t + 3 + d]) {}
+  // nodes of the field and current blocks along axis d for sorting cells c0..c1
+  PXR_DEV void extent(const BoxGeom &b, int d, int c0, int c1, int &fe, int &je) const {
+    const double ulo = (fmax(so + b.sd[d] * c0, lo) - b.x0[d]) * b.di[d] - 1e-7;
+    const double uhi = (fmin(so + b.sd[d] * (c1 + 1), hi) - b.x0[d]) * b.di[d] + 1e-7;
+    int l, h;
+    gather_range(b, ulo, uhi, l, h);
+    fe = max(min(h, b.ghi[d]) - max(l, b.glo[d]) + 1, 0);
+    deposit_range(b, ulo, uhi, b.mv[d], l, h);
+    je = max(min(h, b.ghi[d]) - max(l, b.glo[d]) + 1, 0);
+  }
+};
+
+PXR_DEV bool blocks_fit(const ChunkArgs &a, const int *fe, const int *je) {
   // current block, with room for jroom nodes of motion on each side (the
   // block of k_fused is the box of the pushed particles; for a species whose
   // blocks k_fused_cut can cut down no room is needed) and for its odd
@@ -894,11 +909,14 @@ PXR_DEV bool blocks_fit(const ChunkArgs &a, int t, int z0, int z1, int y0, int y
 // The chunker gives CG lanes to a tile (grouping its planes) or a plane
 // (cutting its rows): the lanes load the counts of CG planes or rows and test
 // CG candidate ends against the LDS budgets at once, and the first that fails
-// closes the group or chunk.  One thread walking them one by one waited for
-// two dependent loads and a block geometry per row: 57 + 59 us for the 34
-// planes of one 33^3-node tile, now 23 + 27 us (37 + 35, now 12 + 14, for
-// 61 x 45 x 70 cells in 60 tiles; grouping the planes of the 4096 tiles of a
-// 128^3 bunch 40, now 21 us).
+// closes the group or chunk.  Row starts are staged in LDS, the block
+// extents along the axes that a walk keeps are computed once, and where there
+// are few units the chunks found while counting are kept for k_chunk_write.
+// The 34 planes of one 33^3-node tile, counted and written: 57 + 59 us with
+// one thread a plane, 23 + 27 us with CG lanes that read rows and geometry
+// from memory at each step and walked twice, now 15 + 4 us (61 x 45 x 70
+// cells in 60 tiles: 37 + 35, 12 + 14, now 9 + 5 us; grouping the planes of
+// the 4096 tiles of a 128^3 bunch: 40, 21, now 12 us).
 constexpr int CG = 16;
 
 // the bits of this lane's group in a ballot
@@ -930,6 +948,14 @@ __global__ __launch_bounds__(256) void k_chunk_groups(ChunkArgs a) {
   }
   for (int z = nz3 + lane; z < a.nzmax; z += CG) grp[z] = GROUP_EMPTY;
   const i64 plane = (i64)ny3 * nx3, base = a.bin_base[t];
+  int fe[3], je[3];
+  AxisFit(a, t, 0).extent(a.bg, 0, 0, nx3 - 1, fe[0], je[0]);
+  AxisFit(a, t, 1).extent(a.bg, 1, 0, ny3 - 1, fe[1], je[1]);
+  const AxisFit az(a, t, 2);
+  auto fit = [&](int z0, int z1) {
+    az.extent(a.bg, 2, z0, z1, fe[2], je[2]);
+    return blocks_fit(a, fe, je);
+  };
   auto count = [&](int z) {
     return z < nz3 ? a.bin_start[base + (z + 1) * plane] - a.bin_start[base + z * plane] : 0;
   };
@@ -938,7 +964,7 @@ __global__ __launch_bounds__(256) void k_chunk_groups(ChunkArgs a) {
     // planes z .. z + CG - 1: empty ones, ones to be cut, ones that may group
     const i64 n = count(z + lane);
     const bool in = z + lane < nz3, empty = n <= 0;
-    const bool cut = !empty && (n > a.ch || !blocks_fit(a, t, z + lane, z + lane, 0, ny3 - 1));
+    const bool cut = !empty && (n > a.ch || !fit(z + lane, z + lane));
     const unsigned whole = cg_ballot(in && !empty && !cut);
     const int skip = whole ? __ffs(whole) - 1 : CG;  // planes before the first groupable one
     if (in && lane < skip) grp[z + lane] = empty ? GROUP_EMPTY : GROUP_ROWS;
@@ -949,7 +975,7 @@ __global__ __launch_bounds__(256) void k_chunk_groups(ChunkArgs a) {
     for (int w = z;; w += CG) {
       const i64 m = count(w + lane);
       const i64 tot = sum + cg_scan(m, lane);
-      const bool ok = m > 0 && tot <= a.ch && blocks_fit(a, t, z, w + lane, 0, ny3 - 1);
+      const bool ok = m > 0 && tot <= a.ch && fit(z, w + lane);
       const unsigned bad = cg_ballot(!ok);
       if (bad) {
         z1 = w + __ffs(bad) - 2;
@@ -970,36 +996,35 @@ __global__ __launch_bounds__(256) void k_chunk_groups(ChunkArgs a) {
 // cut.  Such a chunk spans a compact block of cells: the tile's width in x,
 // a few rows in y, one plane in z.  Without sorting information the tile is
 // one unit cut into runs of ch particles.  Called by the CG lanes of the
-// unit; returns its number of chunks.
-template <bool WRITE>
-PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, i64 pos, int lane) {
+// unit; returns its number of chunks, of which those from `out` on, `room`
+// at most, are stored.  `rs` is LDS for the starts of ROWS rows.
+constexpr int ROWS = 96;
+
+PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, Chunk *out, i64 room, int lane, i64 *rs) {
   int nch = 0;
+  const int nx3 = a.n3[3 * t], ny3 = a.n3[3 * t + 1], nz3 = a.n3[3 * t + 2];
   auto emit = [&](int64_t b, int64_t n, int zz, int zz1, int y0, int y1) {
-    if (WRITE && lane == 0) {
-      if (pos + nch >= a.maxchunks) {
-        count_bad(a.bad);  // cannot happen: see the bound
-      } else {
-        Chunk c;
-        c.begin = b;
-        c.n = (int)n;
-        c.tile = t;
-        c.z = zz;
-        c.z1 = zz1;
-        c.y0 = y0;
-        c.y1 = y1;
-        c.s = 0;
-        c.pad = 0;
-        if (a.sk4 > 0 && zz >= 0) {
-          // lanes a few sorting cells apart: sk4 / 4 times the particles per
-          // cell, to the nearest power of two (on a log scale)
-          const i64 cells = (i64)a.n3[3 * t] * (y1 - y0 + 1) * (zz1 - zz + 1);
-          const double want = (double)a.sk4 * (double)n / (4.0 * (double)cells);
-          int p2 = 1;
-          while (p2 < (1 << 20) && want > 1.4142135623730951 * p2) p2 <<= 1;
-          c.s = p2;
-        }
-        a.out[pos + nch] = c;
+    if (lane == 0 && nch < room) {
+      Chunk c;
+      c.begin = b;
+      c.n = (int)n;
+      c.tile = t;
+      c.z = zz;
+      c.z1 = zz1;
+      c.y0 = y0;
+      c.y1 = y1;
+      c.s = 0;
+      c.pad = 0;
+      if (a.sk4 > 0 && zz >= 0) {
+        // lanes a few sorting cells apart: sk4 / 4 times the particles per
+        // cell, to the nearest power of two (on a log scale)
+        const i64 cells = (i64)nx3 * (y1 - y0 + 1) * (zz1 - zz + 1);
+        const double want = (double)a.sk4 * (double)n, unit = 4.0 * 1.4142135623730951 * (double)cells;
+        int p2 = 1;
+        while (p2 < (1 << 20) && want > unit * p2) p2 <<= 1;
+        c.s = p2;
       }
+      out[nch] = c;
     }
     nch++;
   };
@@ -1010,7 +1035,6 @@ PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, i64 pos, int lane) {
     for (int64_t b = 0; b < np; b += a.ch) emit(off + b, min((int64_t)a.ch, np - b), -1, -1, 0, 0);
     return nch;
   }
-  const int nx3 = a.n3[3 * t], ny3 = a.n3[3 * t + 1], nz3 = a.n3[3 * t + 2];
   if (z >= nz3) return 0;
   const int g = a.group[(i64)t * a.nzmax + z];
   const int64_t base = a.bin_base[t] + (int64_t)z * ny3 * nx3;
@@ -1020,56 +1044,69 @@ PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, i64 pos, int lane) {
     return nch;
   }
   if (g != GROUP_ROWS) return 0;
-  auto rows = [&](int y) {  // particles of row y
-    const int64_t r = base + (int64_t)y * nx3;
-    return y < ny3 ? a.bin_start[r + nx3] - a.bin_start[r] : 0;
+  // start of row y (y = ny3: the end of the plane)
+  for (int y = lane; y <= min(ny3, ROWS - 1); y += CG) rs[y] = a.bin_start[base + (int64_t)y * nx3];
+  auto start = [&](int y) { return y < ROWS ? rs[y] : (i64)a.bin_start[base + (int64_t)y * nx3]; };
+  int fe[3], je[3];
+  AxisFit(a, t, 0).extent(a.bg, 0, 0, nx3 - 1, fe[0], je[0]);
+  AxisFit(a, t, 2).extent(a.bg, 2, z, z, fe[2], je[2]);
+  const AxisFit ay(a, t, 1);
+  auto fit = [&](int y0, int y1) {
+    ay.extent(a.bg, 1, y0, y1, fe[1], je[1]);
+    return blocks_fit(a, fe, je);
   };
-  int y = 0;  // next row to look at
-  int64_t cb = 0, cnt = 0;
-  int y0 = 0, ylast = 0;  // first and last row of the open chunk
+  int y = 0;
   while (y < ny3) {
-    const int64_t rn = rows(y + lane);
-    if (cnt == 0) {  // open a chunk at the first row with particles
-      const unsigned some = cg_ballot(rn > 0);
-      if (!some) {
-        y += CG;
-        continue;
-      }
-      const int f = __ffs(some) - 1;
-      y0 = ylast = y + f;
-      cnt = __shfl(rn, f, CG);
-      cb = a.bin_start[base + (int64_t)y0 * nx3];
-      while (cnt > a.ch) {  // a row denser than a chunk: cut it
-        emit(cb, a.ch, z, z, y0, y0);
-        cb += a.ch;
-        cnt -= a.ch;
-      }
-      y = y0 + 1;
+    // rows y .. y + CG - 1: the first with particles opens a chunk
+    const int yl = min(y + lane, ny3 - 1);
+    i64 row0 = start(yl), row1 = start(yl + 1);
+    const unsigned some = cg_ballot(y + lane < ny3 && row1 > row0);
+    if (!some) {
+      y += CG;
       continue;
     }
-    // the rows from y on that still belong to the open chunk
-    const int64_t sum = cnt + cg_scan(rn, lane);
-    const bool end = rn > 0 && (sum > a.ch || !blocks_fit(a, t, z, z, y0, y + lane));
-    const unsigned ends = cg_ballot(end);
-    const int take = ends ? __ffs(ends) - 1 : CG;
-    const unsigned used = cg_ballot(rn > 0) & ((1u << take) - 1u);
-    if (used) ylast = y + 31 - __clz(used);
-    if (take) cnt = __shfl(sum, take - 1, CG);
-    y += take;
-    if (ends) {
-      emit(cb, cnt, z, z, y0, ylast);
-      cnt = 0;
+    const int f = __ffs(some) - 1, y0 = y + f;
+    int64_t cb = __shfl(row0, f, CG);
+    const int64_t c1 = __shfl(row1, f, CG);
+    while (c1 - cb > a.ch) {  // a row denser than a chunk: cut it
+      emit(cb, a.ch, z, z, y0, y0);
+      cb += a.ch;
     }
+    // the first row after y0 that does not belong to it closes it
+    int64_t last = c1;  // end of its particles
+    int ylast = y0, w = y;
+    for (;;) {
+      const bool row = w + lane > y0 && w + lane < ny3 && row1 > row0;
+      const bool end = row && (row1 - cb > a.ch || !fit(y0, w + lane));
+      const unsigned ends = cg_ballot(end);
+      const int take = ends ? __ffs(ends) - 1 : CG;
+      const unsigned used = cg_ballot(row) & ((1u << take) - 1u);
+      if (used) {
+        const int l = 31 - __clz(used);
+        ylast = w + l;
+        last = __shfl(row1, l, CG);
+      }
+      w += take;
+      if (ends || w >= ny3) break;
+      const int wl = min(w + lane, ny3 - 1);
+      row0 = start(wl);
+      row1 = start(wl + 1);
+    }
+    emit(cb, last - cb, z, z, y0, ylast);
+    y = w;
   }
-  if (cnt > 0) emit(cb, cnt, z, z, y0, ylast);
   return nch;
 }
 
+constexpr int STAGE = CG;  // chunks per unit that k_chunk_count stores
+
 __global__ __launch_bounds__(256) void k_chunk_count(ChunkArgs a) {
+  __shared__ i64 rs[256 / CG][ROWS];
   const i64 u = ((i64)blockIdx.x * blockDim.x + threadIdx.x) / CG;
   const int lane = threadIdx.x % CG;
   if (u >= (i64)a.ntiles * a.nzmax) return;
-  const int n = walk_unit<false>(a, (int)(u / a.nzmax), (int)(u % a.nzmax), 0, lane);
+  const int n = walk_unit(a, (int)(u / a.nzmax), (int)(u % a.nzmax), a.stage + u * STAGE,
+                          a.stage ? STAGE : 0, lane, rs[threadIdx.x / CG]);
   if (lane == 0) a.count[u] = n;
 }
 
@@ -1112,6 +1149,7 @@ constexpr i64 CHUNK_SELF_SCAN = 16384;
 __global__ __launch_bounds__(256) void k_chunk_write(ChunkArgs a) {
   constexpr int PER = 256 / CG;  // units per block
   __shared__ int before[4];
+  __shared__ i64 rs[PER][ROWS];
   const i64 nu = (i64)a.ntiles * a.nzmax;
   const int lane = threadIdx.x % CG, k = threadIdx.x / CG;
   const i64 u0 = (i64)blockIdx.x * PER, u = u0 + k;
@@ -1130,7 +1168,16 @@ __global__ __launch_bounds__(256) void k_chunk_write(ChunkArgs a) {
     for (i64 i = u0; i < min(u, nu); i++) pos += a.count[i];
     tot = pos + (u < nu ? a.count[u] : 0);
   }
-  if (u < nu) walk_unit<true>(a, (int)(u / a.nzmax), (int)(u % a.nzmax), pos, lane);
+  if (u < nu) {
+    const int n = a.count[u];
+    const i64 room = min(a.maxchunks - pos, (i64)n);
+    if (room < n && lane == 0) atomicAdd(a.bad, (unsigned long long)(n - max(room, (i64)0)));  // cannot happen: see the bound
+    if (a.stage && n <= STAGE) {
+      if (lane < room) a.out[pos + lane] = a.stage[u * STAGE + lane];
+    } else {
+      walk_unit(a, (int)(u / a.nzmax), (int)(u % a.nzmax), a.out + pos, room, lane, rs[k]);
+    }
+  }
   if (u == nu - 1 && lane == 0) {
     *a.nchunks = (int)min(tot, a.maxchunks);
     *a.queue = 0;
@@ -1388,6 +1435,11 @@ static int build_chunks(const TileTable *tt, const pxrhip_species *sp, const Box
   int *ctl = (int *)scratch(10, 4 * sizeof(int));
   int2 *ovf = (int2 *)scratch(14, sizeof(int2) * (size_t)maxchunks);
   if (!cnt || !grp || !cstart || !bsum || !chunks || !ctl || !ovf) return set_error(PXRHIP_ERR_HIP, "scratch allocation failed");
+  // few units, as those of one large tile, are each walked for long: the
+  // chunks found while counting are kept and need no second walk
+  Chunk *stage = nullptr;
+  if (nunits <= CHUNK_SELF_SCAN)
+    stage = (Chunk *)scratch(18, sizeof(Chunk) * (size_t)(nunits * STAGE));
   ChunkArgs ca;
   ca.ntiles = tt->ntiles;
   ca.ch = ch;
@@ -1404,6 +1456,7 @@ static int build_chunks(const TileTable *tt, const pxrhip_species *sp, const Box
   ca.bin_base = tt->bin_base;
   ca.count = cnt;
   ca.group = grp;
+  ca.stage = stage;
   ca.start = cstart;
   ca.out = chunks;
   ca.nchunks = ctl;
