@@ -46,6 +46,10 @@ __global__ __launch_bounds__(256) void k_gather(LeafGatherArgs a) {
   a.bz[ip] += out[5];
 }
 
+// Threads per block of the deposition kernels: a set too small for blocks of
+// four waves on every CU is dealt out in single waves.
+static unsigned dep_block(i64 np) { return np < (i64)256 * rt().num_cus ? 64 : 256; }
+
 static void launch_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st) {
   const dim3 grd(grid1d(a.np, 256)), blk(256);
   switch (order * 2 + (lower ? 1 : 0)) {
@@ -222,15 +226,17 @@ __global__ __launch_bounds__(256) void k_set_gamma(i64 np, const double *ux, con
 // current deposition (global atomics)
 // ---------------------------------------------------------------------------
 
-// Particles of the deposition kernels: a block takes 256 * DEP_S of them
-// and the lanes of a wave take particles 4 * DEP_S apart (each lane DEP_S
-// consecutive ones in turn).  In cell-sorted input, as the tiled species
-// hold it, the lanes of one atomic instruction then sit in different cells
-// instead of queueing on the same nodes.
-#define DEP_S 4
-PXR_DEV i64 dep_particle(int k) {
-  const int t = (int)threadIdx.x;
-  return (i64)blockIdx.x * (256 * DEP_S) + (t & 63) * (4 * DEP_S) + (t >> 6) * DEP_S + k;
+// Particles of the deposition kernels, one a thread: the lanes of a wave take
+// particles DEP_S apart out of 64 * DEP_S, which DEP_S waves share.  In
+// cell-sorted input, as the tiled species hold it, the lanes of one atomic
+// instruction then sit in different cells instead of queueing on the same
+// nodes.  The adds are done by the L2, a particle's one after the other, so a
+// small set wants all its particles in flight: 4000 order-1 particles took
+// 45 us with four particles in turn a thread, 9 us so.
+#define DEP_S 16
+PXR_DEV i64 dep_particle() {
+  const i64 w = ((i64)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  return w / DEP_S * (64 * DEP_S) + (threadIdx.x & 63) * DEP_S + w % DEP_S;
 }
 
 template <int N>
@@ -251,10 +257,8 @@ PXR_DEV void esirkepov_one(const DepoArgs &a, i64 ip) {
 
 template <int N>
 __global__ __launch_bounds__(256) void k_esirkepov(DepoArgs a) {
-  for (int k = 0; k < DEP_S; k++) {
-    const i64 ip = dep_particle(k);
-    if (ip < a.np) esirkepov_one<N>(a, ip);
-  }
+  const i64 ip = dep_particle();
+  if (ip < a.np) esirkepov_one<N>(a, ip);
 }
 
 template <int N>
@@ -276,10 +280,8 @@ PXR_DEV void direct_one(const DepoArgs &a, i64 ip) {
 
 template <int N>
 __global__ __launch_bounds__(256) void k_direct(DepoArgs a) {
-  for (int k = 0; k < DEP_S; k++) {
-    const i64 ip = dep_particle(k);
-    if (ip < a.np) direct_one<N>(a, ip);
-  }
+  const i64 ip = dep_particle();
+  if (ip < a.np) direct_one<N>(a, ip);
 }
 
 // charge density, pxr_depose_rho_n (charge_deposition_3d.F90:2081-2228):
@@ -316,10 +318,8 @@ PXR_DEV void rho_one(const RhoArgs &a, i64 ip) {
 
 template <int N>
 __global__ __launch_bounds__(256) void k_rho(RhoArgs a) {
-  for (int k = 0; k < DEP_S; k++) {
-    const i64 ip = dep_particle(k);
-    if (ip < a.np) rho_one<N>(a, ip);
-  }
+  const i64 ip = dep_particle();
+  if (ip < a.np) rho_one<N>(a, ip);
 }
 
 // ---------------------------------------------------------------------------
@@ -1078,7 +1078,7 @@ int pxrhip_depose_jxjyjz(double *jx, double *jy, double *jz, int64_t np, const d
   a.g = mkgeom(nx, ny, nz, nxguard, nyguard, nzguard);
   a.jx = jx; a.jy = jy; a.jz = jz;
   a.bad = rt().d_bad;
-  dim3 grd(grid1d(np, 256 * DEP_S)), blk(256);
+  const dim3 blk(dep_block(np)), grd(grid1d(np, 64 * DEP_S) * (64 * DEP_S / blk.x));
   hipStream_t st = rt().stream;
   const bool direct = current_depo_algo >= 2;  // depose_jxjyjz_generic CASE(2), CASE(3)
   bool done = false;
@@ -1144,7 +1144,7 @@ int pxrhip_depose_rho_n(double *rho, int64_t np, const double *xp, const double 
   a.g = mkgeom(nx, ny, nz, nxguard, nyguard, nzguard);
   a.rho = rho;
   a.bad = rt().d_bad;
-  dim3 grd(grid1d(np, 256 * DEP_S)), blk(256);
+  const dim3 blk(dep_block(np)), grd(grid1d(np, 64 * DEP_S) * (64 * DEP_S / blk.x));
   hipStream_t st = rt().stream;
   bool done = false;
   if (leaf_binned_rho_pays(np, a.g)) {
