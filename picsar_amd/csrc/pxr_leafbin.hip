@@ -464,14 +464,14 @@ static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st
 }
 
 constexpr int LB_EDGE = 8;  // nodes per block edge
-// Particles from which a gather asks for their order, at order 2 and 3.  The
-// question costs a call in cell order 4 to 8 us, so it has to be a small part
-// of the call: order 3, a million on 64^3 cells, 152 -> 156 us in cell order
-// and 615 -> 293 in random order; order 2, two million, 154 -> 160 and
-// 900 -> 371 (a million: 101 us in cell order).  At order 1 a particle's
-// eight-node reads cost no more than ordering it (a million 201 us plain, 395
-// binned).
-constexpr i64 GATHER_BIN_MIN2 = 3 << 19, GATHER_BIN_MIN3 = 3 << 18;
+// Particles from which a gather asks for their order.  The question costs a
+// call in cell order 4 to 8 us, so it has to be a small part of the call.  A
+// million on 64^3 cells: order 3 151 -> 155 us in cell order and 618 -> 293 in
+// random order, order 2 106 -> 109 and 428 -> 227 (600000 on 48^3, order 2:
+// 180 -> 187).  At order 1 a particle's eight-node reads are as fast as
+// ordering it until the fields leave the L2: two million on 64^3 360 -> 347
+// us, four million on 128^3 1020 -> 741 (153 -> 160 in cell order).
+constexpr i64 GATHER_BIN_MIN1 = 3 << 20, GATHER_BIN_MIN = 3 << 18;
 constexpr int GATHER_CHUNK = 1024;  // particles of a gather's work item
 
 // persistent workgroups: as many as the CUs hold at this LDS size, or one
@@ -509,8 +509,8 @@ LeafGatherArgs LeafGatherArgs::part(i64 first, i64 n) const {
 }
 
 bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order) {
-  return order >= 2 && rt().checks && pays(a.np, a.g, LB_EDGE) &&
-         a.np >= (order == 3 ? GATHER_BIN_MIN3 : GATHER_BIN_MIN2);
+  return rt().checks && pays(a.np, a.g, LB_EDGE) &&
+         a.np >= (order == 1 ? GATHER_BIN_MIN1 : GATHER_BIN_MIN);
 }
 
 int leaf_probe_start(LeafGatherArgs &a, hipStream_t st) {
@@ -551,7 +551,9 @@ int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream
       return PXRHIP_OK;
     const dim3 grd(lb_grid(maxitems, lds)), blk(512);
     switch (order * 2 + (lower ? 1 : 0)) {
-      case 4: LB_LAUNCH((k_lb_gather<2, 2, LB_EDGE>), ga); break;
+      case 2: LB_LAUNCH((k_lb_gather<1, 1, LB_EDGE>), ga); break;
+    case 3: LB_LAUNCH((k_lb_gather<1, 0, LB_EDGE>), ga); break;
+    case 4: LB_LAUNCH((k_lb_gather<2, 2, LB_EDGE>), ga); break;
       case 5: LB_LAUNCH((k_lb_gather<2, 1, LB_EDGE>), ga); break;
       case 6: LB_LAUNCH((k_lb_gather<3, 3, LB_EDGE>), ga); break;
       default: LB_LAUNCH((k_lb_gather<3, 2, LB_EDGE>), ga); break;
