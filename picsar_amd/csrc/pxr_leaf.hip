@@ -893,12 +893,13 @@ int pxrhip_geteb3d_energy_conserving(
   a.bad = rt().d_bad;
   const bool lo = l_lower_order_in_v != 0;
   hipStream_t st = rt().stream;
-  const bool probe = leaf_binned_gather_may_pay(a, (int)nox);
-  if (probe && (r = leaf_probe_start(a, st))) return r;
+  const bool ask = leaf_binned_gather_may_pay(a, (int)nox);
+  LeafProbe probe;
+  if (ask && (r = leaf_probe_start(a, st, probe))) return r;
   launch_gather(a, (int)nox, lo, st);
-  if (probe) {
+  if (ask) {
     bool scattered;
-    if ((r = leaf_probe_read(scattered))) return r;
+    if ((r = leaf_probe_read(probe, scattered))) return r;
     a.skip = nullptr;
     i64 done = np;
     if (scattered && (r = leaf_binned_gather(a, (int)nox, lo, st, done))) return r;

@@ -76,8 +76,15 @@ bool leaf_binned_rho_pays(i64 np, const GridGeom &g);
 // leaf_probe_read waits for the answer.  leaf_binned_gather returns how many
 // particles are done: all of them, or fewer where it ran out of memory.
 bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order);
-int leaf_probe_start(LeafGatherArgs &a, hipStream_t st);
-int leaf_probe_read(bool &scattered);
+struct LeafProbe {
+  hipEvent_t done = nullptr;
+  unsigned long long *host = nullptr;
+  ~LeafProbe() {
+    if (done) (void)hipEventDestroy(done);
+  }
+};
+int leaf_probe_start(LeafGatherArgs &a, hipStream_t st, LeafProbe &probe);
+int leaf_probe_read(LeafProbe &probe, bool &scattered);
 int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st, i64 &done);
 
 }  // namespace pxr

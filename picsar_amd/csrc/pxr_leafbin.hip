@@ -22,6 +22,7 @@
 // The gather of the fields (geteb3d_energy_conserving) uses the same order
 // for a large set whose particles are in none.
 #include <algorithm>
+#include <mutex>
 
 #include "pxr_leafbin.h"
 #include "pxr_radix.h"
@@ -410,7 +411,8 @@ __global__ __launch_bounds__(256) void k_lb_gather_add(LeafGatherArgs a, const d
 // set: it is in no order if most particles have another block than their
 // predecessor (a set in cell order crosses blocks a few times a run).
 template <int B>
-__global__ __launch_bounds__(1024) void k_lb_probe(LbPos a, BinGeom bg, int *out, int *host_out) {
+__global__ __launch_bounds__(1024) void k_lb_probe(LbPos a, BinGeom bg, int *out,
+                                                  unsigned long long *host_out) {
   __shared__ int s[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int b[4], n = 0;
@@ -427,7 +429,9 @@ __global__ __launch_bounds__(1024) void k_lb_probe(LbPos a, BinGeom bg, int *out
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 16; w++) n += s[w];
-    *out = *host_out = n > 64 * 24;
+    const int scattered = n > 64 * 24;
+    *out = scattered;
+    *host_out = scattered;
   }
 }
 
@@ -462,6 +466,10 @@ static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st
                      nitems);
   return true;
 }
+
+// The ordering and the kernels behind it share scratch: a call launches them
+// all before another thread's (on the one stream they then run in turn).
+static std::mutex g_order;
 
 constexpr int LB_EDGE = 8;  // nodes per block edge
 // Particles from which a gather asks for their order.  The question costs a
@@ -513,19 +521,21 @@ bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order) {
          a.np >= (order == 1 ? GATHER_BIN_MIN1 : GATHER_BIN_MIN);
 }
 
-int leaf_probe_start(LeafGatherArgs &a, hipStream_t st) {
-  int *out = (int *)(rt().d_bad + 2);
+int leaf_probe_start(LeafGatherArgs &a, hipStream_t st, LeafProbe &probe) {
+  PXR_HIP(hipEventCreateWithFlags(&probe.done, hipEventDisableTiming));
+  probe.host = report_slot();
+  int *out = (int *)(rt().d_bad + 2 + (probe.host - rt().h_report));
   hipLaunchKernelGGL(k_lb_probe<LB_EDGE>, dim3(1), dim3(1024), 0, st, gather_pos(a, nullptr),
-                     make_bin_geom(a.g, LB_EDGE), out, rt().h_probe);
+                     make_bin_geom(a.g, LB_EDGE), out, probe.host);
   PXR_LAUNCHED();
-  PXR_HIP(hipEventRecord(rt().probe_done, st));
+  PXR_HIP(hipEventRecord(probe.done, st));
   a.skip = out;
   return PXRHIP_OK;
 }
 
-int leaf_probe_read(bool &scattered) {
-  PXR_HIP(hipEventSynchronize(rt().probe_done));
-  scattered = *(volatile int *)rt().h_probe != 0;
+int leaf_probe_read(LeafProbe &probe, bool &scattered) {
+  PXR_HIP(hipEventSynchronize(probe.done));
+  scattered = *(volatile unsigned long long *)probe.host != 0;
   return PXRHIP_OK;
 }
 
@@ -536,6 +546,7 @@ int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream
   const i64 nparts = (a.np + most - 1) / most, size = (a.np + nparts - 1) / nparts;
   const int L = LB_EDGE + (order == 3 && !lower ? 4 : 3);
   const size_t lds = sizeof(double) * 6 * (size_t)(L * L * L);
+  std::lock_guard<std::mutex> lock(g_order);
   done = 0;
   LbGather ga;
   if (!(ga.rec = (double *)scratch(30, 6 * sizeof(double) * (size_t)size))) return PXRHIP_OK;
@@ -570,6 +581,7 @@ bool leaf_binned_current_pays(i64 np, const GridGeom &g) { return pays(np, g, LB
 bool leaf_binned_rho_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
 
 int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, bool &done) {
+  std::lock_guard<std::mutex> lock(g_order);
   done = false;
   BinGeom bg;
   int *perm, *nitems;
@@ -593,6 +605,7 @@ int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, bool &done)
 }
 
 int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, bool &done) {
+  std::lock_guard<std::mutex> lock(g_order);
   done = false;
   BinGeom bg;
   int *perm, *nitems;
@@ -616,6 +629,7 @@ int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, bool &do
 }
 
 int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done) {
+  std::lock_guard<std::mutex> lock(g_order);
   done = false;
   constexpr int E = LB_EDGE;
   BinGeom bg;

@@ -9,16 +9,17 @@
 
 namespace pxr {
 
+constexpr int REPORT_SLOTS = 256;
+
 struct Runtime {
   int device = -1;
   hipStream_t stream = nullptr;
   bool own_stream = false;  // created by pxrhip_init
   bool capturing = false;   // a graph capture of the stream is open
   bool checks = true;
-  // device counter of skipped particles; [2] holds the answer of k_lb_probe
+  // device counter of skipped particles; from [2] on a word per report slot
   unsigned long long *d_bad = nullptr;
-  int *h_probe = nullptr;               // pinned host int that a kernel reports through
-  hipEvent_t probe_done = nullptr;
+  unsigned long long *h_report = nullptr;  // pinned host memory, see report_slot
   int num_cus = 256;
   // leaf deposition summed in LDS blocks (pxr_leafbin.hip) from this many
   // particles on (0: never), work items of at most leaf_bin_chunk particles
@@ -37,6 +38,10 @@ int ensure_init();
 // if there is no memory for it (with the runtime's error state cleared, so
 // that a caller that has a form without scratch can launch that)
 void *scratch(int slot, size_t bytes);
+// A word of pinned host memory for a kernel to report through: the caller's
+// own until as many later calls have asked for one (calls of other threads
+// that wait at the same time have theirs).
+unsigned long long *report_slot();
 // read the bad-particle counter (synchronises the stream), reset it to 0
 int take_bad(unsigned long long *n);
 

@@ -3,6 +3,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <atomic>
 #include <vector>
 
 #include "pxr_runtime.h"
@@ -57,12 +58,27 @@ void *scratch(int slot, size_t bytes) {
   return s.p;
 }
 
+unsigned long long *report_slot() {
+  static std::atomic<unsigned> next{0};
+  return g_rt.h_report + next++ % REPORT_SLOTS;
+}
+
+// the counter of skipped particles into host memory, and cleared
+__global__ void k_take_bad(unsigned long long *bad, unsigned long long *host) {
+  *host = *bad;
+  *bad = 0ull;
+}
+
+// Every checked call ends with this: one small launch and one wait.  (A copy
+// into pageable memory goes through a staging buffer of the runtime and
+// waits for itself, 8 us more.)
 int take_bad(unsigned long long *n) {
-  unsigned long long h = 0;
-  PXR_HIP(hipMemcpyAsync(&h, g_rt.d_bad, sizeof(h), hipMemcpyDeviceToHost, g_rt.stream));
+  volatile unsigned long long *h = report_slot();
+  hipLaunchKernelGGL(k_take_bad, dim3(1), dim3(1), 0, g_rt.stream, g_rt.d_bad,
+                     (unsigned long long *)h);
+  PXR_LAUNCHED();
   PXR_HIP(hipStreamSynchronize(g_rt.stream));
-  if (h) PXR_HIP(hipMemsetAsync(g_rt.d_bad, 0, sizeof(h), g_rt.stream));
-  *n = h;
+  *n = *h;
   return PXRHIP_OK;
 }
 
@@ -90,11 +106,11 @@ int pxrhip_init(int device) {
     g_rt.own_stream = true;
   }
   if (!g_rt.d_bad) {
-    PXR_HIP(hipMalloc(&g_rt.d_bad, 3 * sizeof(unsigned long long)));
-    PXR_HIP(hipMemset(g_rt.d_bad, 0, 3 * sizeof(unsigned long long)));
+    PXR_HIP(hipMalloc(&g_rt.d_bad, (2 + REPORT_SLOTS) * sizeof(unsigned long long)));
+    PXR_HIP(hipMemset(g_rt.d_bad, 0, (2 + REPORT_SLOTS) * sizeof(unsigned long long)));
   }
-  if (!g_rt.h_probe) PXR_HIP(hipHostMalloc(&g_rt.h_probe, sizeof(int), 0));
-  if (!g_rt.probe_done) PXR_HIP(hipEventCreateWithFlags(&g_rt.probe_done, hipEventDisableTiming));
+  if (!g_rt.h_report)
+    PXR_HIP(hipHostMalloc(&g_rt.h_report, REPORT_SLOTS * sizeof(unsigned long long), 0));
   g_rt.device = dev;
   return PXRHIP_OK;
 }
@@ -109,10 +125,8 @@ int pxrhip_finalize(void) {
   }
   if (g_rt.d_bad) hipFree(g_rt.d_bad);
   g_rt.d_bad = nullptr;
-  if (g_rt.h_probe) hipHostFree(g_rt.h_probe);
-  g_rt.h_probe = nullptr;
-  if (g_rt.probe_done) hipEventDestroy(g_rt.probe_done);
-  g_rt.probe_done = nullptr;
+  if (g_rt.h_report) hipHostFree(g_rt.h_report);
+  g_rt.h_report = nullptr;
   if (g_rt.own_stream && g_rt.stream) hipStreamDestroy(g_rt.stream);
   g_rt.stream = nullptr;
   g_rt.own_stream = false;

@@ -90,3 +90,41 @@ def test_sets_in_cell_order(dev, swap):
     b, _ = gather(dev, picsar, P, FD, out, 3, True, 1)
     for p, q in zip(a, b):
         np.testing.assert_array_equal(p, q)
+
+
+def test_calls_of_several_threads(dev):
+    """The library's stream and scratch are shared: calls of several threads
+    give what they give one after the other."""
+    import threading
+    from picsar_amd.picsarpy import picsar
+    rng = np.random.default_rng(11)
+    n = 800000
+    FD = [TG(dev, rng.standard_normal(SHAPE)) for _ in range(6)]
+    sets = []
+    for k in range(3):
+        x, y, z = particles(rng, n, margin=1.0)
+        if k == 1:
+            o = np.lexsort((np.floor(x), np.floor(y), np.floor(z)))
+            x, y, z = x[o], y[o], z[o]
+        sets.append([T(dev, a) for a in (x, y, z)])
+    outs = [[[T(dev, np.zeros(n)) for _ in range(6)] for _ in range(4)] for _ in sets]
+
+    def run(k, r):
+        picsar.geteb3d_energy_conserving(n, *sets[k], *outs[k][r], 0.0, 0.0, 0.0, 1.0, 1.0, 1.0,
+                                         NX, NY, NZ, NG, NG, NG, 3, 3, 3, *FD, False, True)
+
+    was, picsar.l_nodalgrid = picsar.l_nodalgrid, False
+    try:
+        for k in range(3):
+            run(k, 0)
+        th = [threading.Thread(target=lambda k=k: [run(k, r) for r in (1, 2, 3)]) for k in range(3)]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+    finally:
+        picsar.l_nodalgrid = was
+    for k in range(3):
+        for r in (1, 2, 3):
+            for a, b in zip(outs[k][0], outs[k][r]):
+                np.testing.assert_array_equal(H(a), H(b))
