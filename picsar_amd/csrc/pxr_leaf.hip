@@ -1485,15 +1485,12 @@ static int bin_sort_run(int64_t np2, double *const *arr, const SortGeom &s, cons
   else sort_move<1>(np2, arr, tmp, idx[0], bad_ctr, st);
   PXR_LAUNCHED();
   unsigned long long bad = 0;
-  PXR_HIP(hipMemcpyAsync(&bad, bad_ctr, sizeof(bad), hipMemcpyDeviceToHost, st));
-  PXR_HIP(hipStreamSynchronize(st));
-  if (bad) {
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, st, bad_ctr, 1, 0ull);
-    PXR_LAUNCHED();
+  int r = take_counter(bad_ctr, &bad);
+  if (r) return r;
+  if (bad)
     return set_error(PXRHIP_ERR_BOUNDS,
                      "particle_bin_sorting: %llu particle(s) have a cell key outside [1,%lld]; "
                      "nothing was moved", bad, (long long)s.nbins);
-  }
   return PXRHIP_OK;
 }
 

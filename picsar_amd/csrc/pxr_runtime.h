@@ -44,6 +44,8 @@ void *scratch(int slot, size_t bytes);
 unsigned long long *report_slot();
 // read the bad-particle counter (synchronises the stream), reset it to 0
 int take_bad(unsigned long long *n);
+// the same for any device counter
+int take_counter(unsigned long long *ctr, unsigned long long *n);
 
 inline unsigned grid1d(int64_t n, int block) {
   int64_t b = (n + block - 1) / block;

@@ -63,24 +63,26 @@ unsigned long long *report_slot() {
   return g_rt.h_report + next++ % REPORT_SLOTS;
 }
 
-// the counter of skipped particles into host memory, and cleared
-__global__ void k_take_bad(unsigned long long *bad, unsigned long long *host) {
-  *host = *bad;
-  *bad = 0ull;
+// a device counter into host memory, and cleared
+__global__ void k_take_counter(unsigned long long *ctr, unsigned long long *host) {
+  *host = *ctr;
+  *ctr = 0ull;
 }
 
 // Every checked call ends with this: one small launch and one wait.  (A copy
 // into pageable memory goes through a staging buffer of the runtime and
 // waits for itself, 8 us more.)
-int take_bad(unsigned long long *n) {
+int take_counter(unsigned long long *ctr, unsigned long long *n) {
   volatile unsigned long long *h = report_slot();
-  hipLaunchKernelGGL(k_take_bad, dim3(1), dim3(1), 0, g_rt.stream, g_rt.d_bad,
+  hipLaunchKernelGGL(k_take_counter, dim3(1), dim3(1), 0, g_rt.stream, ctr,
                      (unsigned long long *)h);
   PXR_LAUNCHED();
   PXR_HIP(hipStreamSynchronize(g_rt.stream));
   *n = *h;
   return PXRHIP_OK;
 }
+
+int take_bad(unsigned long long *n) { return take_counter(g_rt.d_bad, n); }
 
 }  // namespace pxr
 
