@@ -1079,24 +1079,26 @@ int pxrhip_depose_jxjyjz(double *jx, double *jy, double *jz, int64_t np, const d
   a.g = mkgeom(nx, ny, nz, nxguard, nyguard, nzguard);
   a.jx = jx; a.jy = jy; a.jz = jz;
   a.bad = rt().d_bad;
-  const dim3 blk(dep_block(np)), grd(grid1d(np, 64 * DEP_S) * (64 * DEP_S / blk.x));
   hipStream_t st = rt().stream;
   const bool direct = current_depo_algo >= 2;  // depose_jxjyjz_generic CASE(2), CASE(3)
-  bool done = false;
+  i64 done = 0;
   if (leaf_binned_current_pays(np, a.g)) {
     r = direct ? leaf_binned_direct(a, (int)nox, st, done)
                : leaf_binned_esirkepov(a, (int)nox, st, done);
     if (r) return r;
   }
-  if (done) {
-  } else if (direct) {
-    if (nox == 1) hipLaunchKernelGGL(k_direct<1>, grd, blk, 0, st, a);
-    else if (nox == 2) hipLaunchKernelGGL(k_direct<2>, grd, blk, 0, st, a);
-    else hipLaunchKernelGGL(k_direct<3>, grd, blk, 0, st, a);
-  } else {
-    if (nox == 1) hipLaunchKernelGGL(k_esirkepov<1>, grd, blk, 0, st, a);
-    else if (nox == 2) hipLaunchKernelGGL(k_esirkepov<2>, grd, blk, 0, st, a);
-    else hipLaunchKernelGGL(k_esirkepov<3>, grd, blk, 0, st, a);
+  if (done < np) {  // all of them, or those there was no memory to order
+    const DepoArgs p = a.part(done, np - done);
+    const dim3 blk(dep_block(p.np)), grd(grid1d(p.np, 64 * DEP_S) * (64 * DEP_S / blk.x));
+    if (direct) {
+      if (nox == 1) hipLaunchKernelGGL(k_direct<1>, grd, blk, 0, st, p);
+      else if (nox == 2) hipLaunchKernelGGL(k_direct<2>, grd, blk, 0, st, p);
+      else hipLaunchKernelGGL(k_direct<3>, grd, blk, 0, st, p);
+    } else {
+      if (nox == 1) hipLaunchKernelGGL(k_esirkepov<1>, grd, blk, 0, st, p);
+      else if (nox == 2) hipLaunchKernelGGL(k_esirkepov<2>, grd, blk, 0, st, p);
+      else hipLaunchKernelGGL(k_esirkepov<3>, grd, blk, 0, st, p);
+    }
   }
   PXR_LAUNCHED();
   return finish_checked("depose_jxjyjz");

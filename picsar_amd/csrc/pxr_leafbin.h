@@ -17,6 +17,7 @@ struct DepoArgs {
   GridGeom g;
   double *jx, *jy, *jz;
   unsigned long long *bad;
+  DepoArgs part(i64 first, i64 n) const;  // the same call for n particles from `first`
 };
 
 // one call of geteb3d_energy_conserving with one order on all axes
@@ -59,8 +60,8 @@ struct GlobalAcc {
 // and each block's current (or charge) is summed in LDS
 // before one global add per node.  Return PXRHIP_OK, or an error code
 // (scratch memory could not be allocated) before anything is launched.
-int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, bool &done);
-int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, bool &done);
+int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, i64 &done);
+int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, i64 &done);
 int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done);
 // whether a call of np particles on grid g takes the binned form: at least
 // the runtime's leaf_bin_min particles and one per block, and no graph
@@ -79,6 +80,7 @@ bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order);
 struct LeafProbe {
   hipEvent_t done = nullptr;
   unsigned long long *host = nullptr;
+  int *dev = nullptr;
   ~LeafProbe() {
     if (done) (void)hipEventDestroy(done);
   }

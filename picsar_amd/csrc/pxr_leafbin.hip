@@ -58,14 +58,50 @@ template <int B> PXR_DEV int block_axis(double x, int g, int na) {
   return ((int)f + g) / B;
 }
 
+// The eight values of every particle in one record of 64 bytes, written by
+// k_lb_keys and read by the deposition if *use is set (null: never).  In block
+// order a set in no order reads one value of a cache line from each of the
+// eight arrays per particle, which bounds orders 1 and 2: two million particles
+// on 64^3 cells 411 and 423 us (Esirkepov), 281 and 317 with the record (the
+// LDS adds bound order 3: 448 and 475).  A set in cell order shares those
+// lines (177 us at order 1) and would pay for the copy.
+struct DepoRec {
+  double *rec = nullptr;
+  const int *use = nullptr;
+  PXR_DEV bool on() const { return use && *use; }
+};
+
+struct Particle8 {
+  double x, y, z, ux, uy, uz, gi, w;
+};
+
+PXR_DEV Particle8 load8(const DepoArgs &a, const DepoRec &r, bool rec, i64 ip) {
+  Particle8 p;
+  if (rec) {
+    const double2 *q = (const double2 *)(r.rec + 8 * ip);
+    const double2 q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
+    p = Particle8{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
+  } else {
+    p = Particle8{a.xp[ip], a.yp[ip], a.zp[ip], a.ux[ip], a.uy[ip], a.uz[ip], a.gi[ip], a.w[ip]};
+  }
+  return p;
+}
+
 // positions (and, for the mid positions, velocities and h = dt / (2 dx)) of
 // one call
 struct LbPos {
   i64 np;
-  const double *x, *y, *z, *ux, *uy, *uz, *gi;
+  const double *x, *y, *z, *ux, *uy, *uz, *gi, *w;
   double xmin, ymin, zmin, dxi, dyi, dzi, h[3];
   int l4symtry;
   double *rec;  // not null: the normalised positions go to 6-double records too
+  DepoRec packed;
+};
+
+// arguments of the binned deposition: the call's, and the particles' records
+struct LbDepo {
+  DepoArgs c;
+  DepoRec packed;
 };
 
 // arguments of the binned gather: the call's, and the particles' records
@@ -80,13 +116,24 @@ template <int B, bool MID>
 __global__ __launch_bounds__(256) void k_lb_keys(LbPos a, BinGeom bg, int *key) {
   const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
   if (ip >= a.np) return;
-  double x = (a.x[ip] - a.xmin) * a.dxi, y = (a.y[ip] - a.ymin) * a.dyi;
-  double z = (a.z[ip] - a.zmin) * a.dzi;
+  double x = a.x[ip], y = a.y[ip], z = a.z[ip];
+  const bool pack = a.packed.on();
+  double ux = 0.0, uy = 0.0, uz = 0.0, gi = 0.0;
+  if (MID || pack) ux = a.ux[ip], uy = a.uy[ip], uz = a.uz[ip], gi = a.gi[ip];
+  if (pack) {
+    double2 *q = (double2 *)(a.packed.rec + 8 * ip);
+    q[0] = double2{x, y};
+    q[1] = double2{z, ux};
+    q[2] = double2{uy, uz};
+    q[3] = double2{gi, a.w[ip]};
+  }
+  x = (x - a.xmin) * a.dxi;
+  y = (y - a.ymin) * a.dyi;
+  z = (z - a.zmin) * a.dzi;
   if (MID) {
-    const double gi = a.gi[ip];
-    x -= a.h[0] * (a.ux[ip] * gi);
-    y -= a.h[1] * (a.uy[ip] * gi);
-    z -= a.h[2] * (a.uz[ip] * gi);
+    x -= a.h[0] * (ux * gi);
+    y -= a.h[1] * (uy * gi);
+    z -= a.h[2] * (uz * gi);
   } else if (a.l4symtry) {
     x = fabs(x);
     y = fabs(y);
@@ -197,8 +244,10 @@ PXR_DEV int lb_stride(int n) { return (n + (int)blockDim.x - 1) / (int)blockDim.
 // Esirkepov current: the box of an order-N particle lies within
 // [floor(x) - 2, floor(x) + 3] (order 1: [-1, +2]) on each axis.
 template <int N, int B>
-__global__ __launch_bounds__(256) void k_lb_esirkepov(DepoArgs a, BinGeom bg, const int *perm,
+__global__ __launch_bounds__(256) void k_lb_esirkepov(LbDepo d, BinGeom bg, const int *perm,
                                                       const int4 *items, const int *nitems) {
+  const DepoArgs &a = d.c;
+  const bool rec = d.packed.on();
   constexpr int HLO = (N == 1) ? -1 : -2, HHI = (N == 1) ? 2 : 3;
   extern __shared__ double lds[];
   const i64 o = a.g.idx(0, 0, 0);
@@ -214,10 +263,9 @@ __global__ __launch_bounds__(256) void k_lb_esirkepov(DepoArgs a, BinGeom bg, co
   for (int k = 0; k < S; k++) {
     const int p = (int)threadIdx.x * S + k;
     if (p >= n) break;
-    const i64 ip = perm[it.y + p];
+    const Particle8 q = load8(a, d.packed, rec, perm[it.y + p]);
     EsirkepovIn<double> in;
-    esirkepov_prepare<N, double>(in, a.xp[ip], a.yp[ip], a.zp[ip], a.ux[ip], a.uy[ip],
-                                 a.uz[ip], a.gi[ip], a.w[ip], a.ec);
+    esirkepov_prepare<N, double>(in, q.x, q.y, q.z, q.ux, q.uy, q.uz, q.gi, q.w, a.ec);
     int lo[3], hi[3];
     if (!esirkepov_box<N, double>(in, lo, hi) || !a.g.inside(lo[0], lo[1], lo[2]) ||
         !a.g.inside(hi[0], hi[1], hi[2])) {
@@ -240,8 +288,10 @@ __global__ __launch_bounds__(256) void k_lb_esirkepov(DepoArgs a, BinGeom bg, co
 // cells); here they go to LDS and one add per node and block remains
 // (0.12 ms, and 0.06 ms to key and order the particles).
 template <int N, int B>
-__global__ __launch_bounds__(256) void k_lb_direct(DepoArgs a, BinGeom bg, const int *perm,
+__global__ __launch_bounds__(256) void k_lb_direct(LbDepo d, BinGeom bg, const int *perm,
                                                    const int4 *items, const int *nitems) {
+  const DepoArgs &a = d.c;
+  const bool rec = d.packed.on();
   constexpr int HLO = (N == 1) ? -1 : -2, HHI = (N == 1) ? 2 : 3;
   extern __shared__ double lds[];
   const i64 o = a.g.idx(0, 0, 0);
@@ -257,10 +307,9 @@ __global__ __launch_bounds__(256) void k_lb_direct(DepoArgs a, BinGeom bg, const
     for (int k = 0; k < S; k++) {
       const int p = (int)threadIdx.x * S + k;
       if (p >= n) break;
-      const i64 ip = perm[it.y + p];
+      const Particle8 q = load8(a, d.packed, rec, perm[it.y + p]);
       DirectIn<double> in;
-      direct_prepare<N, double>(in, a.xp[ip], a.yp[ip], a.zp[ip], a.ux[ip], a.uy[ip], a.uz[ip],
-                                a.gi[ip], a.w[ip], a.q, a.xmin, a.ymin, a.zmin, a.dt, a.dx, a.dy,
+      direct_prepare<N, double>(in, q.x, q.y, q.z, q.ux, q.uy, q.uz, q.gi, q.w, a.q, a.xmin, a.ymin, a.zmin, a.dt, a.dx, a.dy,
                                 a.dz, a.s);
       int lo[3], hi[3];
       direct_box<N>(in, lo, hi);
@@ -480,6 +529,7 @@ constexpr int LB_EDGE = 8;  // nodes per block edge
 // ordering it until the fields leave the L2: two million on 64^3 360 -> 347
 // us, four million on 128^3 1020 -> 741 (153 -> 160 in cell order).
 constexpr i64 GATHER_BIN_MIN1 = 3 << 20, GATHER_BIN_MIN = 3 << 18;
+constexpr i64 DEPO_REC_MIN = 1 << 19;  // a million random: 236 -> 164 us (Esirkepov, order 1)
 constexpr int GATHER_CHUNK = 1024;  // particles of a gather's work item
 
 // persistent workgroups: as many as the CUs hold at this LDS size, or one
@@ -504,8 +554,15 @@ static bool pays(i64 np, const GridGeom &g, int edge) {
 }
 
 static LbPos gather_pos(const LeafGatherArgs &a, double *rec) {
-  return LbPos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, a.xmin, a.ymin, a.zmin,
-               a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, 0, rec};
+  return LbPos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, nullptr, a.xmin, a.ymin,
+               a.zmin, a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, 0, rec, {}};
+}
+
+DepoArgs DepoArgs::part(i64 first, i64 n) const {
+  DepoArgs p = *this;
+  p.np = n;
+  for (const double **q : {&p.xp, &p.yp, &p.zp, &p.ux, &p.uy, &p.uz, &p.gi, &p.w}) *q += first;
+  return p;
 }
 
 LeafGatherArgs LeafGatherArgs::part(i64 first, i64 n) const {
@@ -521,16 +578,28 @@ bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order) {
          a.np >= (order == 1 ? GATHER_BIN_MIN1 : GATHER_BIN_MIN);
 }
 
+static void launch_probe(const LbPos &pos, const GridGeom &g, hipStream_t st, LeafProbe &probe) {
+  probe.host = report_slot();
+  probe.dev = (int *)(rt().d_bad + 2 + (probe.host - rt().h_report));
+  hipLaunchKernelGGL(k_lb_probe<LB_EDGE>, dim3(1), dim3(1024), 0, st, pos,
+                     make_bin_geom(g, LB_EDGE), probe.dev, probe.host);
+}
+
 int leaf_probe_start(LeafGatherArgs &a, hipStream_t st, LeafProbe &probe) {
   PXR_HIP(hipEventCreateWithFlags(&probe.done, hipEventDisableTiming));
-  probe.host = report_slot();
-  int *out = (int *)(rt().d_bad + 2 + (probe.host - rt().h_report));
-  hipLaunchKernelGGL(k_lb_probe<LB_EDGE>, dim3(1), dim3(1024), 0, st, gather_pos(a, nullptr),
-                     make_bin_geom(a.g, LB_EDGE), out, probe.host);
+  launch_probe(gather_pos(a, nullptr), a.g, st, probe);
   PXR_LAUNCHED();
   PXR_HIP(hipEventRecord(probe.done, st));
-  a.skip = out;
+  a.skip = probe.dev;
   return PXRHIP_OK;
+}
+
+// Particles ordered at a time, in equal parts: 8 million, or 512 per block of
+// the grid, which bounds the records (48 or 64 bytes a particle).
+static i64 part_size(i64 np, const GridGeom &g) {
+  const i64 most = std::max<i64>((i64)1 << 23, 512 * make_bin_geom(g, LB_EDGE).nblocks);
+  const i64 nparts = (np + most - 1) / most;
+  return (np + nparts - 1) / nparts;
 }
 
 int leaf_probe_read(LeafProbe &probe, bool &scattered) {
@@ -541,9 +610,7 @@ int leaf_probe_read(LeafProbe &probe, bool &scattered) {
 
 int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st,
                        i64 &done) {
-  const i64 nblocks = make_bin_geom(a.g, LB_EDGE).nblocks;
-  const i64 most = std::max<i64>((i64)1 << 22, 512 * nblocks);
-  const i64 nparts = (a.np + most - 1) / most, size = (a.np + nparts - 1) / nparts;
+  const i64 size = part_size(a.np, a.g);
   const int L = LB_EDGE + (order == 3 && !lower ? 4 : 3);
   const size_t lds = sizeof(double) * 6 * (size_t)(L * L * L);
   std::lock_guard<std::mutex> lock(g_order);
@@ -580,52 +647,63 @@ int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream
 bool leaf_binned_current_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
 bool leaf_binned_rho_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
 
-int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, bool &done) {
+// the current of a.np particles, in parts that bound the records' memory
+template <bool MID>
+static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &done) {
   std::lock_guard<std::mutex> lock(g_order);
-  done = false;
-  BinGeom bg;
-  int *perm, *nitems;
-  int4 *items;
-  i64 maxitems;
   const EsirkConst<double> &c = a.ec;
-  const LbPos pos{a.np, a.xp, a.yp, a.zp, a.ux, a.uy, a.uz, a.gi, c.xmin, c.ymin, c.zmin, c.dxi,
-                  c.dyi, c.dzi, {0.5 * c.dtsdx0, 0.5 * c.dtsdy0, 0.5 * c.dtsdz0}, 0, nullptr};
-  if (!lb_sort<LB_EDGE, true>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems,
-                                 maxitems))
-    return PXRHIP_OK;
+  const i64 size = part_size(a.np, a.g);
   const int L = LB_EDGE + (order == 1 ? 3 : 5);
   const size_t lds = sizeof(double) * 3 * (size_t)(L * L * L);
-  const dim3 grd(lb_grid(maxitems, lds)), blk(256);
-  if (order == 1) LB_LAUNCH((k_lb_direct<1, LB_EDGE>), a);
-  else if (order == 2) LB_LAUNCH((k_lb_direct<2, LB_EDGE>), a);
-  else LB_LAUNCH((k_lb_direct<3, LB_EDGE>), a);
-  PXR_LAUNCHED();
-  done = true;
+  // A full block holds a few thousand particles at the densities of interest,
+  // and the blocks of a modest grid are too few to share evenly among the CUs:
+  // smaller work items, until clearing and adding up the LDS blocks costs as
+  // much.  Two million in cell order on 64^3 cells, 4096 particles an item and
+  // so: order 1 374 -> 177 us, order 2 402 -> 255, order 3 446 -> 410.
+  const int chunk = std::min(rt().leaf_bin_chunk, order == 1 ? 512 : order == 2 ? 1024 : 2048);
+  done = 0;
+  LbDepo d;
+  if (order <= 2 && a.np >= DEPO_REC_MIN)
+    d.packed.rec = (double *)scratch(30, 8 * sizeof(double) * (size_t)size);
+  while (done < a.np) {
+    d.c = a.part(done, std::min(size, a.np - done));
+    LbPos pos{d.c.np, d.c.xp, d.c.yp, d.c.zp, d.c.ux, d.c.uy, d.c.uz, d.c.gi, d.c.w, c.xmin,
+              c.ymin, c.zmin, c.dxi, c.dyi, c.dzi,
+              {0.5 * c.dtsdx0, 0.5 * c.dtsdy0, 0.5 * c.dtsdz0}, 0, nullptr, {}};
+    if (d.packed.rec) {
+      LeafProbe probe;
+      launch_probe(pos, a.g, st, probe);
+      d.packed.use = probe.dev;
+      pos.packed = d.packed;
+    }
+    BinGeom bg;
+    int *perm, *nitems;
+    int4 *items;
+    i64 maxitems;
+    if (!lb_sort<LB_EDGE, MID>(pos, a.g, chunk, st, bg, perm, items, nitems, maxitems))
+      return PXRHIP_OK;
+    const dim3 grd(lb_grid(maxitems, lds)), blk(256);
+    if constexpr (MID) {
+      if (order == 1) LB_LAUNCH((k_lb_direct<1, LB_EDGE>), d);
+      else if (order == 2) LB_LAUNCH((k_lb_direct<2, LB_EDGE>), d);
+      else LB_LAUNCH((k_lb_direct<3, LB_EDGE>), d);
+    } else {
+      if (order == 1) LB_LAUNCH((k_lb_esirkepov<1, LB_EDGE>), d);
+      else if (order == 2) LB_LAUNCH((k_lb_esirkepov<2, LB_EDGE>), d);
+      else LB_LAUNCH((k_lb_esirkepov<3, LB_EDGE>), d);
+    }
+    PXR_LAUNCHED();
+    done += d.c.np;
+  }
   return PXRHIP_OK;
 }
 
-int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, bool &done) {
-  std::lock_guard<std::mutex> lock(g_order);
-  done = false;
-  BinGeom bg;
-  int *perm, *nitems;
-  int4 *items;
-  i64 maxitems;
-  const EsirkConst<double> &c = a.ec;
-  const LbPos pos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, c.xmin, c.ymin,
-                  c.zmin, c.dxi, c.dyi, c.dzi, {0.0, 0.0, 0.0}, 0, nullptr};
-  if (!lb_sort<LB_EDGE, false>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems,
-                                  maxitems))
-    return PXRHIP_OK;
-  const int L = LB_EDGE + (order == 1 ? 3 : 5);
-  const size_t lds = sizeof(double) * 3 * (size_t)(L * L * L);
-  const dim3 grd(lb_grid(maxitems, lds)), blk(256);
-  if (order == 1) LB_LAUNCH((k_lb_esirkepov<1, LB_EDGE>), a);
-  else if (order == 2) LB_LAUNCH((k_lb_esirkepov<2, LB_EDGE>), a);
-  else LB_LAUNCH((k_lb_esirkepov<3, LB_EDGE>), a);
-  PXR_LAUNCHED();
-  done = true;
-  return PXRHIP_OK;
+int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, i64 &done) {
+  return binned_current<true>(a, order, st, done);
+}
+
+int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, i64 &done) {
+  return binned_current<false>(a, order, st, done);
 }
 
 int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done) {
@@ -636,8 +714,8 @@ int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done) {
   int *perm, *nitems;
   int4 *items;
   i64 maxitems;
-  const LbPos pos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, a.xmin, a.ymin,
-                  a.zmin, a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, a.l4symtry, nullptr};
+  const LbPos pos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, nullptr, a.xmin, a.ymin,
+                  a.zmin, a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, a.l4symtry, nullptr, {}};
   if (!lb_sort<E, false>(pos, a.g, rt().leaf_bin_chunk, st, bg, perm, items, nitems, maxitems))
     return PXRHIP_OK;
   const int L = E + (order == 1 ? 1 : 3);

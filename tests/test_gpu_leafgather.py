@@ -14,7 +14,7 @@ from tests.test_gpu_leaf import NG, NX, NY, NZ, SHAPE, H, T, TG, particles
 pytestmark = pytest.mark.gpu
 
 COUNTS = {1: (3145727, 3145728), 2: (786431, 786432, 1700001),
-          3: (786431, 786432, 900001, 4300001)}
+          3: (786431, 786432, 900001, 8400001)}
 
 
 @pytest.fixture(scope="module")
