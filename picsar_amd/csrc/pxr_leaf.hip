@@ -345,10 +345,30 @@ struct YeeArgs {
   double mudt, cx, cy, cz;
 };
 
+// Workgroups go to the eight XCDs in turn, each with an L2 of its own, and a
+// node's values are wanted again a row and a plane away: in launch order a
+// plane would be fetched by several XCDs.  xcd_block gives each XCD runs of S
+// consecutive blocks instead (a few rows to a plane: longer runs send the
+// XCDs to parts of memory too far apart, and leave a small grid unbalanced).
+// Yee B and E updates, in launch order and with S = 32: 256^3 cells 308 and
+// 366 -> 294 and 344 us, 128^3 49 and 61 -> 47 and 58, 255 x 250 x 37 56 and
+// 73 -> 46 and 58, 320^3 557 and 661 -> 529 and 637 (S = 512: 538 and 655; a
+// single run per XCD: 560 and 677).
+PXR_DEV unsigned xcd_block(unsigned S) {
+  const unsigned b = blockIdx.x, sup = b / (8 * S), r = b % (8 * S);
+  return sup * (8 * S) + (r & 7) * S + (r >> 3);
+}
+constexpr unsigned YEE_RUN = 32;
+
+// blocks of a launch that maps them with xcd_block: whole rounds of the XCDs
+static unsigned xcd_grid(i64 blocks, unsigned S) {
+  return (unsigned)((blocks + 8 * S - 1) / (8 * S) * (8 * S));
+}
+
 __global__ __launch_bounds__(256) void k_yee_e(YeeArgs a) {
   const int nxu = a.un.hi[0] - a.un.lo[0] + 1;
   const int nyu = a.un.hi[1] - a.un.lo[1] + 1;
-  const i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  const i64 t = (i64)xcd_block(YEE_RUN) * 256 + threadIdx.x;
   const i64 tot = (i64)nxu * nyu * (a.un.hi[2] - a.un.lo[2] + 1);
   if (t >= tot) return;
   const int j = a.un.lo[0] + (int)(t % nxu);
@@ -375,7 +395,7 @@ __global__ __launch_bounds__(256) void k_yee_e(YeeArgs a) {
 __global__ __launch_bounds__(256) void k_yee_b(YeeArgs a) {
   const int nxu = a.un.hi[0] - a.un.lo[0] + 1;
   const int nyu = a.un.hi[1] - a.un.lo[1] + 1;
-  const i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  const i64 t = (i64)xcd_block(YEE_RUN) * 256 + threadIdx.x;
   const i64 tot = (i64)nxu * nyu * (a.un.hi[2] - a.un.lo[2] + 1);
   if (t >= tot) return;
   const int j = a.un.lo[0] + (int)(t % nxu);
@@ -1237,7 +1257,7 @@ int pxrhip_push_em3d_evec(const int64_t *xlo, const int64_t *xhi, const int64_t 
   a.cz = dtsdz;
   i64 tot = (i64)(a.un.hi[0] - a.un.lo[0] + 1) * (a.un.hi[1] - a.un.lo[1] + 1) *
             (a.un.hi[2] - a.un.lo[2] + 1);
-  hipLaunchKernelGGL(k_yee_e, dim3(grid1d(tot, 256)), dim3(256), 0, rt().stream, a);
+  hipLaunchKernelGGL(k_yee_e, dim3(xcd_grid(grid1d(tot, 256), YEE_RUN)), dim3(256), 0, rt().stream, a);
   PXR_LAUNCHED();
   return PXRHIP_OK;
 }
@@ -1277,7 +1297,7 @@ int pxrhip_push_em3d_bvec(const int64_t *xlo, const int64_t *xhi, const int64_t 
   a.cz = dtsdz;
   i64 tot = (i64)(a.un.hi[0] - a.un.lo[0] + 1) * (a.un.hi[1] - a.un.lo[1] + 1) *
             (a.un.hi[2] - a.un.lo[2] + 1);
-  hipLaunchKernelGGL(k_yee_b, dim3(grid1d(tot, 256)), dim3(256), 0, rt().stream, a);
+  hipLaunchKernelGGL(k_yee_b, dim3(xcd_grid(grid1d(tot, 256), YEE_RUN)), dim3(256), 0, rt().stream, a);
   PXR_LAUNCHED();
   return PXRHIP_OK;
 }
