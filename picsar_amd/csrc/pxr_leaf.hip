@@ -359,6 +359,10 @@ PXR_DEV unsigned xcd_block(unsigned S) {
   return sup * (8 * S) + (r & 7) * S + (r >> 3);
 }
 constexpr unsigned YEE_RUN = 32;
+// k_norder_z, B and E at order 4: 256^3 cells 388 and 531 -> 369 and 461 us,
+// 128^3 64 and 84 -> 53 and 58, 96 x 96 x 192 50 and 61 -> 42 and 51, 61 x 45 x
+// 70 19.2 and 20.2 -> 18.6 and 18.4 (S = 64: 21.4 and 21.1)
+constexpr unsigned NORDER_RUN = 16;
 
 // blocks of a launch that maps them with xcd_block: whole rounds of the XCDs
 static unsigned xcd_grid(i64 blocks, unsigned S) {
@@ -543,11 +547,14 @@ template <int NH, bool E, int IST>
 __global__ __launch_bounds__(256) void k_norder_z(NorderArgs a) {
   const GridGeom &g = a.g;
   const int nxu = g.nx + 2 * a.nxs + 1, nyu = g.ny + 2 * a.nys + 1, nzu = g.nz + 2 * a.nzs + 1;
-  const int ju = (int)blockIdx.x * ZBX + (int)(threadIdx.x % ZBX);
-  const int ku = (int)blockIdx.y * (256 / ZBX) + (int)(threadIdx.x / ZBX);
-  if (ju >= nxu || ku >= nyu) return;
+  const unsigned gbx = (nxu + ZBX - 1) / ZBX, gby = (nyu + 256 / ZBX - 1) / (256 / ZBX);
+  const unsigned bb = xcd_block(NORDER_RUN), by = bb / gbx;
+  const int ju = (int)(bb % gbx) * ZBX + (int)(threadIdx.x % ZBX);
+  const int ku = (int)(by % gby) * (256 / ZBX) + (int)(threadIdx.x / ZBX);
+  const int bz = by / gby;
+  if (ju >= nxu || ku >= nyu || bz * a.zchunk >= nzu) return;
   const int j = -a.nxs + ju, k = -a.nys + ku;
-  const int l0 = -a.nzs + (int)blockIdx.z * a.zchunk;
+  const int l0 = -a.nzs + bz * a.zchunk;
   const int l1 = min(l0 + a.zchunk, -a.nzs + nzu);  // exclusive
   const int nxh = imin3(a.co.nh[0], (g.nx - j) + g.gx, j + g.gx);
   const int nyh = imin3(a.co.nh[1], (g.ny - k) + g.gy, k + g.gy);
@@ -636,7 +643,7 @@ static void launch_norder_z(NorderArgs a, hipStream_t st) {
   a.zchunk = ZCHUNK;
   while (a.zchunk > 4 && bx * by * ((nzu + a.zchunk - 1) / a.zchunk) < 4 * (i64)rt().num_cus)
     a.zchunk /= 2;
-  const dim3 gr((unsigned)bx, (unsigned)by, (unsigned)((nzu + a.zchunk - 1) / a.zchunk)), bl(256);
+  const dim3 gr(xcd_grid(bx * by * ((nzu + a.zchunk - 1) / a.zchunk), NORDER_RUN)), bl(256);
   if (a.ist) hipLaunchKernelGGL((k_norder_z<NH, E, 1>), gr, bl, 0, st, a);
   else hipLaunchKernelGGL((k_norder_z<NH, E, 0>), gr, bl, 0, st, a);
 }
