@@ -627,9 +627,20 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(
   const int ghi[3] = {g.nx + g.gx, g.ny + g.gy, g.nz + g.gz};
   const double x0[3] = {a.xmin, a.ymin, a.zmin}, di[3] = {a.dxi, a.dyi, a.dzi};
   const int nch = *a.nchunks;
+  // A workgroup's first item is its own number: the adds of a launch's
+  // workgroups on the one counter, 8 ns each, would be as long as a small
+  // launch's work (with them 70, without 63 us for 297 items of 32^3 cells,
+  // order 1; 197 and 192 us for 2544 items of 61 x 45 x 70, order 2).  The
+  // mixed order-3 Esirkepov kernel keeps them: the extra state costs it a
+  // register it does not have (2.29 -> 2.47 ms on 144^3 cells).
+  constexpr bool OWN_FIRST = !(MX && BANKS);
+  bool first = true;
   for (;;) {
     if (threadIdx.x == 0) {
-      const int q = atomicAdd(a.queue, 1);
+      int q;
+      if (OWN_FIRST && first) q = blockIdx.x;
+      else q = (OWN_FIRST ? (int)gridDim.x : 0) + atomicAdd(a.queue, 1);
+      first = false;
       s_chunk = (a.order && q < nch) ? a.order[q] : q;
       for (int d = 0; d < 3; d++) {
         s_box[d] = INT_MAX;

@@ -1325,8 +1325,8 @@ __global__ __launch_bounds__(256) void k_rho_tiles(RhoTileArgs a) {
   const int glo[3] = {-g.gx, -g.gy, -g.gz};
   const int ghi[3] = {g.nx + g.gx, g.ny + g.gy, g.nz + g.gz};
   const int nch = *a.nchunks;
-  for (;;) {
-    if (threadIdx.x == 0) s_chunk = atomicAdd(a.queue, 1);
+  for (bool first = true;; first = false) {  // the first item without the counter, as k_fused
+    if (threadIdx.x == 0) s_chunk = first ? blockIdx.x : (int)gridDim.x + atomicAdd(a.queue, 1);
     __syncthreads();
     const int c = s_chunk;
     __syncthreads();  // read by all before the next fetch overwrites it
