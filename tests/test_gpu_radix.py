@@ -21,7 +21,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,cells", [
     (1, (5, 5, 5)), (63, (3, 2, 1)), (64, (1, 1, 1)), (65, (12, 9, 7)), (4095, (16, 16, 8)),
     (4096, (17, 11, 11)), (4097, (1, 1, 1)), (70001, (16, 16, 8)), (70001, (41, 50, 1)),
-    (300007, (63, 64, 65)), (20011, (200, 170, 130))])
+    (300007, (63, 64, 65)), (20011, (200, 170, 130)), (1023, (5, 5, 5)), (1024, (40, 9, 7)),
+    (1025, (1, 1, 1)), (524287, (16, 16, 8)), (524288, (16, 16, 8)), (524288, (70, 50, 3))])
 def test_sort_sizes_bitexact(dev, pxr, orc, n, cells):
     rng = np.random.default_rng(n + cells[0])
     P = [rng.uniform(0, c, n) for c in cells] + [rng.standard_normal(n) for _ in range(4)]
