@@ -23,9 +23,27 @@ namespace pxr {
 // ---------------------------------------------------------------------------
 // field gathering
 // ---------------------------------------------------------------------------
+// Workgroups go to the eight XCDs in turn, each with an L2 of its own.  Where
+// neighbouring blocks read the same lines, xcd_block gives each XCD runs of S
+// consecutive blocks instead.
+PXR_DEV unsigned xcd_block(unsigned S) {
+  const unsigned b = blockIdx.x, sup = b / (8 * S), r = b % (8 * S);
+  return sup * (8 * S) + (r & 7) * S + (r >> 3);
+}
+// blocks of a launch that maps them with xcd_block: whole rounds of the XCDs
+static unsigned xcd_grid(i64 blocks, unsigned S) {
+  return (unsigned)((blocks + 8 * S - 1) / (8 * S) * (8 * S));
+}
+
+// Particles in cell order share the rows of their stencils with the blocks
+// around.  In launch order and with S = 16, order 3: a million on 64^3 cells
+// 143 -> 136 us, two million 236 -> 221, four million on 128^3 553 -> 530
+// (order 2: 96 -> 93, 147 -> 140, 316 -> 310; S = 4: 138, 233 and 542).
+constexpr unsigned GATHER_RUN = 16;
+
 template <int N, int M>
 __global__ __launch_bounds__(256) void k_gather(LeafGatherArgs a) {
-  const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  const i64 ip = (i64)xcd_block(GATHER_RUN) * 256 + threadIdx.x;
   if (ip >= a.np || (a.skip && *a.skip)) return;
   const double x = (a.xp[ip] - a.xmin) * a.dxi;
   const double y = (a.yp[ip] - a.ymin) * a.dyi;
@@ -51,7 +69,7 @@ __global__ __launch_bounds__(256) void k_gather(LeafGatherArgs a) {
 static unsigned dep_block(i64 np) { return np < (i64)256 * rt().num_cus ? 64 : 256; }
 
 static void launch_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st) {
-  const dim3 grd(grid1d(a.np, 256)), blk(256);
+  const dim3 grd(xcd_grid(grid1d(a.np, 256), GATHER_RUN)), blk(256);
   switch (order * 2 + (lower ? 1 : 0)) {
     case 2: hipLaunchKernelGGL((k_gather<1, 1>), grd, blk, 0, st, a); break;
     case 3: hipLaunchKernelGGL((k_gather<1, 0>), grd, blk, 0, st, a); break;
@@ -345,29 +363,19 @@ struct YeeArgs {
   double mudt, cx, cy, cz;
 };
 
-// Workgroups go to the eight XCDs in turn, each with an L2 of its own, and a
-// node's values are wanted again a row and a plane away: in launch order a
-// plane would be fetched by several XCDs.  xcd_block gives each XCD runs of S
-// consecutive blocks instead (a few rows to a plane: longer runs send the
-// XCDs to parts of memory too far apart, and leave a small grid unbalanced).
+// A node's values are wanted again a row and a plane away: in launch order a
+// plane would be fetched by several XCDs.  Runs of a few rows to a plane;
+// longer ones send the XCDs to parts of memory too far apart, and leave a
+// small grid unbalanced.
 // Yee B and E updates, in launch order and with S = 32: 256^3 cells 308 and
 // 366 -> 294 and 344 us, 128^3 49 and 61 -> 47 and 58, 255 x 250 x 37 56 and
 // 73 -> 46 and 58, 320^3 557 and 661 -> 529 and 637 (S = 512: 538 and 655; a
 // single run per XCD: 560 and 677).
-PXR_DEV unsigned xcd_block(unsigned S) {
-  const unsigned b = blockIdx.x, sup = b / (8 * S), r = b % (8 * S);
-  return sup * (8 * S) + (r & 7) * S + (r >> 3);
-}
 constexpr unsigned YEE_RUN = 32;
 // k_norder_z, B and E at order 4: 256^3 cells 388 and 531 -> 369 and 461 us,
 // 128^3 64 and 84 -> 53 and 58, 96 x 96 x 192 50 and 61 -> 42 and 51, 61 x 45 x
 // 70 19.2 and 20.2 -> 18.6 and 18.4 (S = 64: 21.4 and 21.1)
 constexpr unsigned NORDER_RUN = 16;
-
-// blocks of a launch that maps them with xcd_block: whole rounds of the XCDs
-static unsigned xcd_grid(i64 blocks, unsigned S) {
-  return (unsigned)((blocks + 8 * S - 1) / (8 * S) * (8 * S));
-}
 
 __global__ __launch_bounds__(256) void k_yee_e(YeeArgs a) {
   const int nxu = a.un.hi[0] - a.un.lo[0] + 1;
