@@ -488,11 +488,13 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
  * a mixed-precision species; fused.lds_bytes and fused.wg_per_cu are those
  * of an FP64 one), "rebin.stable" (1, the default: pxrhip_tiles_rebin_sort
  * keeps the source order inside a cell; 0: the order in which the GPU's
- * waves arrive), "leaf.bin_min" (pxrhip_depose_jxjyjz with the Esirkepov
- * current and pxrhip_depose_rho_n sum calls of at least this many particles,
- * and one per 8^3-node block of the arrays, block by block in LDS; default
- * 65536, 0: never) and "leaf.bin_chunk" (largest work item of that form,
- * default 4096 particles).
+ * waves arrive), "leaf.bin_min" (pxrhip_depose_jxjyjz and
+ * pxrhip_depose_rho_n sum calls of at least this many particles, and one per
+ * 8^3-node block of the arrays, block by block in LDS; default 65536, 0:
+ * never, nor does pxrhip_geteb3d_energy_conserving then gather large sets
+ * in no order block by block) and "leaf.bin_chunk" (largest work item of
+ * that form, default 4096 particles; the currents and the gather take
+ * smaller ones by themselves, 512 to 2048).
  * wg_per_cu 0 (the default) is automatic: three workgroups per CU with
  * 52224 bytes each when a work item of four sorting rows of the widest tile
  * fits that, else two with 79616 bytes; a wg_per_cu above 0 takes the
