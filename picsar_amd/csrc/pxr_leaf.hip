@@ -1506,7 +1506,7 @@ constexpr i64 SORT_GROUP_NP = 1 << 24;
 //
 // One workgroup used to place all particles in order, whatever their number:
 // 8.5 ms of a 8.9 ms call for 1,000,003 particles in 48^3 cells.  The radix
-// sort spreads the ranking over the chip: 0.25 ms for the same call, of which
+// sort spreads the ranking over the chip: 0.22 ms for the same call, of which
 // the sort is 0.08 ms, the gather of the eight arrays 0.042 and the store
 // 0.021 ms.
 static int bin_sort_run(int64_t np2, double *const *arr, const SortGeom &s, const RadixPlan &plan,

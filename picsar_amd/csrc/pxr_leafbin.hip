@@ -652,7 +652,8 @@ template <bool MID>
 static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &done) {
   std::lock_guard<std::mutex> lock(g_order);
   const EsirkConst<double> &c = a.ec;
-  const i64 size = part_size(a.np, a.g);
+  const bool records = order <= 2 && a.np >= DEPO_REC_MIN;
+  const i64 size = records ? part_size(a.np, a.g) : a.np;
   const int L = LB_EDGE + (order == 1 ? 3 : 5);
   const size_t lds = sizeof(double) * 3 * (size_t)(L * L * L);
   // A full block holds a few thousand particles at the densities of interest,
@@ -663,7 +664,7 @@ static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &don
   const int chunk = std::min(rt().leaf_bin_chunk, order == 1 ? 512 : order == 2 ? 1024 : 2048);
   done = 0;
   LbDepo d;
-  if (order <= 2 && a.np >= DEPO_REC_MIN)
+  if (records)
     d.packed.rec = (double *)scratch(30, 8 * sizeof(double) * (size_t)size);
   while (done < a.np) {
     d.c = a.part(done, std::min(size, a.np - done));
