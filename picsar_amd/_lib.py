@@ -135,7 +135,7 @@ def last_error() -> str:
 
 
 def call(name: str, *args) -> int:
-    lib = load()
+    lib = _lib if _lib is not None else load()
     fn = getattr(lib, name, None)
     if fn is None:
         raise PxrHipError(ERR_UNSUPPORTED, f"{name} is not exported by {LIB_PATH}")

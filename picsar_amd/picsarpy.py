@@ -28,6 +28,7 @@ attributes of ``picsar``.
 from __future__ import annotations
 
 import ctypes as C
+import sys
 
 import numpy as np
 
@@ -84,6 +85,15 @@ class _Call:
         return t.data_ptr()
 
     def arr(self, a, need, name, write=False, fortran_shape=None):
+        # the usual tensor first: a call of a small set spends more time on
+        # its thirty arguments than on the GPU.  Everything that this does not
+        # accept goes through the checks below, which say what is wrong.
+        t = sys.modules.get("torch")
+        if t is not None and type(a) is t.Tensor and a.dtype is t.float64 and a.is_cuda and \
+                a.is_contiguous() and a.numel() >= need and \
+                (fortran_shape is None or a.dim() != 3 or a.shape == fortran_shape[::-1]):
+            self.torch = True
+            return a.data_ptr()
         if isinstance(a, DeviceArray):
             if a.dtype != np.float64:
                 raise TypeError(f"{name}: expected float64")
@@ -111,6 +121,8 @@ class _Call:
 
     def ptrs(self, handles):
         """Copy the staged numpy arrays to the device; device pointers."""
+        if not self.staged:
+            return handles
         out = []
         for h in handles:
             if isinstance(h, _Staged):
