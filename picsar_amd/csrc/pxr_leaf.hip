@@ -64,10 +64,6 @@ __global__ __launch_bounds__(256) void k_gather(LeafGatherArgs a) {
   a.bz[ip] += out[5];
 }
 
-// Threads per block of the deposition kernels: a set too small for blocks of
-// four waves on every CU is dealt out in single waves.
-static unsigned dep_block(i64 np) { return np < (i64)256 * rt().num_cus ? 64 : 256; }
-
 static void launch_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st) {
   const dim3 grd(xcd_grid(grid1d(a.np, 256), GATHER_RUN)), blk(256);
   switch (order * 2 + (lower ? 1 : 0)) {
@@ -244,18 +240,28 @@ __global__ __launch_bounds__(256) void k_set_gamma(i64 np, const double *ux, con
 // current deposition (global atomics)
 // ---------------------------------------------------------------------------
 
-// Particles of the deposition kernels, one a thread: the lanes of a wave take
-// particles DEP_S apart out of 64 * DEP_S, which DEP_S waves share.  In
-// cell-sorted input, as the tiled species hold it, the lanes of one atomic
-// instruction then sit in different cells instead of queueing on the same
-// nodes.  The adds are done by the L2, a particle's one after the other, so a
-// small set wants all its particles in flight: 4000 order-1 particles took
-// 45 us with four particles in turn a thread, 9 us so.
+// Particles of the deposition kernels: the lanes of a wave take particles
+// DEP_S apart out of 64 * DEP_S, which several waves share.  In cell-sorted
+// input, as the tiled species hold it, the lanes of one atomic instruction
+// then sit in different cells instead of queueing on the same nodes.  A
+// thread of a block of 256 takes four consecutive ones in turn.  The adds are
+// done by the L2, a particle's one after the other, so a small set, launched
+// in single waves, wants all its particles in flight and a thread takes one:
+// 4000 order-1 particles 45 -> 9 us.  (One a thread made 33 million order-3
+// particles in cell order 4% slower, 72 -> 75 ms.)
 #define DEP_S 16
-PXR_DEV i64 dep_particle() {
+PXR_DEV int dep_per_thread() { return blockDim.x == 64 ? 1 : 4; }
+PXR_DEV i64 dep_particle(int k, int per) {
   const i64 w = ((i64)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  return w / DEP_S * (64 * DEP_S) + (threadIdx.x & 63) * DEP_S + w % DEP_S;
+  const int share = DEP_S / per;  // waves
+  return w / share * (64 * DEP_S) + (threadIdx.x & 63) * DEP_S + w % share * per + k;
 }
+
+// Threads per block of the deposition kernels: a set too small for blocks of
+// four waves on every CU is dealt out in single waves.
+static unsigned dep_block(i64 np) { return np < (i64)256 * rt().num_cus ? 64 : 256; }
+// blocks of that size per 64 * DEP_S particles
+static unsigned dep_blocks(unsigned block) { return block == 64 ? DEP_S : 1; }
 
 template <int N>
 PXR_DEV void esirkepov_one(const DepoArgs &a, i64 ip) {
@@ -275,8 +281,10 @@ PXR_DEV void esirkepov_one(const DepoArgs &a, i64 ip) {
 
 template <int N>
 __global__ __launch_bounds__(256) void k_esirkepov(DepoArgs a) {
-  const i64 ip = dep_particle();
-  if (ip < a.np) esirkepov_one<N>(a, ip);
+  for (int k = 0, per = dep_per_thread(); k < per; k++) {
+    const i64 ip = dep_particle(k, per);
+    if (ip < a.np) esirkepov_one<N>(a, ip);
+  }
 }
 
 template <int N>
@@ -298,8 +306,10 @@ PXR_DEV void direct_one(const DepoArgs &a, i64 ip) {
 
 template <int N>
 __global__ __launch_bounds__(256) void k_direct(DepoArgs a) {
-  const i64 ip = dep_particle();
-  if (ip < a.np) direct_one<N>(a, ip);
+  for (int k = 0, per = dep_per_thread(); k < per; k++) {
+    const i64 ip = dep_particle(k, per);
+    if (ip < a.np) direct_one<N>(a, ip);
+  }
 }
 
 // charge density, pxr_depose_rho_n (charge_deposition_3d.F90:2081-2228):
@@ -336,8 +346,10 @@ PXR_DEV void rho_one(const RhoArgs &a, i64 ip) {
 
 template <int N>
 __global__ __launch_bounds__(256) void k_rho(RhoArgs a) {
-  const i64 ip = dep_particle();
-  if (ip < a.np) rho_one<N>(a, ip);
+  for (int k = 0, per = dep_per_thread(); k < per; k++) {
+    const i64 ip = dep_particle(k, per);
+    if (ip < a.np) rho_one<N>(a, ip);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1124,7 +1136,7 @@ int pxrhip_depose_jxjyjz(double *jx, double *jy, double *jz, int64_t np, const d
   }
   if (done < np) {  // all of them, or those there was no memory to order
     const DepoArgs p = a.part(done, np - done);
-    const dim3 blk(dep_block(p.np)), grd(grid1d(p.np, 64 * DEP_S) * (64 * DEP_S / blk.x));
+    const dim3 blk(dep_block(p.np)), grd(grid1d(p.np, 64 * DEP_S) * dep_blocks(blk.x));
     if (direct) {
       if (nox == 1) hipLaunchKernelGGL(k_direct<1>, grd, blk, 0, st, p);
       else if (nox == 2) hipLaunchKernelGGL(k_direct<2>, grd, blk, 0, st, p);
@@ -1182,7 +1194,7 @@ int pxrhip_depose_rho_n(double *rho, int64_t np, const double *xp, const double 
   a.g = mkgeom(nx, ny, nz, nxguard, nyguard, nzguard);
   a.rho = rho;
   a.bad = rt().d_bad;
-  const dim3 blk(dep_block(np)), grd(grid1d(np, 64 * DEP_S) * (64 * DEP_S / blk.x));
+  const dim3 blk(dep_block(np)), grd(grid1d(np, 64 * DEP_S) * dep_blocks(blk.x));
   hipStream_t st = rt().stream;
   bool done = false;
   if (leaf_binned_rho_pays(np, a.g)) {
