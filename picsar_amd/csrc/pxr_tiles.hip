@@ -1046,6 +1046,8 @@ PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, Chunk *out, i64 room, in
   if (g != GROUP_ROWS) return 0;
   // start of row y (y = ny3: the end of the plane)
   for (int y = lane; y <= min(ny3, ROWS - 1); y += CG) rs[y] = a.bin_start[base + (int64_t)y * nx3];
+  // the lanes read each other's entries: one wave, so its own LDS order suffices
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   auto start = [&](int y) { return y < ROWS ? rs[y] : (i64)a.bin_start[base + (int64_t)y * nx3]; };
   int fe[3], je[3];
   AxisFit(a, t, 0).extent(a.bg, 0, 0, nx3 - 1, fe[0], je[0]);

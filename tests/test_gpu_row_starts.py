@@ -1,0 +1,51 @@
+"""Rows of a plane whose starts are staged by one lane of a unit's sixteen and
+read by another: row counts around the sixteen lanes and the 96 staged rows,
+with empty rows among full ones.
+
+As in test_gpu_work_items: the charge density of the work items against the
+leaf routine on the same particles, where a particle left out or taken twice
+changes it by a particle's charge; the bar is n roundings of the largest node
+value.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("chunk", [48, 1024])
+@pytest.mark.parametrize("ny", [1, 2, 15, 16, 17, 31, 32, 33, 95, 96, 97, 112, 113])
+def test_rows_by_other_lanes(ny, chunk):
+    from picsar_amd import _lib
+    from picsar_amd.devmem import DeviceArray, DeviceGrid
+    from picsar_amd.sim import Simulation
+    _lib.call("pxrhip_init", 0)
+    old = C.c_int64()
+    _lib.call("pxrhip_get_tuning", b"fused.chunk", C.byref(old))
+    n = (4, max(ny, 4), 5)
+    rng = np.random.default_rng(ny)
+    rows = np.flatnonzero(rng.random(ny) < 0.6) if ny > 2 else np.arange(ny)
+    npart = 60 * len(rows)
+    sim = Simulation(*n, 1.0, 1.0, 1.0, 0.0, 0.0, 0.0, 1, 1, 1, order=1)
+    pos = [4 * rng.random(npart), rng.choice(rows, npart) + rng.random(npart),
+           5 * rng.random(npart)]
+    sim.add_species("e", -1.0, 1.0, *pos, *np.zeros((3, npart)), 0.5 + rng.random(npart))
+    sp, g = sim.species[0], sim.ng
+    want, got = DeviceGrid(*n, g), DeviceGrid(*n, g)
+    a = sp.arrays()
+    d = [DeviceArray.from_numpy(np.ascontiguousarray(a[k], dtype=np.float64))
+         for k in ("x", "y", "z", "w")]
+    _lib.call("pxrhip_depose_rho_n", want.ptr, npart, *(v.ptr for v in d), sp.q, sim.xmin,
+              sim.ymin, sim.zmin, sim.dx, sim.dy, sim.dz, *n, g, g, g, 1, 1, 1, 1, 0)
+    s = sp.struct(sp.cur)
+    _lib.call("pxrhip_set_tuning", b"fused.chunk", chunk)
+    try:
+        _lib.call("pxrhip_tiles_depose_rho", C.byref(sim.grid), C.byref(s), got.ptr, 1)
+        _lib.call("pxrhip_tiles_check")
+    finally:
+        _lib.call("pxrhip_set_tuning", b"fused.chunk", old.value)
+    want, got = want.numpy(), got.numpy()
+    assert np.abs(want).max() > 0
+    assert np.abs(got - want).max() <= (npart + 8) * np.finfo(float).eps * np.abs(want).max()
