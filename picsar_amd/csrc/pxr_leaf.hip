@@ -9,6 +9,8 @@
 // computation follow the reference's operation order bit for bit.
 #include <stdio.h>
 
+#include <mutex>
+
 #include "pxr_device.h"
 #include "pxr_generic.h"
 #include "pxr_kernels.h"
@@ -1503,6 +1505,8 @@ static int bin_sort_geom(int64_t np2, double *const *arr, int64_t wpid, double x
   return PXRHIP_OK;
 }
 
+static std::mutex g_sort;
+
 // Particles up to which the eight arrays are staged together (64 B each):
 // one gather and one store launch in place of eight of each.
 constexpr i64 SORT_GROUP_NP = 1 << 24;
@@ -1514,7 +1518,10 @@ constexpr i64 SORT_GROUP_NP = 1 << 24;
 // return.  The sorted indices end in idx[0]; key[1], idx[1] are free by the
 // time tmp is used and may overlap it.  A key out of range leaves the arrays
 // as they are: the moving kernels see the counter, the host reads it at the
-// end (the call synchronises the stream once).
+// end (the call synchronises the stream once).  Every moving kernel has to
+// find the same answer there, so nothing but sorts may write the counter, and
+// g_sort is held from the first use of the buffers to that synchronisation:
+// sorts of several threads share both.
 //
 // One workgroup used to place all particles in order, whatever their number:
 // 8.5 ms of a 8.9 ms call for 1,000,003 particles in 48^3 cells.  The radix
@@ -1534,7 +1541,7 @@ static int bin_sort_run(int64_t np2, double *const *arr, const SortGeom &s, cons
   else sort_move<1>(np2, arr, tmp, idx[0], bad_ctr, st);
   PXR_LAUNCHED();
   unsigned long long bad = 0;
-  int r = take_counter(bad_ctr, &bad);
+  int r = take_counter(bad_ctr, &bad, st);
   if (r) return r;
   if (bad)
     return set_error(PXRHIP_ERR_BOUNDS,
@@ -1594,6 +1601,7 @@ int pxrhip_particle_bin_sorting(int64_t np2, double *xp, double *yp, double *zp,
                         empty);
   if (r || empty) return r;
   const RadixPlan plan = radix_plan(np2, s.nbins, 1 << 20);
+  std::lock_guard<std::mutex> lock(g_sort);
   bool group = np2 <= SORT_GROUP_NP;
   int *key0 = (int *)scratch(0, sizeof(int) * np2);
   int *hist = (int *)scratch(1, sizeof(int) * (size_t)plan.hist_ints);
@@ -1606,7 +1614,7 @@ int pxrhip_particle_bin_sorting(int64_t np2, double *xp, double *yp, double *zp,
   }
   if (!key0 || !hist || !idx0 || !tmp) return set_error(PXRHIP_ERR_HIP, "scratch allocation failed");
   int *key[2] = {key0, (int *)tmp}, *idx[2] = {idx0, (int *)tmp + np2};
-  return bin_sort_run(np2, arr, s, plan, key, idx, hist, tmp, group, rt().d_bad);
+  return bin_sort_run(np2, arr, s, plan, key, idx, hist, tmp, group, rt().d_sort_bad);
 }
 
 int pxrhip_particle_bin_sorting_noalloc(int64_t np2, double *xp, double *yp, double *zp,
@@ -1630,6 +1638,7 @@ int pxrhip_particle_bin_sorting_noalloc(int64_t np2, double *xp, double *yp, dou
     return set_error(PXRHIP_ERR_ARG, "the sorting grid has %lld bins, more than the %lld of the "
                      "fixed sort scratch", (long long)s.nbins, (long long)SORT_NA_NBINS);
   unsigned char *base;
+  std::lock_guard<std::mutex> lock(g_sort);
   if ((r = sort_scratch_ptr(&base))) return r;
   const RadixPlan plan = radix_plan(np2, s.nbins, SORT_NA_NBINS);
   double *tmp = (double *)(base + SORT_NA_OFF_TMP);

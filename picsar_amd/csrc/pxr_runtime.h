@@ -19,6 +19,7 @@ struct Runtime {
   bool checks = true;
   // device counter of skipped particles; from [2] on a word per report slot
   unsigned long long *d_bad = nullptr;
+  unsigned long long *d_sort_bad = nullptr;  // the leaf sort's own counter of bad keys (d_bad + 1)
   unsigned long long *h_report = nullptr;  // pinned host memory, see report_slot
   int num_cus = 256;
   // leaf deposition summed in LDS blocks (pxr_leafbin.hip) from this many
@@ -45,7 +46,7 @@ unsigned long long *report_slot();
 // read the bad-particle counter (synchronises the stream), reset it to 0
 int take_bad(unsigned long long *n);
 // the same for any device counter
-int take_counter(unsigned long long *ctr, unsigned long long *n);
+int take_counter(unsigned long long *ctr, unsigned long long *n, hipStream_t st);
 
 inline unsigned grid1d(int64_t n, int block) {
   int64_t b = (n + block - 1) / block;

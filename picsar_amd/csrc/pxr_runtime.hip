@@ -72,17 +72,16 @@ __global__ void k_take_counter(unsigned long long *ctr, unsigned long long *host
 // Every checked call ends with this: one small launch and one wait.  (A copy
 // into pageable memory goes through a staging buffer of the runtime and
 // waits for itself, 8 us more.)
-int take_counter(unsigned long long *ctr, unsigned long long *n) {
+int take_counter(unsigned long long *ctr, unsigned long long *n, hipStream_t st) {
   volatile unsigned long long *h = report_slot();
-  hipLaunchKernelGGL(k_take_counter, dim3(1), dim3(1), 0, g_rt.stream, ctr,
-                     (unsigned long long *)h);
+  hipLaunchKernelGGL(k_take_counter, dim3(1), dim3(1), 0, st, ctr, (unsigned long long *)h);
   PXR_LAUNCHED();
-  PXR_HIP(hipStreamSynchronize(g_rt.stream));
+  PXR_HIP(hipStreamSynchronize(st));
   *n = *h;
   return PXRHIP_OK;
 }
 
-int take_bad(unsigned long long *n) { return take_counter(g_rt.d_bad, n); }
+int take_bad(unsigned long long *n) { return take_counter(g_rt.d_bad, n, g_rt.stream); }
 
 }  // namespace pxr
 
@@ -110,6 +109,7 @@ int pxrhip_init(int device) {
   if (!g_rt.d_bad) {
     PXR_HIP(hipMalloc(&g_rt.d_bad, (2 + REPORT_SLOTS) * sizeof(unsigned long long)));
     PXR_HIP(hipMemset(g_rt.d_bad, 0, (2 + REPORT_SLOTS) * sizeof(unsigned long long)));
+    g_rt.d_sort_bad = g_rt.d_bad + 1;
   }
   if (!g_rt.h_report)
     PXR_HIP(hipHostMalloc(&g_rt.h_report, REPORT_SLOTS * sizeof(unsigned long long), 0));
@@ -126,7 +126,7 @@ int pxrhip_finalize(void) {
     s.bytes = 0;
   }
   if (g_rt.d_bad) hipFree(g_rt.d_bad);
-  g_rt.d_bad = nullptr;
+  g_rt.d_bad = g_rt.d_sort_bad = nullptr;
   if (g_rt.h_report) hipHostFree(g_rt.h_report);
   g_rt.h_report = nullptr;
   if (g_rt.own_stream && g_rt.stream) hipStreamDestroy(g_rt.stream);
