@@ -20,6 +20,11 @@
  *   - Work is enqueued on the library's current stream (pxrhip_set_stream).
  *     With checks on (the default) a call that can find out-of-range
  *     particles synchronises that stream and reports them.
+ *   - Large leaf gathers and depositions, which order their particles in
+ *     scratch that all calls share, wait on the GPU for the one before, on
+ *     whatever stream that was.  The tiled routines and the diagnostics
+ *     share scratch too and do not wait: where pxrhip_set_stream switches
+ *     between streams, their work on one has to be done before the next.
  *   - Every function returns PXRHIP_OK (0) or a negative error code;
  *     pxrhip_last_error() returns the message of the last failure.
  */
