@@ -572,10 +572,19 @@ static unsigned lb_grid(i64 maxitems, size_t lds) {
     hipLaunchKernelGGL(KERNEL, grd, blk, lds, st, ARGS, bg, perm, items, nitems);             \
   } while (0)
 
+// Work recorded into a graph, the library's or one of the caller's own, may
+// not refer to scratch that a later call frees when it needs more.
+static bool recording(hipStream_t st) {
+  if (rt().capturing) return true;
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &s) != hipSuccess) (void)hipGetLastError();
+  return s != hipStreamCaptureStatusNone;
+}
+
 static bool pays(i64 np, const GridGeom &g, int edge) {
   const Runtime &r = rt();
-  return r.leaf_bin_min > 0 && np >= r.leaf_bin_min && !r.capturing &&
-         np >= make_bin_geom(g, edge).nblocks;
+  return r.leaf_bin_min > 0 && np >= r.leaf_bin_min && np >= make_bin_geom(g, edge).nblocks &&
+         !recording(r.stream);
 }
 
 static LbPos gather_pos(const LeafGatherArgs &a, double *rec) {

@@ -1,6 +1,7 @@
 """Large leaf calls with the checks off, one after the other on two streams:
 they share scratch for the order of their particles, and the second may not
-touch it before the first is done.
+touch it before the first is done.  And recorded into a graph of the caller's
+own: the graph may not refer to that scratch, which a later call may free.
 
 Each against the same call alone.  Currents and densities are sums in an order
 that depends on the launch: a node's sum has at most n/100 terms of up to
@@ -34,7 +35,7 @@ def streams(dev):
     s = [C.c_void_p(), C.c_void_p()]
     for p in s:
         assert hip.hipStreamCreate(C.byref(p)) == 0
-    yield s
+    yield hip, s
     dev.call("pxrhip_synchronize")
     assert hip.hipDeviceSynchronize() == 0
     dev.call("pxrhip_set_stream", C.c_void_p(own))
@@ -55,17 +56,20 @@ def rho(dev, J, n, P, order, _):
              1.0, 1.0, NX, NY, NZ, NG, NG, NG, order, order, order, 1, 0)
 
 
+def plasma(dev, rng, n):
+    x = particles(rng, n, margin=1.0)
+    u = [rng.uniform(-1.0, 1.0, n) for _ in range(3)]
+    g = 1 / np.sqrt(1 + u[0] ** 2 + u[1] ** 2 + u[2] ** 2)
+    return [T(dev, a) for a in (*x, *u, g, rng.uniform(0.5, 2.0, n))]
+
+
 @pytest.mark.parametrize("call,order,algo", [(current, 1, 3), (current, 3, 3), (current, 2, 0),
                                              (rho, 2, 0)])
 def test_two_streams_in_turn(dev, streams, call, order, algo):
+    _, streams = streams
     sizes = (900001, 700000, 66000, 1500007)
     rng = np.random.default_rng(order + algo)
-    sets = []
-    for n in sizes:
-        x = particles(rng, n, margin=1.0)
-        u = [rng.uniform(-1.0, 1.0, n) for _ in range(3)]
-        g = 1 / np.sqrt(1 + u[0] ** 2 + u[1] ** 2 + u[2] ** 2)
-        sets.append([T(dev, a) for a in (*x, *u, g, rng.uniform(0.5, 2.0, n))])
+    sets = [plasma(dev, rng, n) for n in sizes]
     alone, turn = ([[TG(dev, np.zeros(SHAPE)) for _ in range(3)] for _ in sizes] for _ in "ab")
     for J, n, P in zip(alone, sizes, sets):
         call(dev, J, n, P, order, algo)
@@ -85,3 +89,41 @@ def test_two_streams_in_turn(dev, streams, call, order, algo):
         for a, b in zip(A, B):
             assert np.abs(HG(a) - HG(b)).max() <= tol
         assert np.abs(HG(A[0])).max() > 0
+
+
+@pytest.mark.parametrize("call,order,algo", [(current, 1, 3), (current, 2, 0), (rho, 1, 0)])
+def test_recorded_by_the_caller(dev, streams, call, order, algo):
+    """each replay adds the call's current once, also after eager calls that
+    make the scratch grow"""
+    hip, streams = streams
+    n = 70001
+    rng = np.random.default_rng(17)
+    P, big = plasma(dev, rng, n), [plasma(dev, rng, m) for m in (2500003, 3500003)]
+    J, once, other = ([TG(dev, np.zeros(SHAPE)) for _ in range(3)] for _ in "abc")
+    dev.call("pxrhip_synchronize")
+    graph, ex = C.c_void_p(), C.c_void_p()
+    dev.call("pxrhip_set_checks", 0)
+    try:
+        dev.call("pxrhip_set_stream", streams[0])
+        call(dev, once, n, P, order, algo)
+        dev.call("pxrhip_synchronize")
+        assert hip.hipStreamBeginCapture(streams[0], 2) == 0  # relaxed
+        call(dev, J, n, P, order, algo)
+        assert hip.hipStreamEndCapture(streams[0], C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+        for k in range(3):
+            assert hip.hipGraphLaunch(ex, streams[0]) == 0
+            dev.call("pxrhip_synchronize")
+            if k < 2:
+                call(dev, other, len(big[k][0]), big[k], order, algo)
+                dev.call("pxrhip_synchronize")
+    finally:
+        dev.call("pxrhip_set_checks", 1)
+        if ex:
+            hip.hipGraphExecDestroy(ex)
+        if graph:
+            hip.hipGraphDestroy(graph)
+    tol = 3 * n / 100 * np.finfo(float).eps * 2.2 * (3 * n / 100)
+    for a, b in zip(once, J):
+        assert np.abs(3 * HG(a) - HG(b)).max() <= tol
+    assert np.abs(HG(once[0])).max() > 0
