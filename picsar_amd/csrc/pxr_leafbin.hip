@@ -111,10 +111,14 @@ struct LbGather {
 };
 
 // Block of every particle, by the node of its position (MID: of its
-// position half a step back, where the direct current is deposited).
+// position half a step back, where the direct current is deposited); clears
+// the blocks' ranges and the number of work items.
 template <int B, bool MID>
-__global__ __launch_bounds__(256) void k_lb_keys(LbPos a, BinGeom bg, int *key) {
+__global__ __launch_bounds__(256) void k_lb_keys(LbPos a, BinGeom bg, int *key, int2 *range,
+                                                 int *nitems) {
   const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (ip == 0) *nitems = 0;
+  if (ip < bg.nblocks) range[ip] = make_int2(0, 0);
   if (ip >= a.np) return;
   double x = a.x[ip], y = a.y[ip], z = a.z[ip];
   const bool pack = a.packed.on();
@@ -148,26 +152,32 @@ __global__ __launch_bounds__(256) void k_lb_keys(LbPos a, BinGeom bg, int *key) 
                         bg.nb[1] * block_axis<B>(z, bg.gd[2], bg.na[2]));
 }
 
-// first[b]: the first sorted particle of block b (first[nblocks] = np)
-__global__ __launch_bounds__(256) void k_lb_first(i64 np, const int *key, i64 nblocks,
-                                                  int *first) {
+// The sorted particles of each block that has any: the first of a run of
+// equal keys writes its start, the last its end.  (One thread per gap used to
+// write the starts of the empty blocks in it too: 4.4 ms for a bunch in 512^3
+// cells, 275 thousand blocks.)
+__global__ __launch_bounds__(256) void k_lb_ranges(i64 np, const int *key, int2 *range) {
   const i64 j = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j > np) return;
-  const i64 prev = j ? key[j - 1] : -1, here = j < np ? key[j] : nblocks;
-  for (i64 b = prev + 1; b <= here; b++) first[b] = (int)j;
+  if (j >= np) return;
+  const int k = key[j];
+  if (j == 0 || key[j - 1] != k) range[k].x = (int)j;
+  if (j == np - 1 || key[j + 1] != k) range[k].y = (int)j + 1;
 }
 
-// One workgroup: the work items (block, first slot, count) of at most
-// `chunk` particles of one block.  Each thread owns a contiguous range of
-// blocks.
-__global__ __launch_bounds__(1024) void k_lb_plan(const int *first, i64 nblocks, int chunk,
+// The work items (block, first slot, count) of at most `chunk` particles of
+// one block, a thread per block.  Their order is that of the blocks inside a
+// workgroup, and between workgroups that of their adds to *nitems.  A block of
+// more than LB_OWN items is cut by its whole wave (eight million particles in
+// one block are 16,000 items).
+constexpr int LB_OWN = 8;
+
+__global__ __launch_bounds__(1024) void k_lb_plan(const int2 *range, i64 nblocks, int chunk,
                                                   int4 *items, int *nitems) {
-  __shared__ int s[16];
+  __shared__ int s[16], first;
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const i64 per = (nblocks + 1023) / 1024;
-  const i64 b0 = min(nblocks, (i64)t * per), b1 = min(nblocks, b0 + per);
-  int ni = 0;
-  for (i64 b = b0; b < b1; b++) ni += (first[b + 1] - first[b] + chunk - 1) / chunk;
+  const i64 b = (i64)blockIdx.x * 1024 + t;
+  const int2 r = b < nblocks ? range[b] : make_int2(0, 0);
+  const int c = r.y - r.x, ni = (c + chunk - 1) / chunk;
   int inc = ni;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -176,13 +186,26 @@ __global__ __launch_bounds__(1024) void k_lb_plan(const int *first, i64 nblocks,
   }
   if (lane == 63) s[w] = inc;
   __syncthreads();
-  int it = inc - ni;
-  for (int k = 0; k < w; k++) it += s[k];
-  for (i64 b = b0; b < b1; b++) {
-    const int f = first[b], c = first[b + 1] - f;
-    for (int k = 0; k < c; k += chunk) items[it++] = make_int4((int)b, f + k, min(chunk, c - k), 0);
+  if (t == 0) {
+    int sum = 0;
+    for (int k = 0; k < 16; k++) sum += s[k];
+    first = sum ? atomicAdd(nitems, sum) : 0;
   }
-  if (t == 1023) *nitems = it;
+  __syncthreads();
+  int at = first + inc - ni;
+  for (int k = 0; k < w; k++) at += s[k];
+  auto put = [&](int bb, int f, int n, int o, int k) {
+    items[o + k] = make_int4(bb, f + k * chunk, min(chunk, n - k * chunk), 0);
+  };
+  if (ni <= LB_OWN)
+    for (int k = 0; k < ni; k++) put((int)b, r.x, c, at, k);
+  unsigned long long many = __ballot(ni > LB_OWN);
+  for (; many; many &= many - 1) {
+    const int l = __ffsll((long long)many) - 1;
+    const int bb = __shfl((int)b, l), f = __shfl(r.x, l), n = __shfl(c, l), o = __shfl(at, l);
+    const int m = __shfl(ni, l);
+    for (int k = lane; k < m; k += 64) put(bb, f, n, o, k);
+  }
 }
 
 // LDS block of one work item: nodes [o0, o0 + L) per axis (grid indices)
@@ -501,18 +524,18 @@ static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st
   int *keys = (int *)scratch(24, 2 * sizeof(int) * (size_t)np);
   int *idxs = (int *)scratch(25, 2 * sizeof(int) * (size_t)np);
   int *hist = (int *)scratch(26, sizeof(int) * (size_t)plan.hist_ints);
-  int *first = (int *)scratch(27, sizeof(int) * (size_t)(bg.nblocks + 1));
+  int2 *range = (int2 *)scratch(27, sizeof(int2) * (size_t)bg.nblocks);
   items = (int4 *)scratch(28, sizeof(int4) * (size_t)maxitems);
   nitems = (int *)scratch(29, sizeof(int));
-  if (!keys || !idxs || !hist || !first || !items || !nitems) return false;
+  if (!keys || !idxs || !hist || !range || !items || !nitems) return false;
   int *key[2] = {keys, keys + np}, *idx[2] = {idxs, idxs + np};
-  hipLaunchKernelGGL((k_lb_keys<B, MID>), dim3(grid1d(np, 256)), dim3(256), 0, st, a, bg, keys);
+  hipLaunchKernelGGL((k_lb_keys<B, MID>), dim3(grid1d(std::max(np, bg.nblocks), 256)), dim3(256), 0,
+                     st, a, bg, keys, range, nitems);
   const int at = radix_sort(plan, key, idx, hist, st);
   perm = idx[at];
-  hipLaunchKernelGGL(k_lb_first, dim3(grid1d(np + 1, 256)), dim3(256), 0, st, np, key[at],
-                     bg.nblocks, first);
-  hipLaunchKernelGGL(k_lb_plan, dim3(1), dim3(1024), 0, st, first, bg.nblocks, chunk, items,
-                     nitems);
+  hipLaunchKernelGGL(k_lb_ranges, dim3(grid1d(np, 256)), dim3(256), 0, st, np, key[at], range);
+  hipLaunchKernelGGL(k_lb_plan, dim3(grid1d(bg.nblocks, 1024)), dim3(1024), 0, st, range,
+                     bg.nblocks, chunk, items, nitems);
   return true;
 }
 
