@@ -110,16 +110,10 @@ struct LbGather {
   double *rec;
 };
 
-// Block of every particle, by the node of its position (MID: of its
-// position half a step back, where the direct current is deposited); clears
-// the blocks' ranges and the number of work items.
+// Block of particle ip, by the node of its position (MID: of its position
+// half a step back, where the direct current is deposited).
 template <int B, bool MID>
-__global__ __launch_bounds__(256) void k_lb_keys(LbPos a, BinGeom bg, int *key, int2 *range,
-                                                 int *nitems) {
-  const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (ip == 0) *nitems = 0;
-  if (ip < bg.nblocks) range[ip] = make_int2(0, 0);
-  if (ip >= a.np) return;
+PXR_DEV int lb_key(const LbPos &a, const BinGeom &bg, i64 ip) {
   double x = a.x[ip], y = a.y[ip], z = a.z[ip];
   const bool pack = a.packed.on();
   double ux = 0.0, uy = 0.0, uz = 0.0, gi = 0.0;
@@ -147,9 +141,44 @@ __global__ __launch_bounds__(256) void k_lb_keys(LbPos a, BinGeom bg, int *key, 
     a.rec[6 * ip + 1] = y;
     a.rec[6 * ip + 2] = z;
   }
-  key[ip] = block_axis<B>(x, bg.gd[0], bg.na[0]) +
-            bg.nb[0] * (block_axis<B>(y, bg.gd[1], bg.na[1]) +
-                        bg.nb[1] * block_axis<B>(z, bg.gd[2], bg.na[2]));
+  return block_axis<B>(x, bg.gd[0], bg.na[0]) +
+         bg.nb[0] * (block_axis<B>(y, bg.gd[1], bg.na[1]) +
+                     bg.nb[1] * block_axis<B>(z, bg.gd[2], bg.na[2]));
+}
+
+// keys; clears the blocks' ranges and the number of work items
+template <int B, bool MID>
+__global__ __launch_bounds__(256) void k_lb_keys(LbPos a, BinGeom bg, int *key, int2 *range,
+                                                 int *nitems) {
+  const i64 ip = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (ip == 0) *nitems = 0;
+  if (range && ip < bg.nblocks) range[ip] = make_int2(0, 0);
+  if (ip < a.np) key[ip] = lb_key<B, MID>(a, bg, ip);
+}
+
+// The same for a set that one pass of the radix sort orders, with the digit
+// counts of that pass (k_rx_count).  A small call is a chain of short launches:
+// this one less, none for the blocks' ranges and one for the scan of few
+// counts take the charge density of 66,000 particles in cell order on 32^3
+// cells from 61 to 39 us at order 1, the Esirkepov current from 62 to 41 (100,000:
+// 61 and 60 -> 43 and 45; 400,000 on 64^3 67 and 82 -> 58 and 74).
+template <int B, bool MID>
+__global__ __launch_bounds__(256) void k_lb_keys_count(LbPos a, BinGeom bg, int *key, i64 seg,
+                                                       int bits, int *hist, int *nitems) {
+  __shared__ int cnt[1 << RX_BITS];
+  const int nd = 1 << bits;
+  for (int d = threadIdx.x; d < nd; d += 256) cnt[d] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *nitems = 0;
+  __syncthreads();
+  const i64 b0 = (i64)blockIdx.x * 4 * seg, b1 = min(a.np, b0 + 4 * seg);
+#pragma unroll 4
+  for (i64 ip = b0 + threadIdx.x; ip < b1; ip += 256) {
+    const int k = lb_key<B, MID>(a, bg, ip);
+    key[ip] = k;
+    atomicAdd(&cnt[k], 1);
+  }
+  __syncthreads();
+  for (int d = threadIdx.x; d < nd; d += 256) hist[(i64)d * gridDim.x + blockIdx.x] = cnt[d];
 }
 
 // The sorted particles of each block that has any: the first of a run of
@@ -164,6 +193,18 @@ __global__ __launch_bounds__(256) void k_lb_ranges(i64 np, const int *key, int2 
   if (j == np - 1 || key[j + 1] != k) range[k].y = (int)j + 1;
 }
 
+// Where the sorted particles of a block lie: the ranges, or, after a sort in
+// one pass, its scanned digit counts (those of a digit's first radix block).
+struct BlockRanges {
+  const int2 *range;  // or null
+  const int *hist;
+  int stride, nd, np;
+  PXR_DEV int2 of(i64 b) const {
+    if (range) return range[b];
+    return make_int2(hist[b * stride], b + 1 < nd ? hist[(b + 1) * stride] : np);
+  }
+};
+
 // The work items (block, first slot, count) of at most `chunk` particles of
 // one block, a thread per block.  Their order is that of the blocks inside a
 // workgroup, and between workgroups that of their adds to *nitems.  A block of
@@ -171,12 +212,12 @@ __global__ __launch_bounds__(256) void k_lb_ranges(i64 np, const int *key, int2 
 // one block are 16,000 items).
 constexpr int LB_OWN = 8;
 
-__global__ __launch_bounds__(1024) void k_lb_plan(const int2 *range, i64 nblocks, int chunk,
+__global__ __launch_bounds__(1024) void k_lb_plan(BlockRanges br, i64 nblocks, int chunk,
                                                   int4 *items, int *nitems) {
   __shared__ int s[16], first;
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const i64 b = (i64)blockIdx.x * 1024 + t;
-  const int2 r = b < nblocks ? range[b] : make_int2(0, 0);
+  const int2 r = b < nblocks ? br.of(b) : make_int2(0, 0);
   const int c = r.y - r.x, ni = (c + chunk - 1) / chunk;
   int inc = ni;
 #pragma unroll
@@ -512,6 +553,11 @@ __global__ __launch_bounds__(1024) void k_lb_probe(LbPos a, BinGeom bg, int *out
 // with global atomics on the blocks' counters took 0.32 ms for two million
 // in random order (every particle its own atomic), this 0.09 ms.  Returns false,
 // with nothing launched, for a set it has no memory or index range for.
+// Particles below which keys and counts take one launch: the radix sort's
+// blocks are of 1024 there, four a thread; of 4096 the key pass would have too
+// few waves in flight.
+constexpr i64 LB_COUNTED = 1 << 19;
+
 template <int B, bool MID>
 static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st, BinGeom &bg,
                     int *&perm, int4 *&items, int *&nitems, i64 &maxitems) {
@@ -524,18 +570,27 @@ static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st
   int *keys = (int *)scratch(24, 2 * sizeof(int) * (size_t)np);
   int *idxs = (int *)scratch(25, 2 * sizeof(int) * (size_t)np);
   int *hist = (int *)scratch(26, sizeof(int) * (size_t)plan.hist_ints);
-  int2 *range = (int2 *)scratch(27, sizeof(int2) * (size_t)bg.nblocks);
+  // one pass of the sort: its counts say where the blocks lie
+  const bool one = plan.npass == 1;
+  int2 *range = one ? nullptr : (int2 *)scratch(27, sizeof(int2) * (size_t)bg.nblocks);
   items = (int4 *)scratch(28, sizeof(int4) * (size_t)maxitems);
   nitems = (int *)scratch(29, sizeof(int));
-  if (!keys || !idxs || !hist || !range || !items || !nitems) return false;
+  if (!keys || !idxs || !hist || !(one || range) || !items || !nitems) return false;
   int *key[2] = {keys, keys + np}, *idx[2] = {idxs, idxs + np};
-  hipLaunchKernelGGL((k_lb_keys<B, MID>), dim3(grid1d(std::max(np, bg.nblocks), 256)), dim3(256), 0,
-                     st, a, bg, keys, range, nitems);
-  const int at = radix_sort(plan, key, idx, hist, st);
+  const bool counted = one && np < LB_COUNTED;
+  if (counted)
+    hipLaunchKernelGGL((k_lb_keys_count<B, MID>), dim3((unsigned)plan.nblk), dim3(256), 0, st, a,
+                       bg, keys, plan.seg, plan.bits, hist, nitems);
+  else
+    hipLaunchKernelGGL((k_lb_keys<B, MID>), dim3(grid1d(std::max(np, bg.nblocks), 256)), dim3(256),
+                       0, st, a, bg, keys, range, nitems);
+  const int at = radix_sort(plan, key, idx, hist, st, counted);
   perm = idx[at];
-  hipLaunchKernelGGL(k_lb_ranges, dim3(grid1d(np, 256)), dim3(256), 0, st, np, key[at], range);
-  hipLaunchKernelGGL(k_lb_plan, dim3(grid1d(bg.nblocks, 1024)), dim3(1024), 0, st, range,
-                     bg.nblocks, chunk, items, nitems);
+  if (!one)
+    hipLaunchKernelGGL(k_lb_ranges, dim3(grid1d(np, 256)), dim3(256), 0, st, np, key[at], range);
+  const BlockRanges br{range, hist, plan.nblk, 1 << plan.bits, (int)np};
+  hipLaunchKernelGGL(k_lb_plan, dim3(grid1d(bg.nblocks, 1024)), dim3(1024), 0, st, br, bg.nblocks,
+                     chunk, items, nitems);
   return true;
 }
 

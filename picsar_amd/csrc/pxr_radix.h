@@ -7,6 +7,8 @@
 
 namespace pxr {
 
+constexpr int RX_BITS = 11;  // widest digit
+
 // How n keys below nkeys are sorted: npass least-significant-digit passes
 // of `bits` bits, each over nblk blocks of 4 * seg items (a wave owns seg
 // consecutive ones).
@@ -23,7 +25,10 @@ RadixPlan radix_plan(i64 n, i64 nkeys, i64 hist_cap);
 // Sorts on stream st.  key[0] holds the keys (all in [0, nkeys)); key[1],
 // idx[0] and idx[1] are n ints each, hist plan.hist_ints.  Returns which of
 // the two buffers holds the sorted keys and, in key order and in increasing
-// order within a key, the indices 0..n-1.
-int radix_sort(const RadixPlan &p, int *const *key, int *const *idx, int *hist, hipStream_t st);
+// order within a key, the indices 0..n-1.  After a single pass hist[d * p.nblk]
+// is the number of keys below d.  counted: the caller has left the first
+// pass's digit counts of every block in hist (as k_rx_count does).
+int radix_sort(const RadixPlan &p, int *const *key, int *const *idx, int *hist, hipStream_t st,
+               bool counted = false);
 
 }  // namespace pxr

@@ -13,7 +13,6 @@
 
 namespace pxr {
 
-constexpr int RX_BITS = 11;      // widest digit
 // Items of a block (a cap on the histogram makes it more).  Few items want
 // more blocks than 4096 a block give: 100,000 particles in 24^3 cells 127 ->
 // 103 us (the whole leaf sort); from half a million on, the histogram costs
@@ -68,7 +67,7 @@ __global__ __launch_bounds__(256) void k_rx_sums(const int *hist, i64 m, int *bs
 }
 
 // exclusive scan in place: every block sums the blocks before it itself
-// (at most a few hundred), which saves a launch
+// (at most 1023), which saves a launch
 __global__ __launch_bounds__(256) void k_rx_scan(int *hist, i64 m, const int *bsum) {
   constexpr int PER = RX_SCAN / 256;
   __shared__ int s[4], before[4];
@@ -98,6 +97,37 @@ __global__ __launch_bounds__(256) void k_rx_scan(int *hist, i64 m, const int *bs
 #pragma unroll
   for (int k = 0; k < PER; k++) {
     if (b0 + k < m) hist[b0 + k] = run;
+    run += v[k];
+  }
+}
+
+// the same for few counts, by one workgroup in one launch
+constexpr int RX_SCAN_ONE = 16384;
+
+__global__ __launch_bounds__(1024) void k_rx_scan_one(int *hist, int m) {
+  constexpr int PER = RX_SCAN_ONE / 1024;
+  __shared__ int s[16];
+  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6;
+  const int per = min(PER, (m + 1023) / 1024);
+  int v[PER], sum = 0;
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    v[k] = k < per && t * per + k < m ? hist[t * per + k] : 0;
+    sum += v[k];
+  }
+  int run = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(run, off);
+    if (lane >= off) run += y;
+  }
+  if (lane == 63) s[w] = run;
+  run -= sum;
+  __syncthreads();
+  for (int k = 0; k < w; k++) run += s[k];
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    if (k < per && t * per + k < m) hist[t * per + k] = run;
     run += v[k];
   }
 }
@@ -151,7 +181,8 @@ __global__ __launch_bounds__(256) void k_rx_scatter(const int *key, const int *i
   }
 }
 
-int radix_sort(const RadixPlan &p, int *const *key, int *const *idx, int *hist, hipStream_t st) {
+int radix_sort(const RadixPlan &p, int *const *key, int *const *idx, int *hist, hipStream_t st,
+               bool counted) {
   const i64 m = (i64)p.nblk << p.bits;
   const unsigned nsum = (unsigned)((m + RX_SCAN - 1) / RX_SCAN);
   int *bsum = hist + m;
@@ -160,9 +191,14 @@ int radix_sort(const RadixPlan &p, int *const *key, int *const *idx, int *hist, 
   int at = 0;
   for (int pass = 0; pass < p.npass; pass++, at ^= 1) {
     const int shift = pass * p.bits;
-    hipLaunchKernelGGL(k_rx_count, grd, blk, 0, st, key[at], p.n, p.seg, shift, p.bits, hist);
-    hipLaunchKernelGGL(k_rx_sums, dim3(nsum), blk, 0, st, hist, m, bsum);
-    hipLaunchKernelGGL(k_rx_scan, dim3(nsum), blk, 0, st, hist, m, bsum);
+    if (pass || !counted)
+      hipLaunchKernelGGL(k_rx_count, grd, blk, 0, st, key[at], p.n, p.seg, shift, p.bits, hist);
+    if (m <= RX_SCAN_ONE) {
+      hipLaunchKernelGGL(k_rx_scan_one, dim3(1), dim3(1024), 0, st, hist, (int)m);
+    } else {
+      hipLaunchKernelGGL(k_rx_sums, dim3(nsum), blk, 0, st, hist, m, bsum);
+      hipLaunchKernelGGL(k_rx_scan, dim3(nsum), blk, 0, st, hist, m, bsum);
+    }
     hipLaunchKernelGGL(k_rx_scatter, grd, blk, lds, st, key[at], pass ? idx[at] : nullptr, p.n,
                        p.seg, shift, p.bits, hist, key[at ^ 1], idx[at ^ 1]);
   }
