@@ -507,8 +507,11 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
  * direct deposition runs at most two workgroups per CU, since its kernel
  * holds registers for two waves per SIMD; it then takes 2 and 79616 bytes.
  * pxrhip_get_tuning also reads "last.wg_per_cu" and "last.lds_bytes", the
- * launch of the last pxrhip_tiles_gather_push_deposit, and
- * "device.num_cus".  Work items whose
+ * launch of the last pxrhip_tiles_gather_push_deposit, "device.num_cus", and
+ * the form of the last leaf call with one order on all axes:
+ * "last.leaf_current", "last.leaf_rho" and "last.leaf_gather" (1 block by
+ * block, 0 particle by particle) and "last.leaf_records" (1 if that current
+ * was deposited from records of the particles; synchronises).  Work items whose
  * field or current block exceeds its LDS budget are completed from global
  * memory by a second kernel (a mixed-precision species' current: through
  * an LDS block cut down to fit, see "mixed.jmargin"). */

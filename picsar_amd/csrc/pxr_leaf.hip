@@ -943,6 +943,7 @@ int pxrhip_geteb3d_energy_conserving(
   const bool lo = l_lower_order_in_v != 0;
   hipStream_t st = rt().stream;
   const bool ask = leaf_binned_gather_may_pay(a, (int)nox);
+  rt().last_leaf_gather = 0;
   LeafProbe probe;
   if (ask && (r = leaf_probe_start(a, st, probe))) return r;
   launch_gather(a, (int)nox, lo, st);
@@ -952,6 +953,7 @@ int pxrhip_geteb3d_energy_conserving(
     a.skip = nullptr;
     i64 done = np;
     if (scattered && (r = leaf_binned_gather(a, (int)nox, lo, st, done))) return r;
+    rt().last_leaf_gather = scattered && done == np;
     if (done < np) launch_gather(a.part(done, np - done), (int)nox, lo, st);
   }
   PXR_LAUNCHED();
@@ -1136,6 +1138,7 @@ int pxrhip_depose_jxjyjz(double *jx, double *jy, double *jz, int64_t np, const d
                : leaf_binned_esirkepov(a, (int)nox, st, done);
     if (r) return r;
   }
+  rt().last_leaf_current = done == np;
   if (done < np) {  // all of them, or those there was no memory to order
     const DepoArgs p = a.part(done, np - done);
     const dim3 blk(dep_block(p.np)), grd(grid1d(p.np, 64 * DEP_S) * dep_blocks(blk.x));
@@ -1203,6 +1206,7 @@ int pxrhip_depose_rho_n(double *rho, int64_t np, const double *xp, const double 
     r = leaf_binned_rho(a, (int)nox, st, done);
     if (r) return r;
   }
+  rt().last_leaf_rho = done;
   if (done) {
   } else if (nox == 1) hipLaunchKernelGGL(k_rho<1>, grd, blk, 0, st, a);
   else if (nox == 2) hipLaunchKernelGGL(k_rho<2>, grd, blk, 0, st, a);

@@ -690,9 +690,12 @@ bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order) {
          a.np >= (order == 1 ? GATHER_BIN_MIN1 : GATHER_BIN_MIN);
 }
 
-static void launch_probe(const LbPos &pos, const GridGeom &g, hipStream_t st, LeafProbe &probe) {
-  probe.host = report_slot();
-  probe.dev = (int *)(rt().d_bad + 2 + (probe.host - rt().h_report));
+// host: where the answer goes on the host (null: the probe's report slot)
+static void launch_probe(const LbPos &pos, const GridGeom &g, hipStream_t st, LeafProbe &probe,
+                         unsigned long long *host = nullptr) {
+  unsigned long long *slot = report_slot();
+  probe.host = host ? host : slot;
+  probe.dev = (int *)(rt().d_bad + 2 + (slot - rt().h_report));
   hipLaunchKernelGGL(k_lb_probe<LB_EDGE>, dim3(1), dim3(1024), 0, st, pos,
                      make_bin_geom(g, LB_EDGE), probe.dev, probe.host);
 }
@@ -776,6 +779,7 @@ static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &don
   const int chunk = std::min(rt().leaf_bin_chunk, order == 1 ? 512 : order == 2 ? 1024 : 2048);
   done = 0;
   LbDepo d;
+  rt().last_leaf_records_asked = false;
   if (records)
     d.packed.rec = (double *)scratch(30, 8 * sizeof(double) * (size_t)size);
   while (done < a.np) {
@@ -785,7 +789,8 @@ static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &don
               {0.5 * c.dtsdx0, 0.5 * c.dtsdy0, 0.5 * c.dtsdz0}, 0, nullptr, {}};
     if (d.packed.rec) {
       LeafProbe probe;
-      launch_probe(pos, a.g, st, probe);
+      launch_probe(pos, a.g, st, probe, records_word());
+      rt().last_leaf_records_asked = true;
       d.packed.use = probe.dev;
       pos.packed = d.packed;
     }

@@ -26,6 +26,11 @@ struct Runtime {
   // particles on (0: never), work items of at most leaf_bin_chunk particles
   int64_t leaf_bin_min = 1 << 16;
   int leaf_bin_chunk = 4096;
+  // form of the last large leaf call (pxrhip_get_tuning "last.leaf_*"): 1 block
+  // by block; whether its deposition could read records (the GPU decides, and
+  // writes its answer behind the report slots)
+  int last_leaf_current = 0, last_leaf_rho = 0, last_leaf_gather = 0;
+  bool last_leaf_records_asked = false;
   // incremented whenever library-owned device memory that recorded work may
   // point at is freed (a scratch slot that grows, the cached tile table):
   // a HIP graph captured before that refers to freed memory
@@ -47,6 +52,10 @@ unsigned long long *report_slot();
 int take_bad(unsigned long long *n);
 // the same for any device counter
 int take_counter(unsigned long long *ctr, unsigned long long *n, hipStream_t st);
+
+// the word after the report slots: whether the last current was deposited from
+// records
+inline unsigned long long *records_word() { return rt().h_report + REPORT_SLOTS; }
 
 inline unsigned grid1d(int64_t n, int block) {
   int64_t b = (n + block - 1) / block;

@@ -112,7 +112,7 @@ int pxrhip_init(int device) {
     g_rt.d_sort_bad = g_rt.d_bad + 1;
   }
   if (!g_rt.h_report)
-    PXR_HIP(hipHostMalloc(&g_rt.h_report, REPORT_SLOTS * sizeof(unsigned long long), 0));
+    PXR_HIP(hipHostMalloc(&g_rt.h_report, (REPORT_SLOTS + 1) * sizeof(unsigned long long), 0));
   g_rt.device = dev;
   return PXRHIP_OK;
 }

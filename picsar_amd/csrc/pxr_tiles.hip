@@ -1579,6 +1579,16 @@ int pxrhip_get_tuning(const char *key, int64_t *value) {
   else if (!strcmp(key, "last.wg_per_cu")) *value = g_last_wg_per_cu;
   else if (!strcmp(key, "device.num_cus")) *value = rt().device >= 0 ? rt().num_cus : 0;
   else if (!strcmp(key, "last.lds_bytes")) *value = g_last_lds_bytes;
+  else if (!strcmp(key, "last.leaf_current")) *value = rt().last_leaf_current;
+  else if (!strcmp(key, "last.leaf_rho")) *value = rt().last_leaf_rho;
+  else if (!strcmp(key, "last.leaf_gather")) *value = rt().last_leaf_gather;
+  else if (!strcmp(key, "last.leaf_records")) {
+    *value = 0;
+    if (rt().last_leaf_current && rt().last_leaf_records_asked) {
+      PXR_HIP(hipStreamSynchronize(rt().stream));
+      *value = *(volatile unsigned long long *)records_word() != 0;
+    }
+  }
   else return set_error(PXRHIP_ERR_ARG, "unknown tuning key '%s'", key);
   return PXRHIP_OK;
 }

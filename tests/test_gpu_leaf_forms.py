@@ -1,0 +1,99 @@
+"""Which form a large leaf call takes, as the library reports it: sets in no
+order and in cell order, sizes on both sides of each rule, sets ordered in
+several parts.  Results are compared in the tests of the forms themselves.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_leaf import NG, NX, NY, NZ, SHAPE, T, TG, particles
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    from picsar_amd import _lib
+    _lib.load()
+    _lib.call("pxrhip_init", 0)
+    return _lib
+
+
+def last(dev, what):
+    v = C.c_int64()
+    dev.call("pxrhip_get_tuning", b"last.leaf_" + what, C.byref(v))
+    return v.value
+
+
+def cell_order(x):
+    return np.lexsort(tuple(np.floor(a) for a in x))
+
+
+def plasma(dev, n, grid, ordered):
+    rng = np.random.default_rng(n)
+    x = particles(rng, n, margin=1.0) if grid is None else [rng.uniform(1, g - 1, n) for g in grid]
+    if ordered:
+        o = cell_order(x)
+        x = [a[o] for a in x]
+    u = [rng.uniform(-1.0, 1.0, n) for _ in range(3)]
+    g = 1 / np.sqrt(1 + u[0] ** 2 + u[1] ** 2 + u[2] ** 2)
+    return [T(dev, a) for a in (*x, *u, g, rng.uniform(0.5, 2.0, n))]
+
+
+def gather(dev, n, x, order, grid=(NX, NY, NZ), lower=1):
+    shape = tuple(g + 1 + 2 * NG for g in grid)
+    F = TG(dev, np.zeros(shape))
+    e = T(dev, np.zeros(n))
+    dev.call("pxrhip_geteb3d_energy_conserving", n, *[a.ptr for a in x], *[e.ptr] * 6, 0.0, 0.0,
+             0.0, 1.0, 1.0, 1.0, *grid, NG, NG, NG, order, order, order, *[F.ptr] * 6, 0, lower, 8,
+             0, 0)
+    return last(dev, b"gather")
+
+
+def current(dev, n, P, order, algo, grid=(NX, NY, NZ)):
+    J = [TG(dev, np.zeros(tuple(g + 1 + 2 * NG for g in grid))) for _ in range(3)]
+    dev.call("pxrhip_depose_jxjyjz", *[j.ptr for j in J], n, *[a.ptr for a in P], -1.1, 0.0, 0.0,
+             0.0, 0.3, 1.0, 1.0, 1.0, *grid, NG, NG, NG, order, order, order, algo, 0)
+    return last(dev, b"current"), last(dev, b"records")
+
+
+@pytest.mark.parametrize("order,n,form", [
+    (1, 3145727, 0), (1, 3145728, 1), (2, 786431, 0), (2, 786432, 1), (3, 786431, 0),
+    (3, 786432, 1), (3, 8400001, 1)])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_gather(dev, order, n, form, ordered):
+    x = plasma(dev, n, None, ordered)[:3]
+    assert gather(dev, n, x, order) == (0 if ordered else form)
+
+
+@pytest.mark.parametrize("exchanged,form", [(20, 0), (900000, 1)])
+def test_gather_of_a_set_losing_its_order(dev, exchanged, form):
+    """a few particles exchanged, and most of them"""
+    n = 900000
+    rng = np.random.default_rng(exchanged)
+    x = particles(rng, n, margin=1.0)
+    o = cell_order(x)
+    i = rng.permutation(n)[:exchanged]
+    o[i] = o[np.roll(i, 1)]
+    assert gather(dev, n, [T(dev, a[o]) for a in x], 3) == form
+
+
+@pytest.mark.parametrize("algo", [0, 3])
+@pytest.mark.parametrize("order,n,records", [
+    (1, 524287, 0), (1, 524288, 1), (2, 524288, 1), (2, 8388609, 1), (3, 524288, 0)])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_records(dev, order, n, records, algo, ordered):
+    P = plasma(dev, n, None, ordered)
+    assert current(dev, n, P, order, algo) == (1, 0 if ordered else records)
+
+
+@pytest.mark.parametrize("n,form", [(65535, 0), (65536, 1)])
+def test_depositions(dev, n, form):
+    P = plasma(dev, n, None, False)
+    for algo in (0, 3):
+        assert current(dev, n, P, 1, algo) == (form, 0)
+    r = TG(dev, np.zeros(SHAPE))
+    dev.call("pxrhip_depose_rho_n", r.ptr, n, *[P[k].ptr for k in (0, 1, 2, 7)], -1.1, 0.0, 0.0,
+             0.0, 1.0, 1.0, 1.0, NX, NY, NZ, NG, NG, NG, 1, 1, 1, 1, 0)
+    assert last(dev, b"rho") == form
