@@ -628,10 +628,21 @@ constexpr int LB_EDGE = 8;  // nodes per block edge
 // call in cell order 4 to 8 us, so it has to be a small part of the call.  A
 // million on 64^3 cells: order 3 151 -> 155 us in cell order and 618 -> 293 in
 // random order, order 2 106 -> 109 and 428 -> 227 (600000 on 48^3, order 2:
-// 180 -> 187).  At order 1 a particle's eight-node reads are as fast as
-// ordering it until the fields leave the L2: two million on 64^3 360 -> 347
-// us, four million on 128^3 1020 -> 741 (153 -> 160 in cell order).
+// 180 -> 187).  At order 1, where a particle reads eight nodes of a field, the
+// staged form gains little on a small grid: one, two and four million on 64^3
+// 170 -> 175, 324 -> 293 and 650 -> 580 us (four million on 128^3 995 -> 692).
 constexpr i64 GATHER_BIN_MIN1 = 3 << 20, GATHER_BIN_MIN = 3 << 18;
+// And particles per block of the grid: a block's six fields are staged whole,
+// 1331 nodes or more each, however few particles read them.  Random order,
+// plain -> staged at about this many per block and at half of it:
+// order 1: four million on 200^3 (228) 1037 -> 896 us, eight on 256^3 (223)
+// 2040 -> 1800; two on 200^3 (114) 530 -> 601, four on 256^3 (111) 1042 -> 1195;
+// order 2: one on 200^3 (57) 749 -> 614, two on 256^3 (56) 1473 -> 1162; four
+// on 384^3 (34) 3450 -> 3464, one on 256^3 (28) 756 -> 1041;
+// order 3: one on 256^3 (28) 1518 -> 1222, eight on 512^3 (29) 14101 -> 9257;
+// two on 384^3 (17) 3234 -> 3828, four on 512^3 (15) 7014 -> 8710.
+// (A million on 512^3, 3.6 a block: 356 -> 5191, 917 -> 6589, 1747 -> 7976.)
+constexpr int GATHER_PER_BLOCK[4] = {0, 192, 48, 24};
 constexpr i64 DEPO_REC_MIN = 1 << 19;  // a million random: 236 -> 164 us (Esirkepov, order 1)
 constexpr int GATHER_CHUNK = 1024;  // particles of a gather's work item
 
@@ -686,8 +697,9 @@ LeafGatherArgs LeafGatherArgs::part(i64 first, i64 n) const {
 }
 
 bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order) {
-  return rt().checks && pays(a.np, a.g, LB_EDGE) &&
-         a.np >= (order == 1 ? GATHER_BIN_MIN1 : GATHER_BIN_MIN);
+  return rt().checks && a.np >= (order == 1 ? GATHER_BIN_MIN1 : GATHER_BIN_MIN) &&
+         a.np >= GATHER_PER_BLOCK[order] * make_bin_geom(a.g, LB_EDGE).nblocks &&
+         pays(a.np, a.g, LB_EDGE);
 }
 
 // host: where the answer goes on the host (null: the probe's report slot)

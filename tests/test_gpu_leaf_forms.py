@@ -97,3 +97,15 @@ def test_depositions(dev, n, form):
     dev.call("pxrhip_depose_rho_n", r.ptr, n, *[P[k].ptr for k in (0, 1, 2, 7)], -1.1, 0.0, 0.0,
              0.0, 1.0, 1.0, 1.0, NX, NY, NZ, NG, NG, NG, 1, 1, 1, 1, 0)
     assert last(dev, b"rho") == form
+
+
+@pytest.mark.parametrize("order,grid,n,form", [
+    # 26^3 = 17576, 35^3 = 42875 and 65 x 65 x 9 = 38025 blocks
+    (1, (200, 200, 200), 192 * 17576 - 1, 0), (1, (200, 200, 200), 192 * 17576, 1),
+    (2, (200, 200, 200), 48 * 17576 - 1, 0), (2, (200, 200, 200), 48 * 17576, 1),
+    (3, (270, 270, 270), 24 * 42875 - 1, 0), (3, (270, 270, 270), 24 * 42875, 1),
+    (3, (512, 512, 64), 24 * 38025 - 1, 0), (3, (512, 512, 64), 24 * 38025, 1)])
+def test_gather_on_a_sparse_grid(dev, order, grid, n, form):
+    """the blocks' fields are staged only where enough particles read them"""
+    rng = np.random.default_rng(n)
+    assert gather(dev, n, [T(dev, rng.uniform(1, g - 1, n)) for g in grid], order, grid) == form
