@@ -497,9 +497,10 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
  * pxrhip_depose_rho_n sum calls of at least this many particles, and one per
  * 8^3-node block of the arrays, block by block in LDS; default 65536, 0:
  * never, nor does pxrhip_geteb3d_energy_conserving then gather large sets
- * in no order block by block) and "leaf.bin_chunk" (largest work item of
- * that form, default 4096 particles; the currents and the gather take
- * smaller ones by themselves, 512 to 2048).
+ * in no order block by block) and "leaf.bin_chunk" (particles of the largest
+ * work item of that form, 1 to 2^20; up to the default, 4096, the routines
+ * take smaller ones by themselves, 512 to 2048, a larger value is taken as it
+ * is).
  * wg_per_cu 0 (the default) is automatic: three workgroups per CU with
  * 52224 bytes each when a work item of four sorting rows of the widest tile
  * fits that, else two with 79616 bytes; a wg_per_cu above 0 takes the
@@ -511,7 +512,9 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
  * the form of the last leaf call with one order on all axes:
  * "last.leaf_current", "last.leaf_rho" and "last.leaf_gather" (1 block by
  * block, 0 particle by particle) and "last.leaf_records" (1 if that current
- * was deposited from records of the particles; synchronises).  Work items whose
+ * was deposited from records of the particles; synchronises), and
+ * "last.leaf_items" the work items of the last call (or part of a call) that
+ * went block by block (synchronises).  Work items whose
  * field or current block exceeds its LDS budget are completed from global
  * memory by a second kernel (a mixed-precision species' current: through
  * an LDS block cut down to fit, see "mixed.jmargin"). */

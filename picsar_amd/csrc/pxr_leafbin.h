@@ -87,6 +87,8 @@ struct LeafProbe {
 };
 int leaf_probe_start(LeafGatherArgs &a, hipStream_t st, LeafProbe &probe);
 int leaf_probe_read(LeafProbe &probe, bool &scattered);
+// work items of the last call, or part of one, that went block by block
+int leaf_last_items(int64_t *n);
 int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st, i64 &done);
 
 }  // namespace pxr

@@ -676,6 +676,21 @@ static bool pays(i64 np, const GridGeom &g, int edge) {
          !recording(r.stream);
 }
 
+// Particles of a work item, of which the routine would take `own`.
+static int item_size(int own) {
+  const int most = rt().leaf_bin_chunk;
+  return most > LEAF_BIN_CHUNK ? most : std::min(most, own);
+}
+
+int leaf_last_items(int64_t *n) {
+  int *nitems = (int *)scratch(29, sizeof(int)), v = 0;
+  if (!nitems) return set_error(PXRHIP_ERR_HIP, "scratch allocation failed");
+  PXR_HIP(hipStreamSynchronize(rt().stream));
+  PXR_HIP(hipMemcpy(&v, nitems, sizeof(int), hipMemcpyDeviceToHost));
+  *n = v;
+  return PXRHIP_OK;
+}
+
 static LbPos gather_pos(const LeafGatherArgs &a, double *rec) {
   return LbPos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, nullptr, a.xmin, a.ymin,
                a.zmin, a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, 0, rec, {}};
@@ -751,7 +766,7 @@ int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream
     int4 *items;
     i64 maxitems;
     if (!lb_sort<LB_EDGE, false>(gather_pos(ga.c, ga.rec), a.g,
-                                 std::min(rt().leaf_bin_chunk, GATHER_CHUNK), st, bg, perm, items,
+                                 item_size(GATHER_CHUNK), st, bg, perm, items,
                                  nitems, maxitems))
       return PXRHIP_OK;
     const dim3 grd(lb_grid(maxitems, lds)), blk(512);
@@ -788,7 +803,7 @@ static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &don
   // smaller work items, until clearing and adding up the LDS blocks costs as
   // much.  Two million in cell order on 64^3 cells, 4096 particles an item and
   // so: order 1 374 -> 177 us, order 2 402 -> 255, order 3 446 -> 410.
-  const int chunk = std::min(rt().leaf_bin_chunk, order == 1 ? 512 : order == 2 ? 1024 : 2048);
+  const int chunk = item_size(order == 1 ? 512 : order == 2 ? 1024 : 2048);
   done = 0;
   LbDepo d;
   rt().last_leaf_records_asked = false;
@@ -849,7 +864,7 @@ int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done) {
   // work items as for the currents: 33.6 million in cell order on 128^3 cells,
   // 4096 particles an item and so, 3.46 -> 1.58, 3.44 -> 1.83 and 3.47 -> 2.85
   // ms at orders 1 to 3
-  const int chunk = std::min(rt().leaf_bin_chunk, order == 3 ? 2048 : 1024);
+  const int chunk = item_size(order == 3 ? 2048 : 1024);
   if (!lb_sort<E, false>(pos, a.g, chunk, st, bg, perm, items, nitems, maxitems))
     return PXRHIP_OK;
   const int L = E + (order == 1 ? 1 : 3);

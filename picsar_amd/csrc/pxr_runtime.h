@@ -10,6 +10,7 @@
 namespace pxr {
 
 constexpr int REPORT_SLOTS = 256;
+constexpr int LEAF_BIN_CHUNK = 4096;
 
 struct Runtime {
   int device = -1;
@@ -23,9 +24,11 @@ struct Runtime {
   unsigned long long *h_report = nullptr;  // pinned host memory, see report_slot
   int num_cus = 256;
   // leaf deposition summed in LDS blocks (pxr_leafbin.hip) from this many
-  // particles on (0: never), work items of at most leaf_bin_chunk particles
+  // particles on (0: never), in work items of at most leaf_bin_chunk particles;
+  // up to LEAF_BIN_CHUNK the routines take smaller ones by themselves, a larger
+  // value is taken as it is
   int64_t leaf_bin_min = 1 << 16;
-  int leaf_bin_chunk = 4096;
+  int leaf_bin_chunk = LEAF_BIN_CHUNK;
   // form of the last large leaf call (pxrhip_get_tuning "last.leaf_*"): 1 block
   // by block; whether its deposition could read records (the GPU decides, and
   // writes its answer behind the report slots)

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "pxr_device.h"
+#include "pxr_leafbin.h"
 #include "pxr_fused.h"
 #include "pxr_kernels.h"
 #include "pxr_runtime.h"
@@ -1582,7 +1583,11 @@ int pxrhip_get_tuning(const char *key, int64_t *value) {
   else if (!strcmp(key, "last.leaf_current")) *value = rt().last_leaf_current;
   else if (!strcmp(key, "last.leaf_rho")) *value = rt().last_leaf_rho;
   else if (!strcmp(key, "last.leaf_gather")) *value = rt().last_leaf_gather;
-  else if (!strcmp(key, "last.leaf_records")) {
+  else if (!strcmp(key, "last.leaf_items")) {
+    *value = 0;
+    if (rt().last_leaf_current || rt().last_leaf_rho || rt().last_leaf_gather)
+      return leaf_last_items(value);
+  } else if (!strcmp(key, "last.leaf_records")) {
     *value = 0;
     if (rt().last_leaf_current && rt().last_leaf_records_asked) {
       PXR_HIP(hipStreamSynchronize(rt().stream));

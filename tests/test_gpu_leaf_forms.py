@@ -109,3 +109,31 @@ def test_gather_on_a_sparse_grid(dev, order, grid, n, form):
     """the blocks' fields are staged only where enough particles read them"""
     rng = np.random.default_rng(n)
     assert gather(dev, n, [T(dev, rng.uniform(1, g - 1, n)) for g in grid], order, grid) == form
+
+
+def block_counts(x, grid):
+    b = [(np.floor(a).astype(int) + NG) // 8 for a in x]
+    nb = [-(-(g + 1 + 2 * NG) // 8) for g in grid]
+    return np.bincount(b[0] + nb[0] * (b[1] + nb[1] * b[2]))
+
+
+@pytest.mark.parametrize("chunk", [1, 100, 512, 4096, 4097, 30000, 1 << 20])
+def test_work_items(dev, chunk):
+    """leaf.bin_chunk bounds the work items and, above its default, sets them"""
+    n, grid = 70001, (NX, NY, NZ)
+    rng = np.random.default_rng(chunk)
+    x = particles(rng, n, margin=1.0)
+    x[0][: n // 2] = rng.uniform(6, 10, n // 2)
+    P = [T(dev, a) for a in (*x, *np.zeros((3, n)), np.ones(n), np.ones(n))]
+    c = block_counts(x, grid)
+    old = C.c_int64()
+    dev.call("pxrhip_get_tuning", b"leaf.bin_chunk", C.byref(old))
+    assert old.value == 4096
+    try:
+        dev.call("pxrhip_set_tuning", b"leaf.bin_chunk", chunk)
+        for order, algo, own in ((1, 0, 512), (2, 3, 1024), (3, 0, 2048)):
+            assert current(dev, n, P, order, algo) == (1, 0)
+            size = chunk if chunk > 4096 else min(chunk, own)
+            assert last(dev, b"items") == (-(-c // size)).sum()
+    finally:
+        dev.call("pxrhip_set_tuning", b"leaf.bin_chunk", old.value)
