@@ -301,14 +301,42 @@ PXR_DEV void lb_flush(const LdsBlock &blk, const GridGeom &g, double *const *dst
   }
 }
 
-// Lanes take particles S = ceil(n / 256) apart, so that in cell-ordered
-// input the lanes of a wave sit in different cells.
+// A thread of 256 takes S = ceil(n / 256) consecutive particles of a work item
+// in turn, lanes S apart, so that in cell-ordered input the lanes of a wave sit
+// in different cells.
 PXR_DEV int lb_stride(int n) { return (n + (int)blockDim.x - 1) / (int)blockDim.x; }
+
+// The first of them.  At order 3, whose adds at one address cost the most, S
+// apart is too near in the small work items of dense sets in cell order: where
+// LB_RUN particles on the caller's order has not changed yet (a block's row of
+// eight cells with 12 or more particles each), the lanes of a wave spread over
+// the whole item, 4 S apart, and the four waves share what lies between.
+// Esirkepov current and charge density with items of 4096 as they were once, of
+// 2048, and so (us): sixteen million on 64^3 cells 3757 and 1722, 6212 and 2876,
+// 2248 and 1152; four million 755 and 408, 701 and 358, 609 and 309; a bunch of
+// four million, up to 1200 a cell, 2650 and 1300, 2912 and 1353, 2176 and 1049.
+// (At 8 a cell it loses, sixteen million on 128^3 2306 -> 2425 us, and in no
+// order, where it scatters the reads of perm: eight million on 64^3 1534 ->
+// 1702.)
+constexpr int LB_RUN = 48;
+
+template <int N> PXR_DEV int lb_first(const int *perm, int n, int S) {
+  const int t = threadIdx.x, lane = t & 63;
+  if (N == 3 && n > 256) {
+    const int p = lane * 4 * S;  // (every wave finds the same)
+    const bool run = p + LB_RUN < n && perm[p + LB_RUN] == perm[p] + LB_RUN;
+    if (__popcll(__ballot(run)) >= 32) return p + (t >> 6) * S;
+  }
+  return t * S;
+}
 
 // Esirkepov current: the box of an order-N particle lies within
 // [floor(x) - 2, floor(x) + 3] (order 1: [-1, +2]) on each axis.
+// (Order 3 at three waves per SIMD, the three workgroups that fit the LDS: two
+// registers more and it runs two, 1512 -> 1655 us for eight million particles
+// in no order on 64^3 cells.)
 template <int N, int B>
-__global__ __launch_bounds__(256) void k_lb_esirkepov(LbDepo d, BinGeom bg, const int *perm,
+__global__ __launch_bounds__(256, N == 3 ? 3 : 1) void k_lb_esirkepov(LbDepo d, BinGeom bg, const int *perm,
                                                       const int4 *items, const int *nitems) {
   const DepoArgs &a = d.c;
   const bool rec = d.packed.on();
@@ -323,9 +351,9 @@ __global__ __launch_bounds__(256) void k_lb_esirkepov(LbDepo d, BinGeom bg, cons
   LdsBlock blk;
   lb_block<B, HLO, HHI>(bg, it.x, blk, lds, 3);
   const LdsAccB acc{lds, blk.o[0], blk.o[1], blk.o[2], blk.L, blk.L * blk.L, blk.nodes};
-  const int n = it.z, S = lb_stride(n);
+  const int n = it.z, S = lb_stride(n), first = lb_first<N>(perm + it.y, n, S);
   for (int k = 0; k < S; k++) {
-    const int p = (int)threadIdx.x * S + k;
+    const int p = first + k;
     if (p >= n) break;
     const Particle8 q = load8(a, d.packed, rec, perm[it.y + p]);
     EsirkepovIn<double> in;
@@ -367,9 +395,9 @@ __global__ __launch_bounds__(256) void k_lb_direct(LbDepo d, BinGeom bg, const i
     LdsBlock blk;
     lb_block<B, HLO, HHI>(bg, it.x, blk, lds, 3);
     const LdsAccB acc{lds, blk.o[0], blk.o[1], blk.o[2], blk.L, blk.L * blk.L, blk.nodes};
-    const int n = it.z, S = lb_stride(n);
+    const int n = it.z, S = lb_stride(n), first = lb_first<N>(perm + it.y, n, S);
     for (int k = 0; k < S; k++) {
-      const int p = (int)threadIdx.x * S + k;
+      const int p = first + k;
       if (p >= n) break;
       const Particle8 q = load8(a, d.packed, rec, perm[it.y + p]);
       DirectIn<double> in;
@@ -401,9 +429,9 @@ __global__ __launch_bounds__(256) void k_lb_rho(RhoArgs a, BinGeom bg, const int
   LdsBlock blk;
   lb_block<B, HLO, HHI>(bg, it.x, blk, lds, 1);
   const int L = blk.L;
-  const int n = it.z, S = lb_stride(n);
+  const int n = it.z, S = lb_stride(n), first = lb_first<N>(perm + it.y, n, S);
   for (int k = 0; k < S; k++) {
-    const int p = (int)threadIdx.x * S + k;
+    const int p = first + k;
     if (p >= n) break;
     const i64 ip = perm[it.y + p];
     double x = (a.xp[ip] - a.xmin) * a.dxi, y = (a.yp[ip] - a.ymin) * a.dyi;
