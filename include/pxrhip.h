@@ -495,7 +495,8 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
  * keeps the source order inside a cell; 0: the order in which the GPU's
  * waves arrive), "leaf.bin_min" (pxrhip_depose_jxjyjz and
  * pxrhip_depose_rho_n sum calls of at least this many particles, and one per
- * 8^3-node block of the arrays, block by block in LDS; default 65536, 0:
+ * 8^3-node block of the arrays (eight for the direct current), block by block
+ * in LDS; default 65536, 0:
  * never, nor does pxrhip_geteb3d_energy_conserving then gather large sets
  * in no order block by block) and "leaf.bin_chunk" (particles of the largest
  * work item of that form, 1 to 2^20; up to the default, 4096, the routines

@@ -1133,7 +1133,7 @@ int pxrhip_depose_jxjyjz(double *jx, double *jy, double *jz, int64_t np, const d
   hipStream_t st = rt().stream;
   const bool direct = current_depo_algo >= 2;  // depose_jxjyjz_generic CASE(2), CASE(3)
   i64 done = 0;
-  if (leaf_binned_current_pays(np, a.g)) {
+  if (leaf_binned_current_pays(np, a.g, direct)) {
     r = direct ? leaf_binned_direct(a, (int)nox, st, done)
                : leaf_binned_esirkepov(a, (int)nox, st, done);
     if (r) return r;

@@ -64,9 +64,9 @@ int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, i64 &don
 int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, i64 &done);
 int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done);
 // whether a call of np particles on grid g takes the binned form: at least
-// the runtime's leaf_bin_min particles and one per block, and no graph
-// capture open (the scratch may have to grow)
-bool leaf_binned_current_pays(i64 np, const GridGeom &g);
+// the runtime's leaf_bin_min particles and one per block (eight for the direct
+// current), and no graph capture open (the scratch may have to grow)
+bool leaf_binned_current_pays(i64 np, const GridGeom &g, bool direct);
 bool leaf_binned_rho_pays(i64 np, const GridGeom &g);
 
 // The gather of a set in no order: particles ordered by blocks, the block's

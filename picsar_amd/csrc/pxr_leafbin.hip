@@ -698,10 +698,10 @@ static bool recording(hipStream_t st) {
   return s != hipStreamCaptureStatusNone;
 }
 
-static bool pays(i64 np, const GridGeom &g, int edge) {
+static bool pays(i64 np, const GridGeom &g, int per_block) {
   const Runtime &r = rt();
-  return r.leaf_bin_min > 0 && np >= r.leaf_bin_min && np >= make_bin_geom(g, edge).nblocks &&
-         !recording(r.stream);
+  return r.leaf_bin_min > 0 && np >= r.leaf_bin_min &&
+         np >= per_block * make_bin_geom(g, LB_EDGE).nblocks && !recording(r.stream);
 }
 
 // Particles of a work item, of which the routine would take `own`.
@@ -741,8 +741,7 @@ LeafGatherArgs LeafGatherArgs::part(i64 first, i64 n) const {
 
 bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order) {
   return rt().checks && a.np >= (order == 1 ? GATHER_BIN_MIN1 : GATHER_BIN_MIN) &&
-         a.np >= GATHER_PER_BLOCK[order] * make_bin_geom(a.g, LB_EDGE).nblocks &&
-         pays(a.np, a.g, LB_EDGE);
+         pays(a.np, a.g, GATHER_PER_BLOCK[order]);
 }
 
 // host: where the answer goes on the host (null: the probe's report slot)
@@ -814,8 +813,20 @@ int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream
   return PXRHIP_OK;
 }
 
-bool leaf_binned_current_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
-bool leaf_binned_rho_pays(i64 np, const GridGeom &g) { return pays(np, g, LB_EDGE); }
+// Particles per block of the grid from which a direct current is summed block
+// by block.  A block's three LDS arrays are cleared and added up whole, so few
+// particles do not repay it.  Unbinned and binned at orders 1, 2 and 3: 66,000
+// on 200^3 cells (3.8 a block) 98, 268, 604 and 154, 355, 626 us; a million on
+// 512^3 (3.6) 1209, 3752, 8629 and 1590, 4834, 9520; on 384^3 (8.5) 1176, 3670,
+// 8501 and 869, 2331, 4483; 300,000 on 200^3 (17) 346, 1110, 2561 and 234, 448,
+// 727.  (The Esirkepov current and the charge density are faster binned at one
+// a block already.)
+constexpr int DIRECT_PER_BLOCK = 8;
+
+bool leaf_binned_current_pays(i64 np, const GridGeom &g, bool direct) {
+  return pays(np, g, direct ? DIRECT_PER_BLOCK : 1);
+}
+bool leaf_binned_rho_pays(i64 np, const GridGeom &g) { return pays(np, g, 1); }
 
 // the current of a.np particles, in parts that bound the records' memory
 template <bool MID>

@@ -137,3 +137,18 @@ def test_work_items(dev, chunk):
             assert last(dev, b"items") == (-(-c // size)).sum()
     finally:
         dev.call("pxrhip_set_tuning", b"leaf.bin_chunk", old.value)
+
+
+@pytest.mark.parametrize("n,direct", [(17575, 0), (17576, 0), (8 * 17576 - 1, 0), (8 * 17576, 1)])
+def test_currents_on_a_sparse_grid(dev, n, direct):
+    """26^3 = 17576 blocks: one particle each for Esirkepov, eight for direct"""
+    grid = (200, 200, 200)
+    P = plasma(dev, n, grid, False)
+    old = C.c_int64()
+    dev.call("pxrhip_get_tuning", b"leaf.bin_min", C.byref(old))
+    try:
+        dev.call("pxrhip_set_tuning", b"leaf.bin_min", 1)
+        assert current(dev, n, P, 1, 0, grid)[0] == (n >= 17576)
+        assert current(dev, n, P, 1, 3, grid)[0] == direct
+    finally:
+        dev.call("pxrhip_set_tuning", b"leaf.bin_min", old.value)
