@@ -945,7 +945,7 @@ int pxrhip_geteb3d_energy_conserving(
   const bool ask = leaf_binned_gather_may_pay(a, (int)nox);
   rt().last_leaf_gather = 0;
   LeafProbe probe;
-  if (ask && (r = leaf_probe_start(a, st, probe))) return r;
+  if (ask && (r = leaf_probe_start(a, (int)nox, st, probe))) return r;
   launch_gather(a, (int)nox, lo, st);
   if (ask) {
     bool scattered;

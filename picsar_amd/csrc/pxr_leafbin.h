@@ -85,7 +85,7 @@ struct LeafProbe {
     if (done) (void)hipEventDestroy(done);
   }
 };
-int leaf_probe_start(LeafGatherArgs &a, hipStream_t st, LeafProbe &probe);
+int leaf_probe_start(LeafGatherArgs &a, int order, hipStream_t st, LeafProbe &probe);
 int leaf_probe_read(LeafProbe &probe, bool &scattered);
 // work items of the last call, or part of one, that went block by block
 int leaf_last_items(int64_t *n);

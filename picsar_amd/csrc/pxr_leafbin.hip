@@ -549,12 +549,16 @@ __global__ __launch_bounds__(256) void k_lb_gather_add(LeafGatherArgs a, const d
 }
 
 // One workgroup looks at 64 runs of 64 consecutive particles spread over the
-// set: it is in no order if most particles have another block than their
-// predecessor (a set in cell order crosses blocks a few times a run).
+// set: it is in no order if more than 24 of the 63 in a run have another block
+// than their predecessor, on average (a set in cell order crosses blocks a few
+// times a run, one in random order nearly always).  `spread` > 0: and if the
+// 4096 particles are spread over at least about that many blocks, by the number
+// of pairs that share one (counted in 4096 hashed counters; n particles in N
+// blocks evenly: n^2 / N).
 template <int B>
-__global__ __launch_bounds__(1024) void k_lb_probe(LbPos a, BinGeom bg, int *out,
+__global__ __launch_bounds__(1024) void k_lb_probe(LbPos a, BinGeom bg, int spread, int *out,
                                                   unsigned long long *host_out) {
-  __shared__ int s[16];
+  __shared__ int s[16], pairs[16], cnt[4096];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int b[4], n = 0;
 #pragma unroll
@@ -568,24 +572,46 @@ __global__ __launch_bounds__(1024) void k_lb_probe(LbPos a, BinGeom bg, int *out
   for (int r = 0; r < 4; r++) n += __popcll(__ballot(lane > 0 && b[r] != __shfl_up(b[r], 1)));
   if (lane == 0) s[wave] = n;
   __syncthreads();
+  n = 0;
+  for (int w = 0; w < 16; w++) n += s[w];
+  int scattered = n > 64 * 24;
+  if (scattered && spread > 0) {  // (the same for all threads)
+#pragma unroll
+    for (int r = 0; r < 4; r++) cnt[threadIdx.x + 1024 * r] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; r++) atomicAdd(&cnt[(unsigned)b[r] * 2654435761u >> 20], 1);
+    __syncthreads();
+    int q = 0;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int c = cnt[threadIdx.x + 1024 * r];
+      q += c * (c - 1);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) q += __shfl_down(q, o);
+    if (lane == 0) pairs[wave] = q;
+    __syncthreads();
+    q = 0;  // at most 2^24
+    for (int w = 0; w < 16; w++) q += pairs[w];
+    scattered = q <= (1 << 24) / spread;
+  }
   if (threadIdx.x == 0) {
-    for (int w = 1; w < 16; w++) n += s[w];
-    const int scattered = n > 64 * 24;
     *out = scattered;
     *host_out = scattered;
   }
 }
+
+// Particles below which keys and counts take one launch: the radix sort's
+// blocks are of 1024 there, four a thread; of 4096 the key pass would have too
+// few waves in flight.
+constexpr i64 LB_COUNTED = 1 << 19;
 
 // Particle indices in block order (radix sort: the input order is kept
 // inside a block) and the work items.  Counting and placing the particles
 // with global atomics on the blocks' counters took 0.32 ms for two million
 // in random order (every particle its own atomic), this 0.09 ms.  Returns false,
 // with nothing launched, for a set it has no memory or index range for.
-// Particles below which keys and counts take one launch: the radix sort's
-// blocks are of 1024 there, four a thread; of 4096 the key pass would have too
-// few waves in flight.
-constexpr i64 LB_COUNTED = 1 << 19;
-
 template <int B, bool MID>
 static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st, BinGeom &bg,
                     int *&perm, int4 *&items, int *&nitems, i64 &maxitems) {
@@ -671,6 +697,18 @@ constexpr i64 GATHER_BIN_MIN1 = 3 << 20, GATHER_BIN_MIN = 3 << 18;
 // two on 384^3 (17) 3234 -> 3828, four on 512^3 (15) 7014 -> 8710.
 // (A million on 512^3, 3.6 a block: 356 -> 5191, 917 -> 6589, 1747 -> 7976.)
 constexpr int GATHER_PER_BLOCK[4] = {0, 192, 48, 24};
+// And blocks over which the particles are spread: in few of them (a bunch) the
+// plain kernel reads the fields from the caches.  A bunch of sigma cells in 128^3,
+// plain and staged (us): order 1, four million, sigma 3 222 and 533, sigma 12
+// (about 150 blocks) 393 and 651, a slab 4 thick (about 330) 313 and 636, 16
+// thick (700) 644 and 628, sigma 24 883 and 699; order 2, a million, sigma 6
+// (about 20) 181 and 209, sigma 12 254 and 239; four million, sigma 3 508 and
+// 556, sigma 6 699 and 603; order 3, a million, sigma 3 234 and 244, sigma 6 342
+// and 270; four million, sigma 1.5 689 and 623.
+static int gather_spread(int order, i64 np) {
+  const bool small = np < GATHER_BIN_MIN1;
+  return order == 1 ? 448 : order == 2 ? (small ? 64 : 10) : (small ? 10 : 0);
+}
 constexpr i64 DEPO_REC_MIN = 1 << 19;  // a million random: 236 -> 164 us (Esirkepov, order 1)
 constexpr int GATHER_CHUNK = 1024;  // particles of a gather's work item
 
@@ -745,18 +783,18 @@ bool leaf_binned_gather_may_pay(const LeafGatherArgs &a, int order) {
 }
 
 // host: where the answer goes on the host (null: the probe's report slot)
-static void launch_probe(const LbPos &pos, const GridGeom &g, hipStream_t st, LeafProbe &probe,
-                         unsigned long long *host = nullptr) {
+static void launch_probe(const LbPos &pos, const GridGeom &g, int spread, hipStream_t st,
+                         LeafProbe &probe, unsigned long long *host = nullptr) {
   unsigned long long *slot = report_slot();
   probe.host = host ? host : slot;
   probe.dev = (int *)(rt().d_bad + 2 + (slot - rt().h_report));
   hipLaunchKernelGGL(k_lb_probe<LB_EDGE>, dim3(1), dim3(1024), 0, st, pos,
-                     make_bin_geom(g, LB_EDGE), probe.dev, probe.host);
+                     make_bin_geom(g, LB_EDGE), spread, probe.dev, probe.host);
 }
 
-int leaf_probe_start(LeafGatherArgs &a, hipStream_t st, LeafProbe &probe) {
+int leaf_probe_start(LeafGatherArgs &a, int order, hipStream_t st, LeafProbe &probe) {
   PXR_HIP(hipEventCreateWithFlags(&probe.done, hipEventDisableTiming));
-  launch_probe(gather_pos(a, nullptr), a.g, st, probe);
+  launch_probe(gather_pos(a, nullptr), a.g, gather_spread(order, a.np), st, probe);
   PXR_LAUNCHED();
   PXR_HIP(hipEventRecord(probe.done, st));
   a.skip = probe.dev;
@@ -855,7 +893,7 @@ static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &don
               {0.5 * c.dtsdx0, 0.5 * c.dtsdy0, 0.5 * c.dtsdz0}, 0, nullptr, {}};
     if (d.packed.rec) {
       LeafProbe probe;
-      launch_probe(pos, a.g, st, probe, records_word());
+      launch_probe(pos, a.g, 0, st, probe, records_word());
       rt().last_leaf_records_asked = true;
       d.packed.use = probe.dev;
       pos.packed = d.packed;

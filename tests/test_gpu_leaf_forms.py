@@ -58,13 +58,16 @@ def current(dev, n, P, order, algo, grid=(NX, NY, NZ)):
     return last(dev, b"current"), last(dev, b"records")
 
 
+BIG = (100, 100, 100)  # 2744 blocks
+
+
 @pytest.mark.parametrize("order,n,form", [
     (1, 3145727, 0), (1, 3145728, 1), (2, 786431, 0), (2, 786432, 1), (3, 786431, 0),
     (3, 786432, 1), (3, 8400001, 1)])
 @pytest.mark.parametrize("ordered", [False, True])
 def test_gather(dev, order, n, form, ordered):
-    x = plasma(dev, n, None, ordered)[:3]
-    assert gather(dev, n, x, order) == (0 if ordered else form)
+    x = plasma(dev, n, BIG, ordered)[:3]
+    assert gather(dev, n, x, order, BIG) == (0 if ordered else form)
 
 
 @pytest.mark.parametrize("exchanged,form", [(20, 0), (900000, 1)])
@@ -72,11 +75,11 @@ def test_gather_of_a_set_losing_its_order(dev, exchanged, form):
     """a few particles exchanged, and most of them"""
     n = 900000
     rng = np.random.default_rng(exchanged)
-    x = particles(rng, n, margin=1.0)
+    x = [rng.uniform(1, g - 1, n) for g in BIG]
     o = cell_order(x)
     i = rng.permutation(n)[:exchanged]
     o[i] = o[np.roll(i, 1)]
-    assert gather(dev, n, [T(dev, a[o]) for a in x], 3) == form
+    assert gather(dev, n, [T(dev, a[o]) for a in x], 3, BIG) == form
 
 
 @pytest.mark.parametrize("algo", [0, 3])
@@ -152,3 +155,15 @@ def test_currents_on_a_sparse_grid(dev, n, direct):
         assert current(dev, n, P, 1, 3, grid)[0] == direct
     finally:
         dev.call("pxrhip_set_tuning", b"leaf.bin_min", old.value)
+
+
+@pytest.mark.parametrize("order,n,sigma,form", [
+    (1, 4000000, 3.0, 0), (1, 4000000, 12.0, 0), (1, 4000000, 30.0, 1), (2, 1000000, 3.0, 0),
+    (2, 1000000, 24.0, 1), (2, 4000000, 1.5, 0), (2, 4000000, 12.0, 1), (3, 1000000, 1.5, 0),
+    (3, 1000000, 12.0, 1), (3, 4000000, 3.0, 1)])
+def test_gather_of_a_bunch(dev, order, n, sigma, form):
+    """particles in few blocks are gathered plainly, whatever their order"""
+    grid = (128, 128, 128)
+    rng = np.random.default_rng(int(10 * sigma))
+    x = [np.clip(rng.normal(0.6 * g, sigma, n), 1.0, g - 1.0) for g in grid]
+    assert gather(dev, n, [T(dev, a) for a in x], order, grid) == form
