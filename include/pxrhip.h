@@ -501,7 +501,10 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
  * in no order block by block) and "leaf.bin_chunk" (particles of the largest
  * work item of that form, 1 to 2^20; up to the default, 4096, the routines
  * take smaller ones by themselves, 512 to 2048, a larger value is taken as it
- * is).
+ * is), "scratch.limit" (bytes: gives the library's scratch buffers back and,
+ * above 0, keeps their total at or below so much from then on; calls that have
+ * a form without take it, others fail with PXRHIP_ERR_HIP; graphs that keep
+ * scratch must be captured again; no other call may be running).
  * wg_per_cu 0 (the default) is automatic: three workgroups per CU with
  * 52224 bytes each when a work item of four sorting rows of the widest tile
  * fits that, else two with 79616 bytes; a wg_per_cu above 0 takes the
@@ -509,7 +512,8 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
  * direct deposition runs at most two workgroups per CU, since its kernel
  * holds registers for two waves per SIMD; it then takes 2 and 79616 bytes.
  * pxrhip_get_tuning also reads "last.wg_per_cu" and "last.lds_bytes", the
- * launch of the last pxrhip_tiles_gather_push_deposit, "device.num_cus", and
+ * launch of the last pxrhip_tiles_gather_push_deposit, "device.num_cus",
+ * "scratch.bytes" (held now), and
  * the form of the last leaf call with one order on all axes:
  * "last.leaf_current", "last.leaf_rho" and "last.leaf_gather" (1 block by
  * block, 0 particle by particle) and "last.leaf_records" (1 if that current

@@ -957,7 +957,9 @@ int pxrhip_geteb3d_energy_conserving(
     if (done < np) launch_gather(a.part(done, np - done), (int)nox, lo, st);
   }
   PXR_LAUNCHED();
-  return finish_checked("geteb3d_energy_conserving");
+  r = finish_checked("geteb3d_energy_conserving");
+  leaf_trim();
+  return r;
 }
 
 int pxrhip_boris_push_u_3d(int64_t np, double *uxp, double *uyp, double *uzp, double *gaminv,
@@ -1153,7 +1155,9 @@ int pxrhip_depose_jxjyjz(double *jx, double *jy, double *jz, int64_t np, const d
     }
   }
   PXR_LAUNCHED();
-  return finish_checked("depose_jxjyjz");
+  r = finish_checked("depose_jxjyjz");
+  leaf_trim();
+  return r;
 }
 
 int pxrhip_depose_rho_n(double *rho, int64_t np, const double *xp, const double *yp,
@@ -1212,7 +1216,9 @@ int pxrhip_depose_rho_n(double *rho, int64_t np, const double *xp, const double 
   else if (nox == 2) hipLaunchKernelGGL(k_rho<2>, grd, blk, 0, st, a);
   else hipLaunchKernelGGL(k_rho<3>, grd, blk, 0, st, a);
   PXR_LAUNCHED();
-  return finish_checked("pxr_depose_rho_n");
+  r = finish_checked("pxr_depose_rho_n");
+  leaf_trim();
+  return r;
 }
 
 static int mk_arr3(Arr3 &a, const double *p, const int64_t *lo, const int64_t *hi) {

@@ -58,8 +58,9 @@ struct GlobalAcc {
 
 // Binned forms: the particles are ordered by cubic blocks of nodes
 // and each block's current (or charge) is summed in LDS
-// before one global add per node.  Return PXRHIP_OK, or an error code
-// (scratch memory could not be allocated) before anything is launched.
+// before one global add per node.  They launch and do not wait.  Without memory
+// for the order they return PXRHIP_OK with nothing done (done = 0 or false),
+// and the unbinned kernels take the particles from `done` on.
 int leaf_binned_esirkepov(const DepoArgs &a, int order, hipStream_t st, i64 &done);
 int leaf_binned_direct(const DepoArgs &a, int order, hipStream_t st, i64 &done);
 int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done);
@@ -87,6 +88,8 @@ struct LeafProbe {
 };
 int leaf_probe_start(LeafGatherArgs &a, int order, hipStream_t st, LeafProbe &probe);
 int leaf_probe_read(LeafProbe &probe, bool &scattered);
+// gives scratch beyond 1 GiB a buffer back, after a call that has waited
+void leaf_trim();
 // work items of the last call, or part of one, that went block by block
 int leaf_last_items(int64_t *n);
 int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st, i64 &done);

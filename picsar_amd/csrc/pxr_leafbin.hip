@@ -39,6 +39,8 @@ struct BinGeom {
   i64 nblocks;
 };
 
+constexpr int LB_EDGE = 8;  // nodes per block edge
+
 static BinGeom make_bin_geom(const GridGeom &g, int B) {
   BinGeom b;
   b.gd[0] = g.gx; b.gd[1] = g.gy; b.gd[2] = g.gz;
@@ -607,29 +609,60 @@ __global__ __launch_bounds__(1024) void k_lb_probe(LbPos a, BinGeom bg, int spre
 // few waves in flight.
 constexpr i64 LB_COUNTED = 1 << 19;
 
+// Scratch: the ordering's, and the records'.
+enum { LB_KEYS = 24, LB_IDX, LB_HIST, LB_RANGES, LB_ITEMS, LB_NITEMS, LB_REC };
+constexpr i64 LB_HIST_CAP = (i64)1 << 21;  // ints of the sort's counts
+// Largest buffer kept from one call to the next.  A call that has waited for
+// itself gives larger ones back (allocating and freeing a few GB takes 0.6 ms,
+// a call that needs them 5 ms and more).
+constexpr size_t LB_KEEP = (size_t)1 << 30;
+
+// Buffers that order up to np particles at a time.
+struct LbOrder {
+  BinGeom bg;
+  i64 maxitems = 0;
+  int *keys, *idxs, *hist, *nitems;
+  int2 *range;
+  int4 *items;
+  int *perm;  // set by lb_sort
+};
+
+// Returns false for a set there is no memory or index range for.  The records
+// are asked for after this; those that an earlier call has left behind are
+// given up for it.
+static bool lb_alloc(i64 np, const GridGeom &g, int chunk, LbOrder &o) {
+  o.bg = make_bin_geom(g, LB_EDGE);
+  o.maxitems = o.bg.nblocks + np / chunk + 1;
+  if (np >= (i64)1 << 31 || o.bg.nblocks >= (i64)1 << 31 || o.maxitems >= (i64)1 << 31)
+    return false;
+  const i64 hist = radix_hist_most(np, o.bg.nblocks, LB_HIST_CAP);
+  for (int attempt = 0; attempt < 2; attempt++) {
+    o.keys = (int *)scratch(LB_KEYS, 2 * sizeof(int) * (size_t)np);
+    o.idxs = (int *)scratch(LB_IDX, 2 * sizeof(int) * (size_t)np);
+    o.hist = (int *)scratch(LB_HIST, sizeof(int) * (size_t)hist);
+    o.range = (int2 *)scratch(LB_RANGES, sizeof(int2) * (size_t)o.bg.nblocks);
+    o.items = (int4 *)scratch(LB_ITEMS, sizeof(int4) * (size_t)o.maxitems);
+    o.nitems = (int *)scratch(LB_NITEMS, sizeof(int));
+    if (o.keys && o.idxs && o.hist && o.range && o.items && o.nitems) return true;
+    if (!scratch_bytes(LB_REC)) return false;
+    scratch_free(LB_REC);
+  }
+  return false;
+}
+
 // Particle indices in block order (radix sort: the input order is kept
 // inside a block) and the work items.  Counting and placing the particles
 // with global atomics on the blocks' counters took 0.32 ms for two million
-// in random order (every particle its own atomic), this 0.09 ms.  Returns false,
-// with nothing launched, for a set it has no memory or index range for.
+// in random order (every particle its own atomic), this 0.09 ms.
 template <int B, bool MID>
-static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st, BinGeom &bg,
-                    int *&perm, int4 *&items, int *&nitems, i64 &maxitems) {
-  bg = make_bin_geom(g, B);
+static void lb_sort(const LbPos &a, int chunk, hipStream_t st, LbOrder &o) {
   const i64 np = a.np;
-  maxitems = bg.nblocks + np / chunk + 1;
-  if (np >= (i64)1 << 31 || bg.nblocks >= (i64)1 << 31 || maxitems >= (i64)1 << 31)
-    return false;
-  const RadixPlan plan = radix_plan(np, bg.nblocks, (i64)1 << 21);
-  int *keys = (int *)scratch(24, 2 * sizeof(int) * (size_t)np);
-  int *idxs = (int *)scratch(25, 2 * sizeof(int) * (size_t)np);
-  int *hist = (int *)scratch(26, sizeof(int) * (size_t)plan.hist_ints);
+  const BinGeom &bg = o.bg;
+  const RadixPlan plan = radix_plan(np, bg.nblocks, LB_HIST_CAP);
+  int *keys = o.keys, *idxs = o.idxs, *hist = o.hist, *nitems = o.nitems;
   // one pass of the sort: its counts say where the blocks lie
   const bool one = plan.npass == 1;
-  int2 *range = one ? nullptr : (int2 *)scratch(27, sizeof(int2) * (size_t)bg.nblocks);
-  items = (int4 *)scratch(28, sizeof(int4) * (size_t)maxitems);
-  nitems = (int *)scratch(29, sizeof(int));
-  if (!keys || !idxs || !hist || !(one || range) || !items || !nitems) return false;
+  int2 *range = one ? nullptr : o.range;
   int *key[2] = {keys, keys + np}, *idx[2] = {idxs, idxs + np};
   const bool counted = one && np < LB_COUNTED;
   if (counted)
@@ -639,13 +672,12 @@ static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st
     hipLaunchKernelGGL((k_lb_keys<B, MID>), dim3(grid1d(std::max(np, bg.nblocks), 256)), dim3(256),
                        0, st, a, bg, keys, range, nitems);
   const int at = radix_sort(plan, key, idx, hist, st, counted);
-  perm = idx[at];
+  o.perm = idx[at];
   if (!one)
     hipLaunchKernelGGL(k_lb_ranges, dim3(grid1d(np, 256)), dim3(256), 0, st, np, key[at], range);
   const BlockRanges br{range, hist, plan.nblk, 1 << plan.bits, (int)np};
   hipLaunchKernelGGL(k_lb_plan, dim3(grid1d(bg.nblocks, 1024)), dim3(1024), 0, st, br, bg.nblocks,
-                     chunk, items, nitems);
-  return true;
+                     chunk, o.items, nitems);
 }
 
 // The ordering and the kernels behind it share scratch.  A call launches them
@@ -655,6 +687,7 @@ static bool lb_sort(const LbPos &a, const GridGeom &g, int chunk, hipStream_t st
 // a gather and a deposition; with checks on every call waits for itself and
 // records none).  Where the event cannot be had the stream is waited for.
 class OrderTurn {
+  friend void leaf_trim();
   static std::mutex mutex;
   static hipEvent_t last;  // end of the last call's work
   std::lock_guard<std::mutex> lock{mutex};
@@ -674,10 +707,17 @@ class OrderTurn {
     }
   }
 };
+void leaf_trim() {
+  if (!rt().checks) return;
+  for (int k = LB_KEYS; k <= LB_REC; k++)
+    if (scratch_bytes(k) > LB_KEEP) {
+      std::lock_guard<std::mutex> lock(OrderTurn::mutex);
+      if (scratch_bytes(k) > LB_KEEP) scratch_free(k);
+    }
+}
 std::mutex OrderTurn::mutex;
 hipEvent_t OrderTurn::last = nullptr;
 
-constexpr int LB_EDGE = 8;  // nodes per block edge
 // Particles from which a gather asks for their order.  The question costs a
 // call in cell order 4 to 8 us, so it has to be a small part of the call.  A
 // million on 64^3 cells: order 3 151 -> 155 us in cell order and 618 -> 293 in
@@ -724,7 +764,7 @@ static unsigned lb_grid(i64 maxitems, size_t lds) {
   do {                                                                                       \
     PXR_HIP(hipFuncSetAttribute((const void *)&KERNEL,                                      \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));     \
-    hipLaunchKernelGGL(KERNEL, grd, blk, lds, st, ARGS, bg, perm, items, nitems);             \
+    hipLaunchKernelGGL(KERNEL, grd, blk, lds, st, ARGS, o.bg, o.perm, o.items, o.nitems);     \
   } while (0)
 
 // Work recorded into a graph, the library's or one of the caller's own, may
@@ -749,7 +789,7 @@ static int item_size(int own) {
 }
 
 int leaf_last_items(int64_t *n) {
-  int *nitems = (int *)scratch(29, sizeof(int)), v = 0;
+  int *nitems = (int *)scratch(LB_NITEMS, sizeof(int)), v = 0;
   if (!nitems) return set_error(PXRHIP_ERR_HIP, "scratch allocation failed");
   PXR_HIP(hipStreamSynchronize(rt().stream));
   PXR_HIP(hipMemcpy(&v, nitems, sizeof(int), hipMemcpyDeviceToHost));
@@ -802,7 +842,10 @@ int leaf_probe_start(LeafGatherArgs &a, int order, hipStream_t st, LeafProbe &pr
 }
 
 // Particles ordered at a time, in equal parts: 8 million, or 512 per block of
-// the grid, which bounds the records (48 or 64 bytes a particle).
+// the grid, which bounds the records (48 or 64 bytes a particle).  Fewer per
+// block cost more than they save: a hundred million in no order on 512^3 cells,
+// order 1, in one part, three, six and twelve 22.8, 26.2, 31.4 and 40.7 ms
+// (Esirkepov; without records 33.4) and 24.6, 33.6, 46.0 and 77.1 (gather).
 static i64 part_size(i64 np, const GridGeom &g) {
   const i64 most = std::max<i64>((i64)1 << 23, 512 * make_bin_geom(g, LB_EDGE).nblocks);
   const i64 nparts = (np + most - 1) / most;
@@ -817,24 +860,24 @@ int leaf_probe_read(LeafProbe &probe, bool &scattered) {
 
 int leaf_binned_gather(const LeafGatherArgs &a, int order, bool lower, hipStream_t st,
                        i64 &done) {
-  const i64 size = part_size(a.np, a.g);
+  i64 size = part_size(a.np, a.g);
+  const int chunk = item_size(GATHER_CHUNK);
   const int L = LB_EDGE + (order == 3 && !lower ? 4 : 3);
   const size_t lds = sizeof(double) * 6 * (size_t)(L * L * L);
   const OrderTurn turn(st);
   done = 0;
   LbGather ga;
-  if (!(ga.rec = (double *)scratch(30, 6 * sizeof(double) * (size_t)size))) return PXRHIP_OK;
+  LbOrder o;
+  if (!lb_alloc(size, a.g, chunk, o)) return PXRHIP_OK;
+  // smaller parts where there is no memory for the records of larger ones
+  while (!(ga.rec = (double *)scratch(LB_REC, 6 * sizeof(double) * (size_t)size))) {
+    if (size < GATHER_BIN_MIN) return PXRHIP_OK;
+    size = (size + 1) / 2;
+  }
   while (done < a.np) {
     ga.c = a.part(done, std::min(size, a.np - done));
-    BinGeom bg;
-    int *perm, *nitems;
-    int4 *items;
-    i64 maxitems;
-    if (!lb_sort<LB_EDGE, false>(gather_pos(ga.c, ga.rec), a.g,
-                                 item_size(GATHER_CHUNK), st, bg, perm, items,
-                                 nitems, maxitems))
-      return PXRHIP_OK;
-    const dim3 grd(lb_grid(maxitems, lds)), blk(512);
+    lb_sort<LB_EDGE, false>(gather_pos(ga.c, ga.rec), chunk, st, o);
+    const dim3 grd(lb_grid(o.maxitems, lds)), blk(512);
     switch (order * 2 + (lower ? 1 : 0)) {
       case 2: LB_LAUNCH((k_lb_gather<1, 1, LB_EDGE>), ga); break;
     case 3: LB_LAUNCH((k_lb_gather<1, 0, LB_EDGE>), ga); break;
@@ -871,7 +914,10 @@ template <bool MID>
 static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &done) {
   const OrderTurn turn(st);
   const EsirkConst<double> &c = a.ec;
-  const bool records = order <= 2 && a.np >= DEPO_REC_MIN;
+  // (with checks off nobody waits, and larger records would be kept)
+  const bool records = order <= 2 && a.np >= DEPO_REC_MIN &&
+                       (rt().checks ||
+                        8 * sizeof(double) * (size_t)part_size(a.np, a.g) <= LB_KEEP);
   const i64 size = records ? part_size(a.np, a.g) : a.np;
   const int L = LB_EDGE + (order == 1 ? 3 : 5);
   const size_t lds = sizeof(double) * 3 * (size_t)(L * L * L);
@@ -884,8 +930,10 @@ static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &don
   done = 0;
   LbDepo d;
   rt().last_leaf_records_asked = false;
-  if (records)
-    d.packed.rec = (double *)scratch(30, 8 * sizeof(double) * (size_t)size);
+  LbOrder o;
+  if (!lb_alloc(size, a.g, chunk, o)) return PXRHIP_OK;
+  if (records)  // (without memory for them the arrays are read)
+    d.packed.rec = (double *)scratch(LB_REC, 8 * sizeof(double) * (size_t)size);
   while (done < a.np) {
     d.c = a.part(done, std::min(size, a.np - done));
     LbPos pos{d.c.np, d.c.xp, d.c.yp, d.c.zp, d.c.ux, d.c.uy, d.c.uz, d.c.gi, d.c.w, c.xmin,
@@ -898,13 +946,8 @@ static int binned_current(const DepoArgs &a, int order, hipStream_t st, i64 &don
       d.packed.use = probe.dev;
       pos.packed = d.packed;
     }
-    BinGeom bg;
-    int *perm, *nitems;
-    int4 *items;
-    i64 maxitems;
-    if (!lb_sort<LB_EDGE, MID>(pos, a.g, chunk, st, bg, perm, items, nitems, maxitems))
-      return PXRHIP_OK;
-    const dim3 grd(lb_grid(maxitems, lds)), blk(256);
+    lb_sort<LB_EDGE, MID>(pos, chunk, st, o);
+    const dim3 grd(lb_grid(o.maxitems, lds)), blk(256);
     if constexpr (MID) {
       if (order == 1) LB_LAUNCH((k_lb_direct<1, LB_EDGE>), d);
       else if (order == 2) LB_LAUNCH((k_lb_direct<2, LB_EDGE>), d);
@@ -932,21 +975,18 @@ int leaf_binned_rho(const RhoArgs &a, int order, hipStream_t st, bool &done) {
   const OrderTurn turn(st);
   done = false;
   constexpr int E = LB_EDGE;
-  BinGeom bg;
-  int *perm, *nitems;
-  int4 *items;
-  i64 maxitems;
+  LbOrder o;
   const LbPos pos{a.np, a.xp, a.yp, a.zp, nullptr, nullptr, nullptr, nullptr, nullptr, a.xmin, a.ymin,
                   a.zmin, a.dxi, a.dyi, a.dzi, {0.0, 0.0, 0.0}, a.l4symtry, nullptr, {}};
   // work items as for the currents: 33.6 million in cell order on 128^3 cells,
   // 4096 particles an item and so, 3.46 -> 1.58, 3.44 -> 1.83 and 3.47 -> 2.85
   // ms at orders 1 to 3
   const int chunk = item_size(order == 3 ? 2048 : 1024);
-  if (!lb_sort<E, false>(pos, a.g, chunk, st, bg, perm, items, nitems, maxitems))
-    return PXRHIP_OK;
+  if (!lb_alloc(a.np, a.g, chunk, o)) return PXRHIP_OK;
+  lb_sort<E, false>(pos, chunk, st, o);
   const int L = E + (order == 1 ? 1 : 3);
   const size_t lds = sizeof(double) * (size_t)(L * L * L);
-  const dim3 grd(lb_grid(maxitems, lds)), blk(256);
+  const dim3 grd(lb_grid(o.maxitems, lds)), blk(256);
   if (order == 1) LB_LAUNCH((k_lb_rho<1, E>), a);
   else if (order == 2) LB_LAUNCH((k_lb_rho<2, E>), a);
   else LB_LAUNCH((k_lb_rho<3, E>), a);

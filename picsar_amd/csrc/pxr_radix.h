@@ -22,6 +22,9 @@ struct RadixPlan {
 // 2^20)
 RadixPlan radix_plan(i64 n, i64 nkeys, i64 hist_cap);
 
+// the largest hist_ints of a plan for n keys or fewer
+i64 radix_hist_most(i64 n, i64 nkeys, i64 hist_cap);
+
 // Sorts on stream st.  key[0] holds the keys (all in [0, nkeys)); key[1],
 // idx[0] and idx[1] are n ints each, hist plan.hist_ints.  Returns which of
 // the two buffers holds the sorted keys and, in key order and in increasing

@@ -18,16 +18,31 @@ namespace pxr {
 // 103 us (the whole leaf sort); from half a million on, the histogram costs
 // as much (a million in 48^3 cells 207 and 203 us; ordering two million by
 // 729 blocks for the leaf step 1110 and 1170).
-PXR_HD i64 rx_items(i64 n) { return n < ((i64)1 << 19) ? 1024 : 4096; }
+constexpr i64 RX_FEW = (i64)1 << 19;
+PXR_HD i64 rx_items(i64 n) { return n < RX_FEW ? 1024 : 4096; }
 constexpr int RX_SCAN = 2048;    // counts per block of the scan
 
-RadixPlan radix_plan(i64 n, i64 nkeys, i64 hist_cap) {
-  RadixPlan p;
-  p.n = n;
+static void rx_digits(i64 nkeys, RadixPlan &p) {
   int kb = 1;
   while (kb < 31 && ((i64)1 << kb) < nkeys) kb++;
   p.npass = (kb + RX_BITS - 1) / RX_BITS;
   p.bits = (kb + p.npass - 1) / p.npass;
+}
+
+// A plan's blocks are at most one per rx_items keys, so the most are those of n
+// keys or of the largest number cut into small ones.
+i64 radix_hist_most(i64 n, i64 nkeys, i64 hist_cap) {
+  RadixPlan p;
+  rx_digits(nkeys, p);
+  const i64 few = std::min(n, RX_FEW - 1), nblk = std::max((n + 4095) / 4096, (few + 1023) / 1024);
+  const i64 m = std::max<i64>(1, std::min(nblk, hist_cap >> p.bits)) << p.bits;
+  return m + (m + RX_SCAN - 1) / RX_SCAN;
+}
+
+RadixPlan radix_plan(i64 n, i64 nkeys, i64 hist_cap) {
+  RadixPlan p;
+  p.n = n;
+  rx_digits(nkeys, p);
   // a block's sums follow the counts in the histogram buffer
   const i64 cap = hist_cap - hist_cap / 1024;
   const i64 nblk = std::min<i64>((n + rx_items(n) - 1) / rx_items(n), cap >> p.bits);

@@ -47,6 +47,14 @@ int ensure_init();
 // if there is no memory for it (with the runtime's error state cleared, so
 // that a caller that has a form without scratch can launch that)
 void *scratch(int slot, size_t bytes);
+// gives a slot's memory back, once the work that uses it is done (hipFree waits
+// for the device)
+void scratch_free(int slot);
+// bytes held in slot (slot < 0: in all of them)
+size_t scratch_bytes(int slot);
+// Gives all scratch back and, with bytes > 0, keeps the total at or below so
+// much from here on: scratch() then returns null as if there was no more memory.
+void scratch_limit(size_t bytes);
 // A word of pinned host memory for a kernel to report through: the caller's
 // own until as many later calls have asked for one (calls of other threads
 // that wait at the same time have theirs).

@@ -19,6 +19,7 @@ struct Scratch {
   bool in_graph = false;  // handed out while a graph was recorded
 };
 static std::vector<Scratch> g_scratch(32);
+static size_t g_scratch_limit = 0;
 
 Runtime &rt() { return g_rt; }
 
@@ -40,15 +41,9 @@ void *scratch(int slot, size_t bytes) {
   Scratch &s = g_scratch[slot];
   if (g_rt.capturing) s.in_graph = true;
   if (s.bytes >= bytes && s.p) return s.p;
-  if (s.p) {
-    hipStreamSynchronize(g_rt.stream);
-    hipFree(s.p);
-    s.p = nullptr;
-    s.bytes = 0;
-    if (s.in_graph) g_rt.mem_gen++;
-    s.in_graph = g_rt.capturing;
-  }
+  scratch_free(slot);
   size_t want = bytes < 4096 ? 4096 : bytes;
+  if (g_scratch_limit && scratch_bytes(-1) + want > g_scratch_limit) return nullptr;
   if (hipMalloc(&s.p, want) != hipSuccess) {
     s.p = nullptr;
     (void)hipGetLastError();
@@ -56,6 +51,29 @@ void *scratch(int slot, size_t bytes) {
   }
   s.bytes = want;
   return s.p;
+}
+
+void scratch_free(int slot) {
+  Scratch &s = g_scratch[slot];
+  if (!s.p) return;
+  hipStreamSynchronize(g_rt.stream);
+  hipFree(s.p);
+  s.p = nullptr;
+  s.bytes = 0;
+  if (s.in_graph) g_rt.mem_gen++;
+  s.in_graph = g_rt.capturing;
+}
+
+size_t scratch_bytes(int slot) {
+  if (slot >= 0) return g_scratch[slot].bytes;
+  size_t sum = 0;
+  for (const Scratch &s : g_scratch) sum += s.bytes;
+  return sum;
+}
+
+void scratch_limit(size_t bytes) {
+  for (int k = 0; k < (int)g_scratch.size(); k++) scratch_free(k);
+  g_scratch_limit = bytes;
 }
 
 unsigned long long *report_slot() {

@@ -1542,6 +1542,10 @@ int pxrhip_set_tuning(const char *key, int64_t value) {
   } else if (!strcmp(key, "leaf.bin_chunk")) {
     if (value < 1 || value > (1 << 20)) return set_error(PXRHIP_ERR_ARG, "leaf.bin_chunk must be in [1, 2^20]");
     rt().leaf_bin_chunk = (int)value;
+  } else if (!strcmp(key, "scratch.limit")) {
+    if (value < 0) return set_error(PXRHIP_ERR_ARG, "scratch.limit must be >= 0 (0: none)");
+    if (rt().capturing) return set_error(PXRHIP_ERR_ARG, "the stream is being captured");
+    scratch_limit((size_t)value);
   } else if (!strcmp(key, "fused.margin_pct")) {
     if (value < 0 || value > 200) return set_error(PXRHIP_ERR_ARG, "fused.margin_pct must be in [0, 200]");
     g_tune.margin_pct = (int)value;
@@ -1583,6 +1587,7 @@ int pxrhip_get_tuning(const char *key, int64_t *value) {
   else if (!strcmp(key, "last.leaf_current")) *value = rt().last_leaf_current;
   else if (!strcmp(key, "last.leaf_rho")) *value = rt().last_leaf_rho;
   else if (!strcmp(key, "last.leaf_gather")) *value = rt().last_leaf_gather;
+  else if (!strcmp(key, "scratch.bytes")) *value = (int64_t)scratch_bytes(-1);
   else if (!strcmp(key, "last.leaf_items")) {
     *value = 0;
     if (rt().last_leaf_current || rt().last_leaf_rho || rt().last_leaf_gather)
