@@ -744,9 +744,9 @@ constexpr int GATHER_PER_BLOCK[4] = {0, 192, 48, 24};
 // thick (700) 644 and 628, sigma 24 883 and 699; order 2, a million, sigma 6
 // (about 20) 181 and 209, sigma 12 254 and 239; four million, sigma 3 508 and
 // 556, sigma 6 699 and 603; order 3, a million, sigma 3 234 and 244, sigma 6 342
-// and 270; four million, sigma 1.5 689 and 623.
+// and 270; two million, sigma 3 445 and 398; four million, sigma 1.5 689 and 623.
 static int gather_spread(int order, i64 np) {
-  const bool small = np < GATHER_BIN_MIN1;
+  const bool small = np < (i64)3 << 19;
   return order == 1 ? 448 : order == 2 ? (small ? 64 : 10) : (small ? 10 : 0);
 }
 constexpr i64 DEPO_REC_MIN = 1 << 19;  // a million random: 236 -> 164 us (Esirkepov, order 1)
