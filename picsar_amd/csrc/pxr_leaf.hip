@@ -565,8 +565,17 @@ constexpr int ZCHUNK = 64;  // most planes per thread
 #ifndef ZBX
 #define ZBX 64     // columns of a block along x (256 / ZBX along y)
 #endif
+// Order 8 and the E step of order 6 are scheduled for three waves per SIMD.
+// Left to aim for four, the compiler waits for a plane's loads a few at a time;
+// for three it has all of a component's in flight (126 to 144 registers).  On
+// 200^3, 256^3 and 320^3 cells: order 8 B half step 443, 894 and 1415 -> 248, 539
+// and 946 us, E step 481, 935 and 1472 -> 286, 609 and 1064; order 6 E step 322,
+// 637 and 1024 -> 248, 533 and 946 (its B half step, 112 registers either way,
+// loses a hundredth at three).
 template <int NH, bool E, int IST>
-__global__ __launch_bounds__(256) void k_norder_z(NorderArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
+    1, NH == 4 || (NH == 3 && E) ? 3 : 8)))
+void k_norder_z(NorderArgs a) {
   const GridGeom &g = a.g;
   const int nxu = g.nx + 2 * a.nxs + 1, nyu = g.ny + 2 * a.nys + 1, nzu = g.nz + 2 * a.nzs + 1;
   const unsigned gbx = (nxu + ZBX - 1) / ZBX, gby = (nyu + 256 / ZBX - 1) / (256 / ZBX);
