@@ -29,8 +29,7 @@ def dev():
 @pytest.fixture
 def streams(dev):
     """two streams of the library's HIP runtime; the library's own afterwards"""
-    path = next(ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln)
-    hip = C.CDLL(path)
+    hip = C.CDLL(dev.LIB_PATH)  # its symbols include those of the runtime it is linked to
     own = dev.load().pxrhip_get_stream()
     s = [C.c_void_p(), C.c_void_p()]
     for p in s:
