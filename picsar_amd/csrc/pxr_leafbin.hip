@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256, N == 3 ? 3 : 1) void k_lb_esirkepov(LbDepo d, 
       continue;
     }
     if (blk.holds(lo, hi)) esirkepov_deposit<N, double>(in, acc);
-    else esirkepov_deposit<N, double>(in, gacc);  // not reached: the halo holds every box
+    else esirkepov_deposit<N, double>(in, gacc);  // a position that is not a number
   }
   lb_flush(blk, a.g, dst, 3);
   }
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(256) void k_lb_direct(LbDepo d, BinGeom bg, const i
         continue;
       }
       if (blk.holds(lo, hi)) direct_deposit<N, double>(in, acc);
-      else direct_deposit<N, double>(in, gacc);  // not reached: the halo holds every box
+      else direct_deposit<N, double>(in, gacc);  // a position that is not a number
     }
     lb_flush(blk, a.g, dst, 3);
   }
