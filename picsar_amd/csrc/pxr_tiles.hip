@@ -1045,7 +1045,9 @@ PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, Chunk *out, i64 room, in
     return nch;
   }
   if (g != GROUP_ROWS) return 0;
-  // start of row y (y = ny3: the end of the plane)
+  // start of row y (y = ny3: the end of the plane); what an earlier walk of
+  // these lanes staged has been read
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   for (int y = lane; y <= min(ny3, ROWS - 1); y += CG) rs[y] = a.bin_start[base + (int64_t)y * nx3];
   // the lanes read each other's entries: one wave, so its own LDS order suffices
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1103,14 +1105,42 @@ PXR_DEV int walk_unit(const ChunkArgs &a, int t, int z, Chunk *out, i64 room, in
 
 constexpr int STAGE = CG;  // chunks per unit that k_chunk_count stores
 
+// Whether unit (t, z) takes a walk of its rows; the others have one chunk or
+// none, or are tiles without sorting information.
+PXR_DEV bool unit_has_rows(const ChunkArgs &a, int t, int z) {
+  return a.bin_start && a.tile_np[t] > 0 && z < a.n3[3 * t + 2] &&
+         a.group[(i64)t * a.nzmax + z] == GROUP_ROWS;
+}
+
+// Few units are each given to the CG lanes, which keep the first chunks.  Of many
+// most are members of a group or heads of one: there each lane does one, and
+// the lanes together those with rows in turn.  All lanes to each took 25 us here
+// and 39 in k_chunk_write for the 294,912 planes of the 8^3-node tiles of 256^3
+// cells, this 6 and 9 (a thread to each, rows included, 5 and 6); for the 4.7
+// million of 512 x 512 x 1024 386 and 654, this 48 and 96 (29 and 72).
+template <bool MANY>
 __global__ __launch_bounds__(256) void k_chunk_count(ChunkArgs a) {
   __shared__ i64 rs[256 / CG][ROWS];
-  const i64 u = ((i64)blockIdx.x * blockDim.x + threadIdx.x) / CG;
-  const int lane = threadIdx.x % CG;
-  if (u >= (i64)a.ntiles * a.nzmax) return;
-  const int n = walk_unit(a, (int)(u / a.nzmax), (int)(u % a.nzmax), a.stage + u * STAGE,
-                          a.stage ? STAGE : 0, lane, rs[threadIdx.x / CG]);
-  if (lane == 0) a.count[u] = n;
+  const i64 nu = (i64)a.ntiles * a.nzmax;
+  const int lane = threadIdx.x % CG, k = threadIdx.x / CG;
+  const i64 th = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (MANY) {
+    const int t = (int)(min(th, nu - 1) / a.nzmax), z = (int)(min(th, nu - 1) % a.nzmax);
+    const bool rows = th < nu && unit_has_rows(a, t, z);
+    int n = th < nu && !rows ? walk_unit(a, t, z, nullptr, 0, 0, rs[k]) : 0;
+    for (unsigned m = cg_ballot(rows); m; m &= m - 1) {
+      const int l = __ffs(m) - 1;
+      const int c = walk_unit(a, __shfl(t, l, CG), __shfl(z, l, CG), nullptr, 0, lane, rs[k]);
+      if (lane == l) n = c;
+    }
+    if (th < nu) a.count[th] = n;
+  } else {
+    const i64 u = th / CG;
+    if (u >= nu) return;
+    const int n = walk_unit(a, (int)(u / a.nzmax), (int)(u % a.nzmax), a.stage + u * STAGE,
+                            a.stage ? STAGE : 0, lane, rs[k]);
+    if (lane == 0) a.count[u] = n;
+  }
 }
 
 // Largest-first queue order of the work items: a counting sort of the
@@ -1144,23 +1174,25 @@ __global__ __launch_bounds__(256) void k_order_scatter(const Chunk *chunks, cons
   order[atomicAdd(bucket + (n > 0 ? 31 - __clz(n) : 0), 1)] = c;
 }
 
-// The chunks of every unit.  a.start null: few units, and each block sums
-// the counts before its own itself, which saves the three launches of the
-// scan.
+// The chunks of every unit.  Few units: each block sums the counts before its
+// own itself, which saves the launches of the scan (a.start is not used).
 constexpr i64 CHUNK_SELF_SCAN = 16384;
 
+template <bool MANY>
 __global__ __launch_bounds__(256) void k_chunk_write(ChunkArgs a) {
-  constexpr int PER = 256 / CG;  // units per block
+  constexpr int PER = 256 / CG;  // units per block at a time
   __shared__ int before[4];
   __shared__ i64 rs[PER][ROWS];
   const i64 nu = (i64)a.ntiles * a.nzmax;
   const int lane = threadIdx.x % CG, k = threadIdx.x / CG;
-  const i64 u0 = (i64)blockIdx.x * PER, u = u0 + k;
+  const i64 u = MANY ? (i64)blockIdx.x * 256 + threadIdx.x : (i64)blockIdx.x * PER + k;
+  const bool first = MANY || lane == 0;  // the lane that answers for unit u
   i64 pos = 0, tot = 0;
-  if (a.start) {
+  if (MANY) {
     if (u < nu) pos = a.start[u];
     tot = a.start[nu];
   } else {
+    const i64 u0 = (i64)blockIdx.x * PER;
     int acc = 0;
     for (i64 i = threadIdx.x; i < u0; i += 256) acc += a.count[i];
 #pragma unroll
@@ -1171,17 +1203,26 @@ __global__ __launch_bounds__(256) void k_chunk_write(ChunkArgs a) {
     for (i64 i = u0; i < min(u, nu); i++) pos += a.count[i];
     tot = pos + (u < nu ? a.count[u] : 0);
   }
-  if (u < nu) {
-    const int n = a.count[u];
-    const i64 room = min(a.maxchunks - pos, (i64)n);
-    if (room < n && lane == 0) atomicAdd(a.bad, (unsigned long long)(n - max(room, (i64)0)));  // cannot happen: see the bound
+  const int n = u < nu ? a.count[u] : 0;
+  const i64 room = min(a.maxchunks - pos, (i64)n);
+  if (room < n && first) atomicAdd(a.bad, (unsigned long long)(n - max(room, (i64)0)));  // cannot happen: see the bound
+  const int t = (int)(min(u, nu - 1) / a.nzmax), z = (int)(min(u, nu - 1) % a.nzmax);
+  if (MANY) {
+    const bool rows = n > 0 && unit_has_rows(a, t, z);
+    if (n > 0 && !rows) walk_unit(a, t, z, a.out + pos, room, 0, rs[k]);
+    for (unsigned m = cg_ballot(rows); m; m &= m - 1) {
+      const int l = __ffs(m) - 1;
+      walk_unit(a, __shfl(t, l, CG), __shfl(z, l, CG), a.out + __shfl(pos, l, CG),
+                __shfl(room, l, CG), lane, rs[k]);
+    }
+  } else if (u < nu) {
     if (a.stage && n <= STAGE) {
       if (lane < room) a.out[pos + lane] = a.stage[u * STAGE + lane];
     } else {
-      walk_unit(a, (int)(u / a.nzmax), (int)(u % a.nzmax), a.out + pos, room, lane, rs[k]);
+      walk_unit(a, t, z, a.out + pos, room, lane, rs[k]);
     }
   }
-  if (u == nu - 1 && lane == 0) {
+  if (u == nu - 1 && first) {
     *a.nchunks = (int)min(tot, a.maxchunks);
     *a.queue = 0;
     a.queue[1] = 0;  // overflow count (ctl[2])
@@ -1469,13 +1510,16 @@ static int build_chunks(const TileTable *tt, const pxrhip_species *sp, const Box
   ca.jroom = jroom;
   ca.sk4 = sk4;
   hipLaunchKernelGGL(k_chunk_groups, dim3(grid1d((i64)tt->ntiles * CG, 256)), dim3(256), 0, st, ca);
-  hipLaunchKernelGGL(k_chunk_count, dim3(grid1d(nunits * CG, 256)), dim3(256), 0, st, ca);
   if (nunits <= CHUNK_SELF_SCAN) {
-    ca.start = nullptr;
+    const dim3 gr(grid1d(nunits * CG, 256));
+    hipLaunchKernelGGL(k_chunk_count<false>, gr, dim3(256), 0, st, ca);
+    hipLaunchKernelGGL(k_chunk_write<false>, gr, dim3(256), 0, st, ca);
   } else {
+    const dim3 gr(grid1d(nunits, 256));
+    hipLaunchKernelGGL(k_chunk_count<true>, gr, dim3(256), 0, st, ca);
     scan_counts(cnt, nunits, bsum, cstart, nullptr, st);
+    hipLaunchKernelGGL(k_chunk_write<true>, gr, dim3(256), 0, st, ca);
   }
-  hipLaunchKernelGGL(k_chunk_write, dim3(grid1d(nunits * CG, 256)), dim3(256), 0, st, ca);
   PXR_LAUNCHED();
   *chunks_out = chunks;
   *ctl_out = ctl;
