@@ -296,8 +296,8 @@ int pxrhip_particle_bin_sorting(int64_t np2, double *xp, double *yp,
  * ends) instead of buffers it allocates.  Limits: np2 <= 2^20 particles and
  * at most 2^20 sorting-grid bins, else PXRHIP_ERR_ARG; pxrhip_init must have
  * been called (it allocates, so this entry point does not call it).  Every
- * call on one GPU uses that GPU's one array: calls that overlap on a GPU
- * (other host threads, other streams) race. */
+ * call on one GPU uses that GPU's one array; calls of several host threads
+ * take turns (each waits for its stream before it returns). */
 int pxrhip_particle_bin_sorting_noalloc(int64_t np2, double *xp, double *yp,
                                         double *zp, double *ux, double *uy,
                                         double *uz, double *gam, double *pid,
@@ -465,7 +465,9 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
 /* Launch parameters of the tiled kernels.  No counterpart in the reference
  * (its CPU blocking factors lvec_* play this role).  Keys:
  * "fused.lds_bytes" (dynamic LDS per workgroup), "fused.wg_per_cu",
- * "fused.spread" (0/1, lane-spread particle order in the deposition phase),
+ * "fused.spread" (0/1, lane-spread particle order in the deposition phase;
+ * it and the strides below have no effect on the order-3 Esirkepov deposition
+ * in fixed point, whose lanes are dealt by LDS bank),
  * "fused.sstride" (largest lane stride of that order, 0: a sixty-fourth of
  * the work item; -1, the default, sets one per work item from its particles
  * per sorting cell and the shape order, none at order 3) and
