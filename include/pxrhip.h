@@ -467,7 +467,8 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
  * "fused.lds_bytes" (dynamic LDS per workgroup), "fused.wg_per_cu",
  * "fused.spread" (0/1, lane-spread particle order in the deposition phase;
  * it and the strides below have no effect on the order-3 Esirkepov deposition
- * in fixed point, whose lanes are dealt by LDS bank),
+ * in fixed point where its lanes are dealt by LDS bank: in mixed precision, and
+ * in FP64 but for species of 0.75 to 2.5 particles per cell),
  * "fused.sstride" (largest lane stride of that order, 0: a sixty-fourth of
  * the work item; -1, the default, sets one per work item from its particles
  * per sorting cell and the shape order, none at order 3) and
@@ -514,7 +515,8 @@ int pxrhip_tiles_depose_rho(const pxrhip_grid *grid, const pxrhip_species *sp,
  * direct deposition runs at most two workgroups per CU, since its kernel
  * holds registers for two waves per SIMD; it then takes 2 and 79616 bytes.
  * pxrhip_get_tuning also reads "last.wg_per_cu" and "last.lds_bytes", the
- * launch of the last pxrhip_tiles_gather_push_deposit, "device.num_cus",
+ * launch of the last pxrhip_tiles_gather_push_deposit, "last.bank_lanes" (1
+ * if its lanes were dealt by LDS bank), "device.num_cus",
  * "scratch.bytes" (held now), and
  * the form of the last leaf call with one order on all axes:
  * "last.leaf_current", "last.leaf_rho" and "last.leaf_gather" (1 block by

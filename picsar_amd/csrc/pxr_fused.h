@@ -238,7 +238,8 @@ PXR_DEV double fx_weight(const FusedArgs &a, double qw, double vx, double vy, do
 // Launch times at 96^3, 8 particles per cell (ms per species, before and with
 // it): FP64 1.07 -> 0.98, mixed precision 0.85 -> 0.81 (0.80 -> 0.75 for the
 // colder ions), the gamma = 10 bunch 0.37 -> 0.34; at 16 particles per cell
-// 1.88 -> 1.68, at 64 (mixed) 0.92 -> 0.82, at 1 0.315 -> 0.325 (FP64) and
+// 1.88 -> 1.68, at 64 (mixed) 0.92 -> 0.82, at 1 0.315 -> 0.325 (FP64, which
+// at about one and two per cell is launched without: a.slots null) and
 // 0.209 -> 0.207 (mixed).  At order 2 it lost 2%, at order 1 15%, and the
 // order-3 direct current was unchanged.
 constexpr bool use_banks(int order, int depo, int jacc) {
@@ -608,7 +609,8 @@ PXR_DEV void fx_scale(const FusedArgs &a, unsigned long long wbits, int n, doubl
 // Registers are capped for three waves per SIMD (three workgroups of 256
 // lanes per CU), except for the order-3 direct deposition of an FP64
 // species, which would spill and keeps two.
-template <int BS, int N, bool LO, int PUSHER, int DEPO, bool MX, int JACC>
+template <int BS, int N, bool LO, int PUSHER, int DEPO, bool MX, int JACC,
+          bool BANKS = use_banks(N, DEPO, JACC)>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(
     (N == 3 && DEPO == 3 && !MX) ? 2 : 3))) void k_fused(FusedArgs a) {
   typedef typename std::conditional<MX, float, double>::type FT;  // field block
@@ -621,7 +623,6 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(
   __shared__ int s_chunk;
   __shared__ int s_box[6];
   __shared__ unsigned long long s_wabs;  // largest |q w| of the work item (JACC 3)
-  constexpr bool BANKS = use_banks(N, DEPO, JACC);
   const GridGeom &g = a.g;
   const int glo[3] = {-g.gx, -g.gy, -g.gz};
   const int ghi[3] = {g.nx + g.gx, g.ny + g.gy, g.nz + g.gz};

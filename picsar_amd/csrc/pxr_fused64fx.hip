@@ -10,12 +10,17 @@ static const int FUSED_BS = 256;
 
 int launch_fused_fp64_fx(int key, const FusedArgs &a, int nwg, size_t lds, hipStream_t st) {
   const dim3 grd(nwg), blk(FUSED_BS);
+#define PXR_FUSED_LAUNCH(N_, LO_, P_, D_, B_)                                                    \
+  do {                                                                                           \
+    if (lds > 65536)                                                                             \
+      PXR_HIP(hipFuncSetAttribute((const void *)&k_fused<FUSED_BS, N_, LO_, P_, D_, false, 3, B_>, \
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));       \
+    hipLaunchKernelGGL((k_fused<FUSED_BS, N_, LO_, P_, D_, false, 3, B_>), grd, blk, lds, st, a);  \
+  } while (0)
 #define PXR_FUSED_CASE(N_, LO_, P_, D_)                                                          \
   case N_ * 100 + (LO_ ? 10 : 0) + P_ * 2 + (D_ ? 1 : 0):                                        \
-    if (lds > 65536)                                                                             \
-      PXR_HIP(hipFuncSetAttribute((const void *)&k_fused<FUSED_BS, N_, LO_, P_, D_, false, 3>,     \
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));       \
-    hipLaunchKernelGGL((k_fused<FUSED_BS, N_, LO_, P_, D_, false, 3>), grd, blk, lds, st, a);      \
+    if (use_banks(N_, D_, 3) && !a.slots) PXR_FUSED_LAUNCH(N_, LO_, P_, D_, false);                 \
+    else PXR_FUSED_LAUNCH(N_, LO_, P_, D_, use_banks(N_, D_, 3));                                  \
     hipLaunchKernelGGL((k_fused_overflow<FUSED_BS, N_, LO_, P_, D_, false>), dim3(2 * rt().num_cus), \
                        blk, 0, st, a);                                                           \
     break;
@@ -33,6 +38,7 @@ int launch_fused_fp64_fx(int key, const FusedArgs &a, int nwg, size_t lds, hipSt
       return set_error(PXRHIP_ERR_ARG, "unsupported kernel combination");
   }
 #undef PXR_FUSED_CASE
+#undef PXR_FUSED_LAUNCH
   PXR_LAUNCHED();
   return PXRHIP_OK;
 }

@@ -1323,7 +1323,7 @@ static int sstride_k4(int order, bool mx) {
   return mx ? 12 : 0;
 }
 // the launch chosen by the last pxrhip_tiles_gather_push_deposit
-static int g_last_wg_per_cu = 0, g_last_lds_bytes = 0;
+static int g_last_wg_per_cu = 0, g_last_lds_bytes = 0, g_last_banks = 0;
 }  // namespace pxr
 
 // Charge density of a binned species, per work item: the tile blocks of
@@ -1628,6 +1628,7 @@ int pxrhip_get_tuning(const char *key, int64_t *value) {
   else if (!strcmp(key, "last.wg_per_cu")) *value = g_last_wg_per_cu;
   else if (!strcmp(key, "device.num_cus")) *value = rt().device >= 0 ? rt().num_cus : 0;
   else if (!strcmp(key, "last.lds_bytes")) *value = g_last_lds_bytes;
+  else if (!strcmp(key, "last.bank_lanes")) *value = g_last_banks;
   else if (!strcmp(key, "last.leaf_current")) *value = rt().last_leaf_current;
   else if (!strcmp(key, "last.leaf_rho")) *value = rt().last_leaf_rho;
   else if (!strcmp(key, "last.leaf_gather")) *value = rt().last_leaf_gather;
@@ -1951,9 +1952,19 @@ static int tiles_fused(const pxrhip_grid *grid, const pxrhip_species *sp, const 
   }
   const bool mx = sp->precision == 1;
   // lanes dealt by bank: the slots hold 16-bit places in a work item, and a
-  // row of them is kept for every workgroup
+  // row of them is kept for every workgroup.  An FP64 species of about one or
+  // two particles per cell of the grid does without: there the dealing costs
+  // more than it gives (whole steps of two species at 1, 2, 3 and 4 per cell,
+  // with it and without: 484, 516, 594 and 663 us and 462, 498, 592 and 676 on
+  // 64^3 cells in 16^3-node tiles, 832, 1072, 1334 and 1563 and 817, 1073, 1345
+  // and 1603 on 96^3 in 8^3).  Fewer than three in four cells are taken for a
+  // bunch, which fills a part of the box densely (a peak of 64 per cell 475 and
+  // 470, of 512 810 and 882 us).
+  const double per_cell = (double)sp->capacity / ((double)grid->nx * grid->ny * grid->nz);
+  const bool sparse = !mx && per_cell >= 0.75 && per_cell < 2.5;
   const bool banks = use_banks((int)order, depo_algo ? 3 : 0,
-                               mx ? g_tune.jacc : g_tune.fp64_jacc) && (phase & PHASE_DEPOSIT);
+                               mx ? g_tune.jacc : g_tune.fp64_jacc) &&
+                     (phase & PHASE_DEPOSIT) && !sparse;
   if (banks && ch > BANK_CHUNK) ch = BANK_CHUNK;
   const int esize = mx ? 4 : 8;
   // LDS current: mixed.jacc (0 FP32, 1 compensated FP32, 2 FP64, 3 fixed
@@ -2073,6 +2084,7 @@ static int tiles_fused(const pxrhip_grid *grid, const pxrhip_species *sp, const 
   const int nwg = rt().num_cus * wg_per_cu;
   g_last_wg_per_cu = wg_per_cu;
   g_last_lds_bytes = (int)lds_bytes;
+  g_last_banks = banks;
   const size_t lds = (size_t)lds_bytes;
   const int key = (int)(order * 100 + (l_lower_order_in_v ? 10 : 0) + pusher * 2 + (depo_algo ? 1 : 0));
   if (!mx)
